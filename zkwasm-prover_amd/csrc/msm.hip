@@ -11,21 +11,25 @@
 //               digits d_w in (-2^(c-1), 2^(c-1)], written window-major.
 //               Zero digits add nothing.
 //   2. sort     two-level counting sort of (bucket, point index | sign):
-//               per-tile LDS histograms of the high 8 bucket bits, one global
+//               per-tile LDS histograms of the high bucket bits, one global
 //               scan, scatter into (item, window, high bits) groups with LDS
-//               ranks, then an LDS counting sort of each group on the low 8
+//               ranks, then an LDS counting sort of each group on the low
 //               bits that also emits the bucket offsets.  Writes land in
 //               short contiguous runs instead of 4-byte random scatters.
+//               Small items: one workgroup sorts a whole window.
 //   3. accumulate  threads own equal chunks of the sorted entries (perfect
 //               load balance for any digit distribution); runs of one bucket
 //               are summed with XYZZ mixed additions in 29-bit-limb lazy
 //               Montgomery arithmetic (ff29.h); runs cut by a chunk border
 //               are left as head/tail partials.
-//   4. fixup    partials of buckets that span chunks are merged.
-//   5. reduce   S_w = sum_b (b+1) B_{w,b}: per segment of L1 buckets a
-//               running sum gives (WS, SUM); then
-//               S_w = sum_s WS_s + L1 * sum_bit 2^bit * (sum_{s has bit} SUM_s),
-//               the masked sums being parallel tree reductions.
+//   4. fixup    partials of buckets that span chunks are merged, by quads of
+//               lanes (x29quad.h).
+//   5. reduce   S_w = sum_b (b+1) B_{w,b}.  Few buckets: butterfly sums over
+//               quads of lanes give T = sum_b B_b and, per bit k of b, the
+//               masked sum Q_k; S_w = T + sum_k 2^k Q_k.  Many: per segment of
+//               L1 buckets a running sum gives (WS, SUM); then S_w = sum_s
+//               WS_s + L1 * sum_bit 2^bit * (sum_{s has bit} SUM_s), the masked
+//               sums being parallel tree reductions.
 //   6. collect  sum_w 2^(c w) S_w by Horner over windows, normalised to z = 1
 //               so the bytes are canonical (host cores by default).
 // The bucket semantics restate cuda/msm.cu:9-181 (digit d of window w adds
@@ -44,6 +48,7 @@
 #include "guard.h"
 #include "ff29.h"
 #include "host_ec.h"
+#include "x29quad.h"
 #include "zkcore.h"
 
 using namespace zk;
@@ -56,25 +61,36 @@ constexpr uint32_t kL1 = 8;          // buckets per first-level reduction segmen
 // cost of a slightly longer last wave (2^22 points: fixup 0.31 -> 0.11 ms,
 // accumulation +0.05 ms)
 constexpr uint32_t kChunk = 96;
-// A pass with few sorted entries would leave most of the device idle with
-// chunks of kChunk (2^12 points at c = 8: 131k entries, ~1.4k threads, each
-// a chain of 96 dependent additions); below kSmallEntries the chunk shrinks
-// toward kSmallThreads threads, down to kMinChunk entries.
-constexpr uint64_t kSmallEntries = (uint64_t)1 << 21;
-constexpr uint64_t kSmallThreads = (uint64_t)1 << 16;
+// With few sorted entries, chunks of kChunk would leave most of the device
+// idle (2^12 points at c = 7: 150k entries, 1.6k threads, each a chain of 96
+// dependent additions).  The chunk is therefore chosen on the device from
+// the number of entries there really are (zero digits leave none): the
+// smallest number of rounds of kRoundThreads threads (one 256-thread
+// workgroup per CU) with at most kChunk entries each, and up to kMinRounds
+// rounds while that leaves at least kMinChunk entries.  Whole rounds keep the
+// last one from running on a few CUs.
+constexpr uint32_t kRoundThreads = 256 * 256;
+constexpr uint32_t kMinRounds = 3;
 constexpr uint32_t kMinChunk = 8;
-constexpr uint32_t kWalk = 32;       // chunk partials one fixup thread sums; longer buckets go to a workgroup
+// Buckets whose run spans more chunks than this go to a workgroup each
+// (k_msm_fixup_long), the others to one quad of lanes, a serial chain.
+constexpr uint32_t kWalk = 12;
+// Bucket reduction: up to this many buckets in the pass by quads of lanes
+// (k_msm_bits: a chain of 4 + B / 1024 + 6 additions), above it by one lane
+// per 8 buckets (k_msm_reduce_fold: 22 additions, a third less lane work).
+constexpr uint64_t kQuadBuckets = (uint64_t)1 << 17;
 constexpr uint32_t kNone = 0xffffffffu;
 constexpr uint32_t kMagic = 0x4d534d32u;  // "MSM2": masked sums present in the slice
 // Curve-slice layout left by msm() for batch_msm_collect:
 //   [0, 96)          the result (Jacobian), written last
 //   [64, 96)         header {magic, c, W, nbits}
-//   [128, ...)       Q[w][0..nbits]: W * (nbits + 1) XYZZ masked sums
+//   [128, ...)       Q[w][0..nbits]: W * (nbits + 1) XYZZ masked sums; window
+//                   w's sum is Q[w][nbits] + sum_k 2^(l1 + k) Q[w][k]
 //   then            S[w]: W Jacobian window sums (device tail only)
 constexpr size_t kSliceQ = 128;
 // bytes of a slice the layout above can use: W * (nbits + 1) masked sums and
-// W window sums stay below 31200 B for every window 2 <= c <= 17 (kL1 >= 4)
-constexpr size_t kSliceReserve = 32 * 1024;
+// W window sums stay below 34300 B for every window 2 <= c <= 17
+constexpr size_t kSliceReserve = 36 * 1024;
 
 // Arrays placed into caller memory, in two lifetimes: phase 1 (the sort) and
 // phase 2 (accumulation and reduction).  offsets, entries and the long-bucket
@@ -83,13 +99,22 @@ constexpr size_t kSliceReserve = 32 * 1024;
 enum MsmArr {
     A_ITEMS, A_SLOTS, A_OFFSETS, A_ENTRIES, A_LONG,                // both phases
     A_TMP, A_HIST, A_STARTS, A_SCAN,                               // phase 1
-    A_BUCKETS, A_PHEAD, A_PTAIL, A_HB, A_TB, A_WS1, A_SUM1,        // phase 2
+    A_BUCKETS, A_PHEAD, A_PTAIL, A_TB, A_PART,                     // phase 2
     A_COUNT
 };
 constexpr int kFirstPhase2 = A_BUCKETS;
 
-constexpr uint32_t kSortTile = 4096;  // scalars per histogram / scatter tile
-constexpr uint32_t kPackedMaxN = 1u << 23;  // items up to this size sort with one-word entries
+// scalars per histogram / scatter tile: 4096, or 1024 while that leaves fewer
+// than kFewTiles tiles (one workgroup each: 2^17 points had 25 workgroups,
+// digits and histogram 51 us against 18)
+constexpr uint32_t kSortTile = 4096, kSmallTile = 1024, kFewTiles = 512;
+// Items of at most this many scalars are sorted by one workgroup per (item,
+// window) straight from the digits (k_msm_sort_window): no histogram, no
+// scan, no scatter.  Needs the window's buckets as LDS counters.
+constexpr uint32_t kWindowSortMax = 24576, kWindowSortBuckets = 1024;
+// entries a sort group should have at most: what k_msm_sort_group sorts in
+// one read (kGroupMax), less a margin for uneven digits
+constexpr uint32_t kGroupWant = 20000;
 
 // One MSM of a batch as the kernels see it (built on the device).
 struct MsmItemDev {
@@ -114,13 +139,17 @@ constexpr uint32_t kFixedModelMaxC = 17;  // the widest window zk_msm_table_wind
 constexpr uint32_t kFixedMaxBins = 1024, kFixedMaxKeys = 512;
 
 struct MsmPlan {
-    uint32_t count, c, W, B, T1, nbits;
+    uint32_t count, c, W, B;
+    bool quads;          // bucket reduction by quads of lanes (k_msm_bits), else k_msm_reduce_fold
+    uint32_t T1;         // first-level segments per window of k_msm_reduce_fold
+    uint32_t nbits, l1;  // masked sums per window and the weight 2^l1 of the lowest (slice layout)
     uint32_t Wd;     // digit windows per scalar (= W, or ceil(255 / c) with W = 1 in fixed-base mode)
     bool fixed;      // fixed-base mode: points are window tables, one bucket set per item
-    uint32_t hi_bits, lo_bits, nbins;
+    uint32_t hi_bits, lo_bits, nbins, tile;
+    bool window_sort;  // one sort workgroup per (item, window), see kWindowSortMax
     uint64_t ntot, ntiles, nhist, NB, max_entries, chunks;
-    uint32_t chunk;  // sorted entries per accumulation thread
-    bool packed;  // every item has at most kPackedMaxN scalars: one-word sort entries
+    uint32_t chunk;  // smallest number of sorted entries per accumulation thread (see chunk_of)
+    bool packed;  // one-word sort entries: sign, low bucket bits and index fit 32 bits
     size_t size[A_COUNT];
     uint8_t *ptr[A_COUNT];
 };
@@ -129,18 +158,48 @@ __host__ __device__ inline uint64_t align256(uint64_t x) { return (x + 255) & ~(
 
 __host__ __device__ inline uint32_t fixed_windows(uint32_t c) { return (255 + c - 1) / c; }
 
-// high bucket bits of fixed-base mode: as many as the per-tile LDS counters
-// (Wd * 2^hi <= kHistMaxFixed) and the scatter's bins (<= 2^10) allow, so the
-// low-level sort has many groups; the rest (<= 9 bits) are low bits
+// most high bucket bits of fixed-base mode: the per-tile LDS counters (Wd *
+// 2^hi <= kHistMaxFixed) and the scatter's bins (<= 2^10); the rest (<= 9
+// bits) are low bits
 inline uint32_t fixed_hi_bits(uint32_t c) {
     const uint32_t Wd = fixed_windows(c);
     uint32_t hi = 0;
     while (hi < c - 1 && (2u << hi) <= kFixedMaxBins && (uint64_t)Wd * (2u << hi) <= kHistMaxFixed) hi++;
     return hi;
 }
+// the same for plain windows: W * 2^hi <= kHistMax, at most 8
+inline uint32_t plain_hi_bits(uint32_t c) {
+    const uint32_t W = (255 + c - 1) / c;
+    uint32_t hi = 0;
+    while (hi < c - 1 && hi < 8 && (uint64_t)W * (2u << hi) <= kHistMax) hi++;
+    return hi;
+}
 
-// small: the chunk for few entries (see kSmallEntries), else kChunk
-MsmPlan make_plan(const uint32_t *ns, uint32_t count, uint32_t c, bool fixed = false, bool small = true) {
+constexpr uint32_t kBitParts = 5;   // k_msm_bits: T and four masked sums per 16 buckets
+constexpr uint32_t kFoldParts = 8;  // k_msm_reduce_fold: T, six masked sums and A per 64 segments
+
+// workgroups per output of k_msm_bit_sums (B <= 2^17: at most 16, see kQuadBuckets)
+inline uint32_t bit_sum_parts(uint32_t hw) { return hw <= 256 ? 1 : (hw / 256 < 16 ? hw / 256 : 16); }
+
+// Entries per accumulation thread for `total` entries, at least cmin.
+__host__ __device__ inline uint32_t chunk_of(uint32_t total, uint32_t cmin) {
+    uint32_t rounds = (uint32_t)(((uint64_t)total + (uint64_t)kRoundThreads * kChunk - 1) / ((uint64_t)kRoundThreads * kChunk));
+    const uint32_t most = total / (kRoundThreads * kMinChunk);
+    if (rounds < kMinRounds) rounds = most < kMinRounds ? most : kMinRounds;
+    if (rounds < 1) rounds = 1;
+    const uint32_t ch = (uint32_t)(((uint64_t)total + (uint64_t)rounds * kRoundThreads - 1) / ((uint64_t)rounds * kRoundThreads));
+    return ch < cmin ? cmin : ch;
+}
+// The smallest chunk worth room for its partial sums: what chunk_of gives
+// when half of the digits are zero (witness columns).
+inline uint32_t min_chunk(uint64_t max_entries) {
+    const uint32_t ch = chunk_of((uint32_t)(max_entries / 2 < 0x7fffffffu ? max_entries / 2 : 0x7fffffffu), kMinChunk);
+    return ch < kChunk ? ch : kChunk;
+}
+
+// chunk: smallest chunk of the accumulation (the partial sums' arrays are
+// sized for it), 0 = what the pass would like
+MsmPlan make_plan(const uint32_t *ns, uint32_t count, uint32_t c, bool fixed = false, uint32_t chunk = 0) {
     MsmPlan p;
     memset(&p, 0, sizeof(p));
     p.count = count;
@@ -149,41 +208,55 @@ MsmPlan make_plan(const uint32_t *ns, uint32_t count, uint32_t c, bool fixed = f
     p.Wd = (255 + c - 1) / c;
     p.W = fixed ? 1 : p.Wd;
     p.B = 1u << (c - 1);
-    p.T1 = (p.B + kL1 - 1) / kL1;
-    p.nbits = log2_exact(p.T1);
-    if (fixed) {
-        p.hi_bits = fixed_hi_bits(c);
-    } else {
-        // as many high bits (<= 8) as the per-tile LDS counters allow (W *
-        // 2^hi <= kHistMax): the low-level sort gets W * 2^hi groups, so a
-        // narrow window still spreads over the device (c = 13 with 16 bins
-        // had 320 groups of 16K entries: 2^18 points took 0.62 ms to sort)
-        uint32_t hi = 0;
-        while (hi < c - 1 && hi < 8 && (uint64_t)p.W * (2u << hi) <= kHistMax) hi++;
+    uint32_t nmax = 0;
+    for (uint32_t m = 0; m < count; m++) {
+        nmax = ns[m] > nmax ? ns[m] : nmax;
+        p.ntot += ns[m];
+        p.ntiles += (ns[m] + kSortTile - 1) / kSortTile;
+    }
+    p.tile = kSortTile;
+    if (p.ntiles < kFewTiles) {
+        p.tile = kSmallTile;
+        p.ntiles = 0;
+        for (uint32_t m = 0; m < count; m++) p.ntiles += (ns[m] + p.tile - 1) / p.tile;
+    }
+    p.window_sort = !fixed && nmax <= kWindowSortMax && p.B <= kWindowSortBuckets;
+    {
+        // as few high bits as leave groups of kGroupWant entries (longer runs
+        // in the scatter, and in fixed-base mode the smaller kernels: 16
+        // columns of 2^18, scatter 375 -> 211 us and group sort 273 -> 250
+        // with 8 instead of 9 bits and one-word entries), but more while the
+        // low-level sort would have too few workgroups
+        const uint32_t most = fixed ? fixed_hi_bits(c) : plain_hi_bits(c), lo_most = fixed ? 9 : 8;
+        uint32_t hi = c - 1 > lo_most ? c - 1 - lo_most : 0;
+        const uint64_t per = (uint64_t)nmax * (fixed ? p.Wd : 1);  // an item's entries in one bucket set
+        while (hi < most && ((per >> hi) > kGroupWant ||
+                             ((uint64_t)count * p.W << hi) < kFewTiles && (per >> hi) > 2048))
+            hi++;
         p.hi_bits = hi;
     }
     p.lo_bits = (c - 1) - p.hi_bits;
     p.nbins = 1u << p.hi_bits;
-    p.packed = !fixed;  // the virtual indices of fixed-base mode need the two-word entries
-    for (uint32_t m = 0; m < count; m++) {
-        if (ns[m] > kPackedMaxN) p.packed = false;
-        p.ntot += ns[m];
-        p.ntiles += (ns[m] + kSortTile - 1) / kSortTile;
-    }
+    // one word: sign, lo_bits of bucket, the scalar's index (fixed-base: table row)
+    p.packed = (uint64_t)nmax * (fixed ? p.Wd : 1) <= (1ull << (31 - p.lo_bits));
     p.NB = (uint64_t)count * p.W * p.B;
-    p.nhist = (uint64_t)p.Wd * p.nbins * p.ntiles;
+    // a window sort keeps its windows' entry counts in the histogram's place
+    p.nhist = p.window_sort ? (uint64_t)count * p.W : (uint64_t)p.Wd * p.nbins * p.ntiles;
     p.max_entries = p.ntot * p.Wd;
-    p.chunk = kChunk;
-    if (small && p.max_entries < kSmallEntries) {
-        const uint64_t ch = (p.max_entries + kSmallThreads - 1) / kSmallThreads;
-        p.chunk = ch < kMinChunk ? kMinChunk : (uint32_t)ch;
-    }
+    // the reduction's outputs: Q bits 1 .. c - 2 and T + Q_0 by quads, else
+    // the segment bits of k_msm_reduce_fold and the weighted total
+    p.T1 = p.B / kL1;
+    p.quads = p.T1 < 64 || p.NB <= kQuadBuckets;
+    p.l1 = p.quads ? 1 : log2_exact(kL1);
+    p.nbits = p.quads ? c - 2 : log2_exact(p.T1);
+    p.chunk = chunk ? chunk : min_chunk(p.max_entries);
     p.chunks = (p.max_entries + p.chunk - 1) / p.chunk;
     p.size[A_ITEMS] = (size_t)(count + 1) * sizeof(MsmItemDev);
     p.size[A_SLOTS] = (size_t)count * sizeof(uint8_t *);
     p.size[A_OFFSETS] = (size_t)(p.NB + 1) * 4;
     // digits (window-major per item, ntot * W u32) share this array with the entries
     p.size[A_ENTRIES] = (size_t)p.max_entries * 4;
+    // (a window sort writes its entries beside the digits instead)
     p.size[A_TMP] = (size_t)p.max_entries * (p.packed ? 4 : 8);
     p.size[A_HIST] = (size_t)p.nhist * 4;
     p.size[A_STARTS] = (size_t)(p.nhist + 1) * 4;
@@ -191,10 +264,10 @@ MsmPlan make_plan(const uint32_t *ns, uint32_t count, uint32_t c, bool fixed = f
     p.size[A_BUCKETS] = (size_t)p.NB * sizeof(X29S);
     p.size[A_PHEAD] = (size_t)p.chunks * sizeof(X29S);
     p.size[A_PTAIL] = (size_t)p.chunks * sizeof(X29S);
-    p.size[A_HB] = (size_t)p.chunks * 4;
+    const uint32_t hw = (p.B + 15) / 16;
     p.size[A_TB] = (size_t)p.chunks * 4;
-    p.size[A_WS1] = (size_t)count * p.W * p.T1 * sizeof(X29S);
-    p.size[A_SUM1] = (size_t)count * p.W * p.T1 * sizeof(X29S);
+    p.size[A_PART] = p.quads ? (size_t)count * p.W * (hw * kBitParts + (p.nbits + 1) * bit_sum_parts(hw)) * sizeof(X29S)
+                             : (size_t)count * p.W * (p.T1 / 64) * kFoldParts * sizeof(X29S);
     // [count, (bucket, first chunk, last chunk) per bucket spanning > kWalk chunks]
     p.size[A_LONG] = (size_t)(1 + 3 * (p.chunks / kWalk + 1)) * 4;
     return p;
@@ -326,13 +399,19 @@ struct ItemPack {
     uint8_t *slot[kItemsPerLaunch];  // the item's curve slice
     uint32_t first, k;
 };
-__global__ void k_msm_put_items(ItemPack pk, MsmItemDev *__restrict__ items, uint8_t **__restrict__ slots,
-                                uint32_t *__restrict__ long_count) {
+__global__ __launch_bounds__(256) void k_msm_put_items(ItemPack pk, MsmItemDev *__restrict__ items,
+                                                       uint8_t **__restrict__ slots, uint32_t *__restrict__ long_count,
+                                                       uint32_t *__restrict__ wcount, uint32_t nw) {
     uint32_t j = threadIdx.x;
-    if (pk.first == 0 && j == 0) *long_count = 0;
+    if (pk.first == 0) {
+        if (j == 0) *long_count = 0;
+        for (uint32_t k = j; k < nw; k += blockDim.x) wcount[k] = 0;
+    }
     if (j >= pk.k) return;
     items[pk.first + j] = pk.it[j];
     slots[pk.first + j] = pk.slot[j];
+    // the slice's header cleared, so a stale one is never trusted (its first word is the magic)
+    *reinterpret_cast<uint32_t *>(pk.slot[j] + 64) = 0;
 }
 
 // hist index of (item m, digit window w, bin, tile-in-item).  Plain mode:
@@ -350,8 +429,8 @@ __device__ __forceinline__ uint32_t group_tiles(const MsmItemDev &it, uint32_t W
     return fixed ? Wd * it.ntiles : it.ntiles;
 }
 
-// Digits and their histogram in one pass, one block per sort tile (4096
-// scalars of one item, 4 per thread, coalesced).  digits[dig0 + w * n + i] =
+// Digits and their histogram in one pass, one block per sort tile (1024 or
+// 4096 scalars of one item, up to 4 per thread, coalesced).  digits[dig0 + w * n + i] =
 // 0 for a zero digit, else |d| | (d < 0) << 31 with |d| in [1, 2^(c-1)]
 // (bucket |d| - 1); per digit window the counts of the high bucket bits are
 // kept in LDS (Wd * nbins <= HMAX counters: 3840 for every plain window 2 <=
@@ -361,7 +440,7 @@ constexpr uint32_t kDigitThreads = 1024;
 template <uint32_t HMAX>
 __global__ __launch_bounds__(kDigitThreads) void k_msm_digits_hist(const MsmItemDev *__restrict__ items, uint32_t count,
                                                          uint32_t c, uint32_t Wd, uint32_t lo_bits, uint32_t nbins,
-                                                         uint32_t fixed, uint32_t *__restrict__ digits,
+                                                         uint32_t fixed, uint32_t tile, uint32_t *__restrict__ digits,
                                                          uint32_t *__restrict__ hist) {
     __shared__ uint32_t h[HMAX];
     const uint32_t m = item_of(items, count, blockIdx.x);
@@ -371,8 +450,8 @@ __global__ __launch_bounds__(kDigitThreads) void k_msm_digits_hist(const MsmItem
     for (uint32_t k = threadIdx.x; k < nh; k += blockDim.x) h[k] = 0;
     __syncthreads();
     uint32_t *dst = digits + it.dig0;
-    const uint32_t end = (tl + 1) * kSortTile < it.n ? (tl + 1) * kSortTile : it.n;
-    for (uint32_t i = tl * kSortTile + threadIdx.x; i < end; i += blockDim.x) {
+    const uint32_t end = (tl + 1) * tile < it.n ? (tl + 1) * tile : it.n;
+    for (uint32_t i = tl * tile + threadIdx.x; i < end; i += blockDim.x) {
         const Fr s = fe_from_mont<FrParams>(fe_load<FrParams>(&it.scalars[i]));
         uint32_t carry = 0;
         for (uint32_t w = 0; w < Wd; w++) {
@@ -385,6 +464,52 @@ __global__ __launch_bounds__(kDigitThreads) void k_msm_digits_hist(const MsmItem
     __syncthreads();
     for (uint32_t k = threadIdx.x; k < nh; k += blockDim.x)
         hist[hist_index(it, Wd, nbins, fixed != 0, k / nbins, k % nbins, tl)] = h[k];
+}
+
+// Digits for a window sort, one scalar per thread and kDigitWindows windows
+// per workgroup, and per (item, window) the number of nonzero ones (wcount,
+// zeroed before).  With H = sum_{w < W-1} 2^(c w + c - 1) added to the scalar,
+// window w of the sum less 2^(c-1) is a signed digit in [-2^(c-1), 2^(c-1)) of
+// its own (the top one, without the offset, ends the carry chain), so the
+// windows need not be walked in order: 2^12 points took 22 us with one
+// workgroup row doing all 37, 16 with five.
+constexpr uint32_t kDigitWindows = 8;
+struct DigitOffset {
+    uint32_t h[8];
+};
+inline DigitOffset digit_offset(uint32_t c, uint32_t W) {
+    DigitOffset o;
+    memset(&o, 0, sizeof(o));
+    for (uint32_t w = 0; w + 1 < W; w++) {
+        const uint32_t bit = c * w + c - 1;  // below 256: c (W - 1) < 255
+        o.h[bit >> 5] |= 1u << (bit & 31);
+    }
+    return o;
+}
+__global__ __launch_bounds__(256) void k_msm_digits(const MsmItemDev *__restrict__ items, uint32_t count, uint32_t c,
+                                                    uint32_t W, uint32_t tile, const DigitOffset off,
+                                                    uint32_t *__restrict__ digits, uint32_t *__restrict__ wcount) {
+    const uint32_t m = item_of(items, count, blockIdx.x);
+    const MsmItemDev it = items[m];
+    const uint32_t i = (blockIdx.x - it.tile0) * tile + blockIdx.y * blockDim.x + threadIdx.x;
+    if ((i & ~63u) >= it.n) return;  // wave-uniform: i & 63 is the lane
+    const bool live = i < it.n;
+    uint32_t *dst = digits + it.dig0;
+    Fr s = fe_zero<FrParams>();
+    if (live) s = fe_from_mont<FrParams>(fe_load<FrParams>(&it.scalars[i]));
+    uint32_t cy = 0;
+#pragma unroll
+    for (int k = 0; k < 8; k++) s.v[k] = add_cc(s.v[k], off.h[k], cy);
+    const uint32_t w0 = blockIdx.z * kDigitWindows, w1 = w0 + kDigitWindows < W ? w0 + kDigitWindows : W;
+    const int32_t half = 1 << (c - 1);
+    for (uint32_t w = w0; w < w1; w++) {
+        const int32_t v = (int32_t)scalar_bits(s.v, w * c, c);
+        const int32_t d = !live ? 0 : w + 1 < W ? v - half : v;
+        const uint32_t a = (uint32_t)(d < 0 ? -d : d);
+        if (live) dst[(size_t)w * it.n + i] = d ? (a | (d < 0 ? 0x80000000u : 0u)) : 0u;
+        const uint32_t nz = (uint32_t)__builtin_popcountll(__ballot(d != 0));
+        if ((threadIdx.x & 63) == 0 && nz) atomicAdd(&wcount[m * W + w], nz);
+    }
 }
 
 // exclusive scan of x[0..256) in LDS by 256 threads (4 waves): a
@@ -445,23 +570,23 @@ __device__ __forceinline__ void lds_exclusive_scan(uint32_t *x, uint32_t *t) {
 }
 
 // Entries between the two sort levels: (low bucket bits, scalar index |
-// sign << 31), as a pair of words, or packed into one word when every item
-// has at most 2^23 scalars (sign | low bits << 23 | index), which halves the
-// traffic of the pass between the two levels.
+// sign << 31), as a pair of words, or packed into one word (sign | low bits |
+// index) when the index fits the 31 - lo_bits bits left, which halves the
+// traffic of the pass between the two levels.  sh = 31 - lo_bits.
 template <bool kPacked> struct TmpEnt;
 template <> struct TmpEnt<false> {
     using T = uint2;
-    static __device__ __forceinline__ T make(uint32_t lo, uint32_t v) { return make_uint2(lo, v); }
-    static __device__ __forceinline__ uint32_t key(const T &e) { return e.x; }
-    static __device__ __forceinline__ uint32_t val(const T &e) { return e.y; }
+    static __device__ __forceinline__ T make(uint32_t lo, uint32_t v, uint32_t) { return make_uint2(lo, v); }
+    static __device__ __forceinline__ uint32_t key(const T &e, uint32_t) { return e.x; }
+    static __device__ __forceinline__ uint32_t val(const T &e, uint32_t) { return e.y; }
 };
 template <> struct TmpEnt<true> {
     using T = uint32_t;
-    static __device__ __forceinline__ T make(uint32_t lo, uint32_t v) {
-        return (v & 0x80000000u) | (lo << 23) | (v & 0x7fffffu);
+    static __device__ __forceinline__ T make(uint32_t lo, uint32_t v, uint32_t sh) { return v | (lo << sh); }
+    static __device__ __forceinline__ uint32_t key(const T &e, uint32_t sh) { return (e & 0x7fffffffu) >> sh; }
+    static __device__ __forceinline__ uint32_t val(const T &e, uint32_t sh) {
+        return e & (0x80000000u | ((1u << sh) - 1));
     }
-    static __device__ __forceinline__ uint32_t key(const T &e) { return (e >> 23) & 0xffu; }
-    static __device__ __forceinline__ uint32_t val(const T &e) { return e & 0x807fffffu; }
 };
 // per (tile, digit window): place each nonzero digit into its sort group
 // ((item, window, bin), or (item, bin) in fixed-base mode); tmp entry = (low
@@ -475,7 +600,7 @@ template <bool kPacked, uint32_t NBMAX>
 __global__ __launch_bounds__(256) void k_msm_scatter_hi(const MsmItemDev *__restrict__ items, uint32_t count,
                                                         uint32_t Wd, const uint32_t *__restrict__ digits,
                                                         uint32_t lo_bits, uint32_t nbins, uint32_t fixed,
-                                                        const uint32_t *__restrict__ hist,
+                                                        uint32_t tile, const uint32_t *__restrict__ hist,
                                                         const uint32_t *__restrict__ starts,
                                                         typename TmpEnt<kPacked>::T *__restrict__ tmp) {
     using E = TmpEnt<kPacked>;
@@ -504,14 +629,14 @@ __global__ __launch_bounds__(256) void k_msm_scatter_hi(const MsmItemDev *__rest
     const uint32_t *dw = digits + it.dig0 + (size_t)w * it.n;
     const uint32_t vbase = fixed ? w * it.n : 0u;  // fixed-base: the table row of (w, i) is w * n + i
     const uint32_t lo_mask = (1u << lo_bits) - 1;
-    const uint32_t begin = tl * kSortTile;
-    const uint32_t end = begin + kSortTile < it.n ? begin + kSortTile : it.n;
+    const uint32_t begin = tl * tile;
+    const uint32_t end = begin + tile < it.n ? begin + tile : it.n;
     for (uint32_t i = begin + tid; i < end; i += blockDim.x) {
         uint32_t d = dw[i];
         if (d) {
             uint32_t b = (d & 0x7fffffffu) - 1;
             uint32_t p = atomicAdd(&lcur[b >> lo_bits], 1u);
-            stage[p] = E::make(b & lo_mask, (vbase + i) | (d & 0x80000000u));
+            stage[p] = E::make(b & lo_mask, (vbase + i) | (d & 0x80000000u), 31 - lo_bits);
             sbin[p] = (BinT)(b >> lo_bits);
         }
     }
@@ -578,7 +703,7 @@ __global__ __launch_bounds__(kGroupThreads) void k_msm_sort_group(
     const uint32_t gs = starts[idx];
     const uint32_t ge = starts[idx + group_tiles(it, Wd, fixed != 0)];  // the next group's start (or the total)
     const uint32_t tid = threadIdx.x;
-    const uint32_t nlo = 1u << lo_bits;
+    const uint32_t nlo = 1u << lo_bits, sh = 31 - lo_bits;
     const uint64_t base = ((uint64_t)m * W + w) * B + ((uint64_t)bin << lo_bits);
     if (g == ngroups - 1 && tid == 0) offsets[base + nlo] = ge;  // = total: offsets[NB]
     typename E::T v[kGroupPer];
@@ -591,7 +716,7 @@ __global__ __launch_bounds__(kGroupThreads) void k_msm_sort_group(
             const uint32_t q = k * kGroupThreads + tid;
             if (q < cnt) {
                 v[k] = tmp[gs + q];
-                atomicAdd(&h[E::key(v[k])], 1u);
+                atomicAdd(&h[E::key(v[k], sh)], 1u);
             }
         }
         __syncthreads();
@@ -601,7 +726,7 @@ __global__ __launch_bounds__(kGroupThreads) void k_msm_sort_group(
 #pragma unroll
         for (uint32_t k = 0; k < kGroupPer; k++) {
             const uint32_t q = k * kGroupThreads + tid;
-            if (q < cnt) stage[atomicAdd(&h[E::key(v[k])], 1u)] = E::val(v[k]);
+            if (q < cnt) stage[atomicAdd(&h[E::key(v[k], sh)], 1u)] = E::val(v[k], sh);
         }
         __syncthreads();
         for (uint32_t q = tid; q < cnt; q += kGroupThreads) entries[gs + q] = stage[q];
@@ -610,7 +735,7 @@ __global__ __launch_bounds__(kGroupThreads) void k_msm_sort_group(
     // a larger group: bucket offsets from a counting pass over the group
     for (uint32_t k = tid; k < KEYS; k += kGroupThreads) cur[k] = 0;
     __syncthreads();
-    for (uint32_t p = gs + tid; p < ge; p += kGroupThreads) atomicAdd(&cur[E::key(tmp[p])], 1u);
+    for (uint32_t p = gs + tid; p < ge; p += kGroupThreads) atomicAdd(&cur[E::key(tmp[p], sh)], 1u);
     __syncthreads();
     lds_exclusive_scan1024<KEYS>(cur, sc);
     for (uint32_t k = tid; k < KEYS; k += kGroupThreads) cur[k] += gs;
@@ -625,7 +750,7 @@ __global__ __launch_bounds__(kGroupThreads) void k_msm_sort_group(
             const uint32_t q = k * kGroupThreads + tid;
             if (q < cnt) {
                 v[k] = tmp[t0 + q];
-                atomicAdd(&th[E::key(v[k])], 1u);
+                atomicAdd(&th[E::key(v[k], sh)], 1u);
             }
         }
         __syncthreads();
@@ -638,9 +763,9 @@ __global__ __launch_bounds__(kGroupThreads) void k_msm_sort_group(
         for (uint32_t k = 0; k < kGroupPer; k++) {
             const uint32_t q = k * kGroupThreads + tid;
             if (q < cnt) {
-                const uint32_t key = E::key(v[k]);
+                const uint32_t key = E::key(v[k], sh);
                 const uint32_t at = atomicAdd(&tcur[key], 1u);
-                stage[at] = E::val(v[k]);
+                stage[at] = E::val(v[k], sh);
                 skey[at] = (KeyT)key;
             }
         }
@@ -653,6 +778,49 @@ __global__ __launch_bounds__(kGroupThreads) void k_msm_sort_group(
         for (uint32_t k = tid; k < KEYS; k += kGroupThreads) cur[k] += th[k];
         __syncthreads();
     }
+}
+
+// Window sort: one block of 1024 threads per (item, window) group g sorts the
+// window's nonzero digits (at most kWindowSortMax) by bucket, straight from
+// the digit array, and writes the bucket offsets.  The group starts at the sum
+// of the earlier groups' counts.  Dynamic LDS: the largest item's scalars.
+__global__ __launch_bounds__(kGroupThreads) void k_msm_sort_window(const MsmItemDev *__restrict__ items, uint32_t W,
+                                                                   uint32_t B, uint32_t ngroups,
+                                                                   const uint32_t *__restrict__ digits,
+                                                                   const uint32_t *__restrict__ wcount,
+                                                                   uint32_t *__restrict__ entries,
+                                                                   uint32_t *__restrict__ offsets) {
+    extern __shared__ uint32_t stage[];
+    __shared__ uint32_t h[kWindowSortBuckets], sc[kGroupThreads / 64], start;
+    const uint32_t g = blockIdx.x, m = g / W, w = g % W, tid = threadIdx.x;
+    const MsmItemDev it = items[m];
+    if (tid == 0) start = 0;
+    h[tid] = 0;
+    __syncthreads();
+    uint32_t before = 0;
+    for (uint32_t k = tid; k < g; k += kGroupThreads) before += wcount[k];
+    if (before) atomicAdd(&start, before);
+    const uint32_t *dw = digits + it.dig0 + (size_t)w * it.n;
+    uint32_t v[kGroupPer];
+#pragma unroll
+    for (uint32_t k = 0; k < kGroupPer; k++) {
+        const uint32_t i = k * kGroupThreads + tid;
+        v[k] = i < it.n ? dw[i] : 0u;
+        if (v[k]) atomicAdd(&h[(v[k] & 0x7fffffffu) - 1], 1u);
+    }
+    __syncthreads();
+    lds_exclusive_scan1024<kWindowSortBuckets>(h, sc);
+    const uint32_t gs = start, cnt = wcount[g];
+    if (tid < B) offsets[(size_t)g * B + tid] = gs + h[tid];
+    if (g == ngroups - 1 && tid == 0) offsets[(size_t)ngroups * B] = gs + cnt;
+    __syncthreads();  // h becomes the cursors
+#pragma unroll
+    for (uint32_t k = 0; k < kGroupPer; k++)
+        if (v[k])
+            stage[atomicAdd(&h[(v[k] & 0x7fffffffu) - 1], 1u)] =
+                (k * kGroupThreads + tid) | (v[k] & 0x80000000u);
+    __syncthreads();
+    for (uint32_t p = tid; p < cnt; p += kGroupThreads) entries[gs + p] = stage[p];
 }
 
 // ---- exclusive scan of u32 counts (3 kernels) ---------------------------
@@ -735,15 +903,16 @@ __global__ __launch_bounds__(256) void k_msm_accumulate(const uint32_t *__restri
                                                         const uint32_t *__restrict__ off, uint32_t NB, uint32_t WB,
                                                         const MsmItemDev *__restrict__ items,
                                                         X29S *__restrict__ buckets, X29S *__restrict__ phead,
-                                                        X29S *__restrict__ ptail, uint32_t *__restrict__ hb,
-                                                        uint32_t *__restrict__ tb, uint64_t nchunks, uint32_t chunk) {
+                                                        X29S *__restrict__ ptail, uint32_t *__restrict__ tb,
+                                                        uint64_t nchunks, uint32_t cmin) {
     uint64_t t = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (t >= nchunks) return;
-    const uint32_t total = off[NB];
-    const uint32_t s = (uint32_t)(t * chunk);
-    uint32_t head_bucket = kNone, tail_bucket = kNone;
-    if (s < total) {
-        const uint32_t e = s + chunk < total ? s + chunk : total;
+    const uint32_t total = off[NB], chunk = chunk_of(total, cmin);
+    const uint64_t s64 = t * chunk;
+    uint32_t tail_bucket = kNone;
+    if (s64 < total) {
+        const uint32_t s = (uint32_t)s64;
+        const uint32_t e = total - s > chunk ? s + chunk : total;
         uint32_t b = find_bucket(off, NB, s);
         uint32_t bend = off[b + 1];
         bool first = true, before = off[b] < s;
@@ -783,7 +952,6 @@ __global__ __launch_bounds__(256) void k_msm_accumulate(const uint32_t *__restri
                 // form: the fixup and the reduction continue in it)
                 if (first && before) {
                     x29_store_acc(&phead[t], acc, empty);
-                    head_bucket = b;
                 } else if (bend > e) {
                     x29_store_acc(&ptail[t], acc, empty);
                     tail_bucket = b;
@@ -809,74 +977,107 @@ __global__ __launch_bounds__(256) void k_msm_accumulate(const uint32_t *__restri
             qcur = qnext;
         }
     }
-    hb[t] = head_bucket;
     tb[t] = tail_bucket;
 }
 
-// merges the partial sums of buckets that span several chunks.  A bucket b
-// whose run starts in chunk t (tail partial) ends in chunk t' = (off[b+1]-1) /
-// chunk, and chunks t+1..t' all hold head partials of b.  Spans up to kWalk
-// chunks are summed by the thread; longer ones (few: their count is at most
-// nchunks / kWalk) are listed for k_msm_fixup_long, one workgroup each, so a
-// heavy bucket (e.g. the multiplicities of a lookup, all in a handful of
-// buckets) never becomes a serial chain.
+// merges the partial sums of buckets that span several chunks, one quad of
+// lanes per bucket: bucket b's entries [off[b], off[b+1]) start in chunk t and
+// end in chunk t', chunk t holds the tail partial and chunks t+1..t' head
+// partials of b.  The quads are numbered by bucket when an average bucket
+// is longer than a chunk (nearly all have something to merge), else by chunk
+// t (nearly all end inside a bucket, tb[t]); the other way round a wave works
+// for a few of its quads only (2^12 points, 8 chunks per bucket: 41 us by
+// bucket, 112 by chunk; 16 columns of 2^18, a third of a chunk per bucket: 36 us
+// by chunk, 176 by bucket).  Spans of more than kWalk chunks (few: their
+// count is at most nchunks / kWalk) are listed for k_msm_fixup_long, one
+// workgroup each, so a heavy bucket (e.g. the multiplicities of a lookup, all
+// in a handful of buckets) never becomes a serial chain.  The chains are what
+// this takes (the additions themselves are few), hence quads.
 __global__ __launch_bounds__(256) void k_msm_fixup(X29S *__restrict__ buckets, const X29S *__restrict__ phead,
                                                    const X29S *__restrict__ ptail, const uint32_t *__restrict__ tb,
-                                                   const uint32_t *__restrict__ off, uint32_t *__restrict__ longs,
-                                                   uint64_t nchunks, uint32_t chunk) {
-    uint64_t t = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (t >= nchunks) return;
-    uint32_t b = tb[t];
-    if (b == kNone) return;
-    const uint64_t last = (uint64_t)(off[b + 1] - 1) / chunk;
+                                                   const uint32_t *__restrict__ off, uint32_t NB,
+                                                   uint32_t *__restrict__ longs, uint32_t nchunks, uint32_t cmin) {
+    const uint32_t i = (uint32_t)(((uint64_t)blockIdx.x * blockDim.x + threadIdx.x) >> 2);
+    const uint32_t q = threadIdx.x & 3;
+    const uint32_t total = off[NB], chunk = chunk_of(total, cmin);
+    uint32_t b = i;
+    if ((uint64_t)chunk * NB > total) {
+        if (i >= nchunks) return;
+        b = tb[i];
+    }
+    if (b >= NB) return;  // kNone: the chunk ends where a bucket does
+    const uint32_t lo = off[b], hi = off[b + 1];
+    if (lo == hi) return;
+    const uint32_t t = lo / chunk, last = (hi - 1) / chunk;
+    if (t == last) return;  // one chunk owned the whole run and stored it
     if (last - t > kWalk) {
-        uint32_t i = atomicAdd(&longs[0], 1u);
-        longs[1 + 3 * i] = b;
-        longs[2 + 3 * i] = (uint32_t)t;
-        longs[3 + 3 * i] = (uint32_t)last;
+        if (q == 0) {
+            const uint32_t k = atomicAdd(&longs[0], 1u);
+            longs[1 + 3 * k] = b;
+            longs[2 + 3 * k] = t;
+            longs[3 + 3 * k] = last;
+        }
         return;
     }
     bool ae, qe;
-    X29 acc = x29_load(&ptail[t], ae);
-    for (uint64_t u = t + 1; u <= last; u++) {
-        const X29 q = x29_load(&phead[u], qe);
-        x29_add(acc, ae, q, qe);
+    Q29 acc = q29_load(&ptail[t], ae, q);
+    Q29 nxt = q29_load(&phead[t + 1], qe, q);
+    for (uint32_t u = t + 1; u <= last; u++) {
+        const Q29 cur = nxt;
+        const bool ce = qe;
+        // unconditional, so that the load stays in flight during the addition
+        nxt = q29_load(&phead[u < last ? u + 1 : last], qe, q);
+        q29_add(acc, ae, cur, ce, q);
     }
-    x29_store(&buckets[b], acc, ae);
+    q29_store(&buckets[b], acc, ae, q);
 }
 
-// one workgroup per listed long bucket: ptail[t] + sum of phead[t+1..last]
+// sum over the wave's 16 quads (the result in every quad)
+__device__ __forceinline__ void q29_wave_sum(Q29 &p, bool &pe, uint32_t q) {
+#pragma unroll 1
+    for (int m = 4; m < 64; m <<= 1) {
+        bool oe;
+        const Q29 o = q29_shfl_xor(p, pe, oe, m);
+        q29_add(p, pe, o, oe, q);
+    }
+}
+// sum over the quads of a workgroup of at most 256 threads, in wave 0's quads
+__device__ __forceinline__ void q29_block_sum(Q29 &p, bool &pe, uint32_t q, X29S *sh) {
+    q29_wave_sum(p, pe, q);
+    const uint32_t lane = threadIdx.x & 63, wv = threadIdx.x >> 6, waves = blockDim.x >> 6;
+    if (waves == 1) return;
+    if (lane < 4) q29_store(&sh[wv], p, pe, q);
+    __syncthreads();
+    if (wv == 0) {
+#pragma unroll 1
+        for (uint32_t k = 1; k < waves; k++) {
+            bool oe;
+            const Q29 o = q29_load(&sh[k], oe, q);
+            q29_add(p, pe, o, oe, q);
+        }
+    }
+    __syncthreads();
+}
+
+// one workgroup of 64 quads per listed long bucket: ptail[t] + sum of
+// phead[t+1..last]
 __global__ __launch_bounds__(256) void k_msm_fixup_long(X29S *__restrict__ buckets,
                                                         const X29S *__restrict__ phead,
                                                         const X29S *__restrict__ ptail,
                                                         const uint32_t *__restrict__ longs) {
-    __shared__ X29S sh[256];
-    const uint32_t count = longs[0];
+    __shared__ X29S sh[4];
+    const uint32_t count = longs[0], q = threadIdx.x & 3, quad = threadIdx.x >> 2;
     for (uint32_t i = blockIdx.x; i < count; i += gridDim.x) {
         const uint32_t b = longs[1 + 3 * i], t = longs[2 + 3 * i], last = longs[3 + 3 * i];
         bool ae = true, qe;
-        X29 acc;
-        if (threadIdx.x == 0) acc = x29_load(&ptail[t], ae);
-        for (uint32_t u = t + 1 + threadIdx.x; u <= last; u += blockDim.x) {
-            const X29 q = x29_load(&phead[u], qe);
-            x29_add(acc, ae, q, qe);
+        Q29 acc{};
+        if (quad == 0) acc = q29_load(&ptail[t], ae, q);
+        for (uint32_t u = t + 1 + quad; u <= last; u += blockDim.x / 4) {
+            const Q29 v = q29_load(&phead[u], qe, q);
+            q29_add(acc, ae, v, qe, q);
         }
-        x29_store(&sh[threadIdx.x], acc, ae);
-        __syncthreads();
-        for (uint32_t st = 128; st; st >>= 1) {
-            if (threadIdx.x < st) {
-                X29 l = x29_load(&sh[threadIdx.x], ae);
-                const X29 r = x29_load(&sh[threadIdx.x + st], qe);
-                x29_add(l, ae, r, qe);
-                x29_store(&sh[threadIdx.x], l, ae);
-            }
-            __syncthreads();
-        }
-        if (threadIdx.x == 0) {
-            const X29 r = x29_load(&sh[0], ae);
-            x29_store(&buckets[b], r, ae);
-        }
-        __syncthreads();
+        q29_block_sum(acc, ae, q, sh);
+        if (threadIdx.x < 4) q29_store(&buckets[b], acc, ae, q);
     }
 }
 
@@ -885,27 +1086,17 @@ __global__ __launch_bounds__(256) void k_msm_fixup_long(X29S *__restrict__ bucke
 // directly.  Empty buckets are never read (their count is zero).
 
 // ---- reduction -------------------------------------------------------------
-// one thread per (item window, segment of kL1 buckets); W = items * windows
-__global__ __launch_bounds__(64) void k_msm_reduce_l1(const X29S *__restrict__ buckets, const uint32_t *__restrict__ off,
-                                uint32_t W, uint32_t B, uint32_t T1, X29S *__restrict__ ws1,
-                                X29S *__restrict__ sum1) {
-    uint32_t g = blockIdx.x * blockDim.x + threadIdx.x;
-    if (g >= W * T1) return;
-    uint32_t w = g / T1, s = g % T1;
-    X29 run, acc;
-    bool re = true, ae = true, be;
-    uint32_t lo = s * kL1;
-    uint32_t hi = lo + kL1 < B ? lo + kL1 : B;
-    for (uint32_t b = hi; b-- > lo;) {
-        uint32_t idx = w * B + b;
-        if (off[idx + 1] != off[idx]) {
-            const X29 q = x29_load(&buckets[idx], be);
-            x29_add(run, re, q, be);
-        }
-        x29_add(acc, ae, run, re);
-    }
-    x29_store(&ws1[g], acc, ae);
-    x29_store(&sum1[g], run, re);
+struct SliceHeader {
+    uint32_t magic, c, W, nbits, l1, pad[3];
+};
+// the slice's header, written by the last kernel of the pipeline
+__device__ __forceinline__ void slice_header(uint8_t *slice, uint32_t c, uint32_t W, uint32_t nbits, uint32_t l1) {
+    SliceHeader *h = reinterpret_cast<SliceHeader *>(slice + 64);
+    h->c = c;
+    h->W = W;
+    h->nbits = nbits;
+    h->l1 = l1;
+    h->magic = kMagic;
 }
 
 // the item window g's masked sum Q[bit] in its curve slice
@@ -940,8 +1131,8 @@ __device__ __forceinline__ X29 x29_select(bool c, const X29 &a, const X29 &b) {
 
 // Level-1 reduction with the masked sums folded in (T1 >= 64): one wave per 64
 // consecutive segments s = 64 h + lane of an item window g.  Each lane forms
-// its segment's run (plain sum of its kL1 buckets) and acc (weighted sum) as
-// k_msm_reduce_l1 does; then six butterfly steps over the lanes: at step k a
+// its segment's run (plain sum of its kL1 buckets) and acc (sum weighted 1 ..
+// kL1); then six butterfly steps over the lanes: at step k a
 // lane with bit k clear adds its partner's run, a lane with bit k set its
 // partner's acc, so every lane does one point addition per step.  Afterwards
 // lane 0 holds the wave's total run T, lane 2^j (j < 6) the sum of the runs
@@ -997,7 +1188,7 @@ __global__ __launch_bounds__(64) void k_msm_reduce_fold(const X29S *__restrict__
 // the waves' lane-bit partials j = o; 6 <= o < nbits: sum of the totals T_h
 // of the waves with bit o - 6 of h set; o = nbits: sum of the waves' A.
 __global__ __launch_bounds__(64) void k_msm_fold_sums(const X29S *__restrict__ part, uint32_t T1, uint32_t nbits,
-                                                      uint32_t W, uint8_t *const *__restrict__ slots) {
+                                                      uint32_t c, uint32_t W, uint8_t *const *__restrict__ slots) {
     const uint32_t o = blockIdx.x, g = blockIdx.y, lane = threadIdx.x, hw = T1 >> 6;
     const uint32_t slot = o < 6 ? 1 + o : (o < nbits ? 0 : 7);
     X29 acc;
@@ -1014,92 +1205,99 @@ __global__ __launch_bounds__(64) void k_msm_fold_sums(const X29S *__restrict__ p
         x29_shfl_xor(q, qe, acc, ae, 1 << k);
         x29_add(acc, ae, q, qe);
     }
-    if (lane == 0) xyzz_store(slot_q(slots, g, W, nbits, o), x29_to_xyzz(acc, ae));
-}
-
-// grid (nbits + 1, items * W, parts): q < nbits -> sum of sum1[g][s] over s
-// with bit q set; q == nbits -> sum of ws1[g][s] over all s.  With one part
-// the sum goes into the item's curve slice at Q[w][q]; with several, block z
-// sums the z-th slice of s into qpart[(g * (nbits + 1) + q) * parts + z] and
-// k_msm_masked_merge adds the parts (a single MSM has only (nbits+1) * W
-// sums, too few workgroups to fill the device).
-// LDS tree over the 256 threads' X29 values in sh; the sum ends in sh[0]
-__device__ __forceinline__ void x29_block_tree(X29S *sh) {
-    bool ae, qe;
-    for (uint32_t st = 128; st; st >>= 1) {
-        if (threadIdx.x < st) {
-            X29 l = x29_load(&sh[threadIdx.x], ae);
-            const X29 r = x29_load(&sh[threadIdx.x + st], qe);
-            x29_add(l, ae, r, qe);
-            x29_store(&sh[threadIdx.x], l, ae);
-        }
-        __syncthreads();
+    if (lane == 0) {
+        xyzz_store(slot_q(slots, g, W, nbits, o), x29_to_xyzz(acc, ae));
+        if (o == nbits && g % W == 0) slice_header(slots[g / W], c, W, nbits, __builtin_ctz(kL1));
     }
 }
 
-__global__ __launch_bounds__(256) void k_msm_masked_sums(const X29S *__restrict__ ws1,
-                                                         const X29S *__restrict__ sum1, uint32_t T1,
-                                                         uint32_t nbits, uint32_t W,
-                                                         uint8_t *const *__restrict__ slots,
-                                                         X29S *__restrict__ qpart) {
-    __shared__ X29S sh[256];
-    const uint32_t bit = blockIdx.x, g = blockIdx.y, parts = gridDim.z, part = blockIdx.z;
-    const uint32_t span = T1 / parts, s0 = part * span;
-    const X29S *src = (bit == nbits ? ws1 : sum1) + (size_t)g * T1;
-    X29 acc;
-    bool ae = true, qe;
-    for (uint32_t s = s0 + threadIdx.x; s < s0 + span; s += blockDim.x) {
-        if (bit == nbits || ((s >> bit) & 1u)) {
-            const X29 q = x29_load(&src[s], qe);
-            x29_add(acc, ae, q, qe);
+// Bucket reduction by quads of lanes, one wave per 16 consecutive buckets b =
+// 16 h + i of an item window g (padded with empty ones when B < 16): S_w =
+// sum_b (b + 1) B_b = T + sum_k 2^k Q_k with T the sum of all buckets and Q_k
+// that of the buckets with bit k of b set.  Four butterfly steps over the
+// quads: at step k a quad with bit k of i clear adds its partner's value;
+// afterwards quad 0 holds the wave's T and quad 2^k its Q_k (k < 4).  They go
+// to part[(g * hw + h) * kBitParts + {0, 1 + k}] for k_msm_bit_sums.
+__global__ __launch_bounds__(256) void k_msm_bits(const X29S *__restrict__ buckets, const uint32_t *__restrict__ off,
+                                                  uint32_t B, uint32_t hw, uint32_t nwaves,
+                                                  X29S *__restrict__ part) {
+    const uint32_t gh = (blockIdx.x * blockDim.x + threadIdx.x) >> 6;
+    if (gh >= nwaves) return;
+    const uint32_t g = gh / hw, h = gh % hw;
+    const uint32_t i = (threadIdx.x & 63) >> 2, q = threadIdx.x & 3;
+    const uint32_t b = h * 16 + i, idx = g * B + b;
+    Q29 p{};
+    bool pe = true;
+    if (b < B && off[idx + 1] != off[idx]) p = q29_load(&buckets[idx], pe, q);
+#pragma unroll 1
+    for (int k = 0; k < 4; k++) {
+        bool oe;
+        const Q29 o = q29_shfl_xor(p, pe, oe, 4 << k);
+        if (!((i >> k) & 1u)) q29_add(p, pe, o, oe, q);
+    }
+    X29S *dst = part + (size_t)gh * kBitParts;
+    if (i == 0)
+        q29_store(&dst[0], p, pe, q);
+    else if ((i & (i - 1)) == 0)
+        q29_store(&dst[1 + __builtin_ctz(i)], p, pe, q);
+}
+
+// lane q's coordinate of a masked sum into its curve slice (the identity as
+// (1, 1, 0, 0)), and with the item's last one its header
+__device__ __forceinline__ void q29_slot_store(uint8_t *const *slots, uint32_t g, uint32_t c, uint32_t W, uint32_t o,
+                                               const Q29 &p, bool pe, uint32_t q) {
+    const uint32_t nbits = c - 2;
+    Fp v = q < 2 ? fe_one<FpParams>() : fe_zero<FpParams>();
+    if (!pe) v = f29_to32(p.c);
+    fe_store<FpParams>(reinterpret_cast<Fp *>(slot_q(slots, g, W, nbits, o)) + q, v);
+    if (q == 0 && o == nbits && g % W == 0) slice_header(slots[g / W], c, W, nbits, 1);
+}
+
+// grid (nbits + 1, gw, parts), nbits = c - 2: the item window's outputs from
+// the partials of k_msm_bits.  o < nbits: Q_k for k = o + 1 (k < 4: the sum of
+// the waves' Q_k; else the sum of T_h over the waves with bit k - 4 of h set);
+// o = nbits: T + Q_0.  With several parts (wide windows: up to 256 waves
+// each), part z's sum goes to qpart[(g * (nbits + 1) + o) * parts + z] for
+// k_msm_bit_merge.
+__global__ __launch_bounds__(256) void k_msm_bit_sums(const X29S *__restrict__ part, uint32_t hw, uint32_t c,
+                                                      uint32_t W, uint8_t *const *__restrict__ slots,
+                                                      X29S *__restrict__ qpart) {
+    __shared__ X29S sh[4];
+    const uint32_t o = blockIdx.x, g = blockIdx.y, nbits = c - 2, k = o + 1, parts = gridDim.z;
+    const uint32_t q = threadIdx.x & 3, span = (hw + parts - 1) / parts, h0 = blockIdx.z * span;
+    const uint32_t h1 = h0 + span < hw ? h0 + span : hw;
+    const X29S *src = part + (size_t)g * hw * kBitParts;
+    Q29 acc{};
+    bool ae = true, ve;
+    for (uint32_t h = h0 + (threadIdx.x >> 2); h < h1; h += blockDim.x >> 2) {
+        if (o == nbits || k < 4 || ((h >> (k - 4)) & 1u)) {
+            const Q29 v = q29_load(&src[h * kBitParts + (o < nbits && k < 4 ? 1 + k : 0)], ve, q);
+            q29_add(acc, ae, v, ve, q);
+        }
+        if (o == nbits) {
+            const Q29 v = q29_load(&src[h * kBitParts + 1], ve, q);
+            q29_add(acc, ae, v, ve, q);
         }
     }
-    x29_store(&sh[threadIdx.x], acc, ae);
-    __syncthreads();
-    x29_block_tree(sh);
-    if (threadIdx.x == 0) {
-        const X29 r = x29_load(&sh[0], ae);
+    q29_block_sum(acc, ae, q, sh);
+    if (threadIdx.x < 4) {
         if (parts == 1)
-            xyzz_store(slot_q(slots, g, W, nbits, bit), x29_to_xyzz(r, ae));
+            q29_slot_store(slots, g, c, W, o, acc, ae, q);
         else
-            x29_store(&qpart[((size_t)g * (nbits + 1) + bit) * parts + part], r, ae);
+            q29_store(&qpart[((size_t)g * (nbits + 1) + o) * parts + blockIdx.z], acc, ae, q);
     }
 }
 
-// the parts of each (item window, bit) sum: a workgroup takes 256 / parts
-// sums, one thread per part, and adds them as a tree in LDS
-__global__ __launch_bounds__(256) void k_msm_masked_merge(const X29S *__restrict__ qpart, uint32_t parts,
-                                                          uint32_t nbits, uint32_t W, uint32_t gw,
-                                                          uint8_t *const *__restrict__ slots) {
-    __shared__ X29S sh[256];
-    const uint32_t per = 256 / parts, z = threadIdx.x % parts;
-    const uint64_t total = (uint64_t)gw * (nbits + 1);
-    const uint64_t i = (uint64_t)blockIdx.x * per + threadIdx.x / parts;
-    const bool live = i < total;
-    bool ae = true, qe;
-    X29 v;
-    if (live) v = x29_load(&qpart[i * parts + z], ae);
-    x29_store(&sh[threadIdx.x], v, ae);
-    __syncthreads();
-    for (uint32_t st = parts / 2; st; st >>= 1) {
-        if (z < st) {
-            X29 l = x29_load(&sh[threadIdx.x], ae);
-            const X29 r = x29_load(&sh[threadIdx.x + st], qe);
-            x29_add(l, ae, r, qe);
-            x29_store(&sh[threadIdx.x], l, ae);
-        }
-        __syncthreads();
-    }
-    if (live && z == 0) {
-        const X29 r = x29_load(&sh[threadIdx.x], ae);
-        xyzz_store(slot_q(slots, (uint32_t)(i / (nbits + 1)), W, nbits, (uint32_t)(i % (nbits + 1))),
-                   x29_to_xyzz(r, ae));
-    }
+// grid (nbits + 1, gw), one wave: adds the parts (at most 16) of each sum
+__global__ __launch_bounds__(64) void k_msm_bit_merge(const X29S *__restrict__ qpart, uint32_t parts, uint32_t c,
+                                                      uint32_t W, uint8_t *const *__restrict__ slots) {
+    const uint32_t o = blockIdx.x, g = blockIdx.y, z = threadIdx.x >> 2, q = threadIdx.x & 3;
+    Q29 p{};
+    bool pe = true;
+    if (z < parts) p = q29_load(&qpart[((size_t)g * (c - 1) + o) * parts + z], pe, q);
+    q29_wave_sum(p, pe, q);
+    if (threadIdx.x < 4) q29_slot_store(slots, g, c, W, o, p, pe, q);
 }
-
-struct SliceHeader {
-    uint32_t magic, c, W, nbits, pad[4];
-};
 
 __host__ __device__ inline size_t slice_sums_off(uint32_t W, uint32_t nbits) {
     return kSliceQ + (size_t)W * (nbits + 1) * sizeof(G1Xyzz);
@@ -1108,22 +1306,13 @@ __host__ __device__ inline size_t slice_bytes_needed(uint32_t W, uint32_t nbits)
     return slice_sums_off(W, nbits) + (size_t)W * sizeof(G1Jac);
 }
 
-__global__ void k_slice_header(uint8_t *const *slots, uint32_t count, uint32_t c, uint32_t W, uint32_t nbits) {
-    uint32_t m = blockIdx.x * blockDim.x + threadIdx.x;
-    if (m >= count) return;
-    SliceHeader *h = reinterpret_cast<SliceHeader *>(slots[m] + 64);
-    h->c = c;
-    h->W = W;
-    h->nbits = nbits;
-    h->magic = kMagic;
-}
-
 __host__ __device__ __forceinline__ bool header_ok(const SliceHeader *h) {
-    return h->magic == kMagic && h->W >= 1 && h->W <= 128 && h->c >= 2 && h->c <= kFixedMaxC && h->nbits <= 16;
+    return h->magic == kMagic && h->W >= 1 && h->W <= 128 && h->c >= 2 && h->c <= kFixedMaxC && h->nbits <= 16 &&
+           h->l1 <= 3;
 }
 
 // Device tail, step 1 (grid: W threads per slice, y = slice):
-// S_w = A + L1 * sum_bit 2^bit Q_bit, written to the slice's S array.
+// S_w = Q[nbits] + 2^l1 * sum_bit 2^bit Q[bit], written to the slice's S array.
 __global__ __launch_bounds__(64) void k_msm_window_finalize(uint8_t *const *__restrict__ slices) {
     uint8_t *slice = slices[blockIdx.y];
     const SliceHeader *h = reinterpret_cast<const SliceHeader *>(slice + 64);
@@ -1137,7 +1326,7 @@ __global__ __launch_bounds__(64) void k_msm_window_finalize(uint8_t *const *__re
         acc = jac_dbl(acc);
         acc = jac_add(acc, xyzz_to_jac(xyzz_load(&qw[b])));
     }
-    for (uint32_t k = 1; k < kL1; k <<= 1) acc = jac_dbl(acc);
+    for (uint32_t k = 0; k < h->l1; k++) acc = jac_dbl(acc);
     acc = jac_add(acc, xyzz_to_jac(xyzz_load(&qw[nbits])));
     jac_store(reinterpret_cast<G1Jac *>(slice + slice_sums_off(W, nbits)) + w, acc);
 }
@@ -1167,12 +1356,6 @@ __global__ __launch_bounds__(64) void k_msm_collect(uint8_t *const *__restrict__
     uint32_t m = blockIdx.x * blockDim.x + threadIdx.x;
     if (m >= batch) return;
     collect_slice(slices[m]);
-}
-
-// device-side slice header reset so a stale header is never trusted
-__global__ void k_slice_clear(uint8_t *const *slots, uint32_t count) {
-    uint32_t m = blockIdx.x * blockDim.x + threadIdx.x;
-    if (m < count) reinterpret_cast<SliceHeader *>(slots[m] + 64)->magic = 0;
 }
 
 // Fixed-base table T[w * n + i] = 2^(c w) P_i for w < Wd (affine, Montgomery,
@@ -1295,6 +1478,28 @@ size_t msm_scratch_bytes(const uint32_t *ns, uint32_t count, uint32_t c, bool fi
     return plan_total(make_plan(ns, count, c, fixed));
 }
 uint32_t msm_default_window(uint32_t n) { return default_window(n); }
+// The size by which zk_msm_noalloc accepts or refuses an MSM of n points at
+// window c (0 = default): one block per array of a fixed layout (4096-scalar
+// sort tiles, chunks of 96 entries, or 2^16 of at least 8 below 2^21 entries).
+// A limit of that entry only, kept apart from the plan, which sizes its
+// chunks to the room there is and fits wherever this does.
+size_t msm_noalloc_bytes(uint32_t n, uint32_t c) {
+    if (!c) c = default_window(n);
+    const uint64_t W = (255 + c - 1) / c, B = 1ull << (c - 1), NB = W * B, entries = (uint64_t)n * W;
+    uint64_t bins = 1;
+    while (bins < B && bins < 256 && W * 2 * bins <= kHistMax) bins *= 2;
+    const uint64_t hist = W * bins * ((n + kSortTile - 1) / kSortTile);
+    const uint64_t chunk = entries < (1u << 21) ? std::max<uint64_t>(8, (entries + 65535) / 65536) : 96;
+    const uint64_t chunks = (entries + chunk - 1) / chunk, segs = W * ((B + 7) / 8);
+    const uint64_t arrays[] = {2 * sizeof(MsmItemDev), 8, (NB + 1) * 4, entries * 4,
+                               (1 + 3 * (chunks / 32 + 1)) * 4, entries * (n > (1u << 23) ? 8 : 4),
+                               hist * 4, (hist + 1) * 4, ((hist + 1 + 1023) / 1024 + 1) * 4,
+                               NB * sizeof(X29S), chunks * sizeof(X29S), chunks * sizeof(X29S),
+                               chunks * 4, chunks * 4, segs * sizeof(X29S), segs * sizeof(X29S)};
+    size_t t = 256 + 256;
+    for (const uint64_t a : arrays) t += align256(a);
+    return t;
+}
 // window for a batch: the default for its mean size
 uint32_t batch_default_window(const uint32_t *ns, uint32_t count) {
     uint64_t t = 0;
@@ -1317,14 +1522,15 @@ bool choose_plan(const uint32_t *ns, uint32_t count, size_t slice_bytes, uint32_
         for (uint32_t cc = c0 - 1; cc >= 2; cc--) order[norder++] = cc;
     }
     for (int k = 0; k < norder; k++) {
-        // the small-pass chunk first, kChunk when its partials do not fit
-        for (int small = 1; small >= 0; small--) {
-            p = make_plan(ns, count, order[k], fixed, small != 0);
+        // the chunk the pass would like first, larger ones (fewer partial
+        // sums) while they do not fit
+        for (uint32_t ch = 0;; ch = p.chunk + p.chunk / 2 < kChunk ? p.chunk + p.chunk / 2 : kChunk) {
+            p = make_plan(ns, count, order[k], fixed, ch);
             // entry positions are u32 and the masked-sum grid's y is < 2^16
             if (p.max_entries < 0x80000000ull && (uint64_t)count * p.W < 65536 &&
                 slice_bytes_needed(p.W, p.nbits) <= slice_bytes && place(p, regions, region_bytes, nreg))
                 return true;
-            if (p.chunk == kChunk) break;  // the same plan again
+            if (p.chunk >= kChunk) break;
         }
     }
     return false;
@@ -1382,10 +1588,8 @@ hipError_t msm_run(const MsmJob *jobs, uint32_t count, size_t slice_bytes, uint3
     X29S *buckets = (X29S *)p.ptr[A_BUCKETS];
     X29S *phead = (X29S *)p.ptr[A_PHEAD];
     X29S *ptail = (X29S *)p.ptr[A_PTAIL];
-    uint32_t *hb = (uint32_t *)p.ptr[A_HB];
     uint32_t *tb = (uint32_t *)p.ptr[A_TB];
-    X29S *ws1 = (X29S *)p.ptr[A_WS1];
-    X29S *sum1 = (X29S *)p.ptr[A_SUM1];
+    X29S *part = (X29S *)p.ptr[A_PART];
     uint32_t *scan_sums = (uint32_t *)p.ptr[A_SCAN];
     uint32_t *longs = (uint32_t *)p.ptr[A_LONG];
 
@@ -1406,63 +1610,76 @@ hipError_t msm_run(const MsmJob *jobs, uint32_t count, size_t slice_bytes, uint3
                 it.scalars = jb.scalars;
                 it.n = jb.n;
                 it.tile0 = tile;
-                it.ntiles = (jb.n + kSortTile - 1) / kSortTile;
+                it.ntiles = (jb.n + p.tile - 1) / p.tile;
                 it.dig0 = dig;
                 pk.slot[j] = jb.slice;
                 tile += it.ntiles;
                 dig += (uint64_t)jb.n * p.Wd;
             }
-            k_msm_put_items<<<1, kItemsPerLaunch, 0, stream>>>(pk, items, slots, longs);
+            k_msm_put_items<<<1, 256, 0, stream>>>(pk, items, slots, longs, hist,
+                                                   p.window_sort ? (uint32_t)p.nhist : 0u);
             ZK_CHECK(hipGetLastError());
         }
     }
-    k_slice_clear<<<(count + 63) / 64, 64, 0, stream>>>(slots, count);
-    ZK_CHECK(hipGetLastError());
     const uint32_t fx = p.fixed ? 1u : 0u;
-    if (p.fixed) {
-        if ((uint64_t)p.Wd * p.nbins > kHistMaxFixed || p.nbins > kFixedMaxBins || (1u << p.lo_bits) > kFixedMaxKeys)
-            return hipErrorInvalidValue;  // not for kFixedMinC <= c <= kFixedMaxC
-        k_msm_digits_hist<kHistMaxFixed><<<(uint32_t)p.ntiles, kDigitThreads, 0, stream>>>(
-            items, count, c, p.Wd, p.lo_bits, p.nbins, fx, digits, hist);
+    if (p.window_sort) {
+        // digits beside the entries (the array between the two sort levels is free)
+        uint32_t *dig = (uint32_t *)tmp;
+        k_msm_digits<<<dim3((uint32_t)p.ntiles, p.tile / 256, (p.W + kDigitWindows - 1) / kDigitWindows), 256, 0,
+                       stream>>>(items, count, c, p.W, p.tile, digit_offset(c, p.W), dig, hist);
+        ZK_CHECK(hipGetLastError());
+        ZK_CHECK(prof_mark(prof, PH_SCAN, stream));
+        ZK_CHECK(prof_mark(prof, PH_SCATTER, stream));
+        uint32_t nmax = 0;
+        for (uint32_t m = 0; m < count; m++) nmax = ns[m] > nmax ? ns[m] : nmax;
+        k_msm_sort_window<<<count * p.W, kGroupThreads, nmax * 4, stream>>>(items, p.W, p.B, count * p.W, dig, hist,
+                                                                           entries, offsets);
+        ZK_CHECK(hipGetLastError());
     } else {
-        if ((uint64_t)p.W * p.nbins > kHistMax || p.nbins > 256 || p.lo_bits > 8)
-            return hipErrorInvalidValue;  // not for 2 <= c <= 17
-        k_msm_digits_hist<kHistMax><<<(uint32_t)p.ntiles, kDigitThreads, 0, stream>>>(items, count, c, p.Wd, p.lo_bits,
-                                                                                   p.nbins, fx, digits, hist);
+        // the kernels for at most 256 bins and 256 keys, or (fixed-base mode)
+        // 1024 bins and 512 keys
+        const bool wide = p.nbins > 256 || p.lo_bits > 8 || (uint64_t)p.Wd * p.nbins > kHistMax;
+        if (wide && ((uint64_t)p.Wd * p.nbins > kHistMaxFixed || p.nbins > kFixedMaxBins ||
+                     (1u << p.lo_bits) > kFixedMaxKeys))
+            return hipErrorInvalidValue;  // not for 2 <= c <= 17, kFixedMinC <= c <= kFixedMaxC
+        if (wide)
+            k_msm_digits_hist<kHistMaxFixed><<<(uint32_t)p.ntiles, kDigitThreads, 0, stream>>>(
+                items, count, c, p.Wd, p.lo_bits, p.nbins, fx, p.tile, digits, hist);
+        else
+            k_msm_digits_hist<kHistMax><<<(uint32_t)p.ntiles, kDigitThreads, 0, stream>>>(
+                items, count, c, p.Wd, p.lo_bits, p.nbins, fx, p.tile, digits, hist);
+        ZK_CHECK(hipGetLastError());
+        ZK_CHECK(prof_mark(prof, PH_SCAN, stream));
+        ZK_CHECK(launch_scan(hist, (uint32_t)p.nhist, starts, nullptr, scan_sums, stream));
+        ZK_CHECK(prof_mark(prof, PH_SCATTER, stream));
+        const uint32_t ngroups = count * p.W * p.nbins;
+        const dim3 sgrid((uint32_t)p.ntiles, p.Wd);
+        auto sort = [&](auto packed, auto bins, auto keys) -> hipError_t {
+            using T = typename TmpEnt<decltype(packed)::value>::T;
+            k_msm_scatter_hi<decltype(packed)::value, decltype(bins)::value><<<sgrid, 256, 0, stream>>>(
+                items, count, p.Wd, digits, p.lo_bits, p.nbins, fx, p.tile, hist, starts, (T *)tmp);
+            ZK_CHECK(hipGetLastError());
+            k_msm_sort_group<decltype(packed)::value, decltype(keys)::value><<<ngroups, kGroupThreads, 0, stream>>>(
+                items, p.W, p.Wd, p.nbins, fx, (const T *)tmp, starts, p.lo_bits, p.B, ngroups, entries, offsets);
+            return hipGetLastError();
+        };
+        using Narrow = std::integral_constant<uint32_t, 256>;
+        using WideBins = std::integral_constant<uint32_t, kFixedMaxBins>;
+        using WideKeys = std::integral_constant<uint32_t, kFixedMaxKeys>;
+        if (p.packed)
+            ZK_CHECK(wide ? sort(std::true_type{}, WideBins{}, WideKeys{}) : sort(std::true_type{}, Narrow{}, Narrow{}));
+        else
+            ZK_CHECK(wide ? sort(std::false_type{}, WideBins{}, WideKeys{}) : sort(std::false_type{}, Narrow{}, Narrow{}));
     }
-    ZK_CHECK(hipGetLastError());
-    ZK_CHECK(prof_mark(prof, PH_SCAN, stream));
-    ZK_CHECK(launch_scan(hist, (uint32_t)p.nhist, starts, nullptr, scan_sums, stream));
-    ZK_CHECK(prof_mark(prof, PH_SCATTER, stream));
-    const uint32_t ngroups = count * p.W * p.nbins;
-    const dim3 sgrid((uint32_t)p.ntiles, p.Wd);
-    if (p.fixed) {
-        k_msm_scatter_hi<false, kFixedMaxBins><<<sgrid, 256, 0, stream>>>(items, count, p.Wd, digits, p.lo_bits,
-                                                                         p.nbins, fx, hist, starts, (uint2 *)tmp);
-        ZK_CHECK(hipGetLastError());
-        k_msm_sort_group<false, kFixedMaxKeys><<<ngroups, kGroupThreads, 0, stream>>>(
-            items, p.W, p.Wd, p.nbins, fx, (const uint2 *)tmp, starts, p.lo_bits, p.B, ngroups, entries, offsets);
-    } else if (p.packed) {
-        k_msm_scatter_hi<true, 256><<<sgrid, 256, 0, stream>>>(items, count, p.Wd, digits, p.lo_bits, p.nbins, fx,
-                                                               hist, starts, (uint32_t *)tmp);
-        ZK_CHECK(hipGetLastError());
-        k_msm_sort_group<true, 256><<<ngroups, kGroupThreads, 0, stream>>>(
-            items, p.W, p.Wd, p.nbins, fx, (const uint32_t *)tmp, starts, p.lo_bits, p.B, ngroups, entries, offsets);
-    } else {
-        k_msm_scatter_hi<false, 256><<<sgrid, 256, 0, stream>>>(items, count, p.Wd, digits, p.lo_bits, p.nbins, fx,
-                                                                hist, starts, (uint2 *)tmp);
-        ZK_CHECK(hipGetLastError());
-        k_msm_sort_group<false, 256><<<ngroups, kGroupThreads, 0, stream>>>(
-            items, p.W, p.Wd, p.nbins, fx, (const uint2 *)tmp, starts, p.lo_bits, p.B, ngroups, entries, offsets);
-    }
-    ZK_CHECK(hipGetLastError());
     ZK_CHECK(prof_mark(prof, PH_ACCUMULATE, stream));
     const uint32_t cblocks = (uint32_t)((p.chunks + 255) / 256);
     k_msm_accumulate<<<cblocks, 256, 0, stream>>>(entries, offsets, (uint32_t)p.NB, p.W * p.B, items, buckets,
-                                                  phead, ptail, hb, tb, p.chunks, p.chunk);
+                                                  phead, ptail, tb, p.chunks, p.chunk);
     ZK_CHECK(hipGetLastError());
     ZK_CHECK(prof_mark(prof, PH_FIXUP, stream));
-    k_msm_fixup<<<cblocks, 256, 0, stream>>>(buckets, phead, ptail, tb, offsets, longs, p.chunks, p.chunk);
+    const uint64_t fquads = p.NB > p.chunks ? p.NB : p.chunks;
+    k_msm_fixup<<<(uint32_t)((fquads + 63) / 64), 256, 0, stream>>>(buckets, phead, ptail, tb, offsets, (uint32_t)p.NB,
+                                                                   longs, (uint32_t)p.chunks, p.chunk);
     ZK_CHECK(hipGetLastError());
     {
         const uint64_t max_long = p.chunks / kWalk + 1;
@@ -1472,39 +1689,28 @@ hipError_t msm_run(const MsmJob *jobs, uint32_t count, size_t slice_bytes, uint3
     }
     ZK_CHECK(prof_mark(prof, PH_REDUCE, stream));
     const uint32_t gw = count * p.W;
-    const uint32_t nseg = gw * p.T1;
-    if (p.T1 >= 64) {
-        // one wave per 64 segments; its 8 partials go to the ws1 array (gw *
-        // T1 / 8 entries, within its gw * T1)
-        k_msm_reduce_fold<<<nseg / 64, 64, 0, stream>>>(buckets, offsets, p.B, p.T1, ws1);
+    if (p.quads) {
+        const uint32_t hw = (p.B + 15) / 16, nwaves = gw * hw;
+        k_msm_bits<<<(nwaves + 3) / 4, 256, 0, stream>>>(buckets, offsets, p.B, hw, nwaves, part);
         ZK_CHECK(hipGetLastError());
-        k_msm_fold_sums<<<dim3(p.nbits + 1, gw), 64, 0, stream>>>(ws1, p.T1, p.nbits, p.W, slots);
-        ZK_CHECK(hipGetLastError());
-    } else {
-        k_msm_reduce_l1<<<(nseg + 63) / 64, 64, 0, stream>>>(buckets, offsets, gw, p.B, p.T1, ws1, sum1);
-        ZK_CHECK(hipGetLastError());
-        // split each masked sum over `parts` workgroups when there are too
-        // few sums to give every SIMD a wave (the sums are latency-bound
-        // chains of point additions; more parts than that only adds tree
-        // levels); the parts go to the chunk partials' array (dead after the
-        // fixup)
-        const uint64_t sums = (uint64_t)gw * (p.nbits + 1);
-        uint32_t parts = 1;
-        while (sums * parts * 2 <= 1024 && parts * 2 * 256 <= p.T1 && parts < 256 && sums * parts * 2 <= p.chunks)
-            parts *= 2;
-        k_msm_masked_sums<<<dim3(p.nbits + 1, gw, parts), 256, 0, stream>>>(ws1, sum1, p.T1, p.nbits, p.W, slots,
-                                                                          phead);
+        // at most 256 waves' partials per workgroup: a chain of 4 to 8
+        // additions before its tree
+        const uint32_t parts = bit_sum_parts(hw);
+        X29S *qpart = part + (size_t)nwaves * kBitParts;
+        k_msm_bit_sums<<<dim3(p.nbits + 1, gw, parts), hw > 16 ? 256 : 64, 0, stream>>>(part, hw, c, p.W, slots,
+                                                                                     qpart);
         ZK_CHECK(hipGetLastError());
         if (parts > 1) {
-            const uint32_t per = 256 / parts;
-            k_msm_masked_merge<<<(uint32_t)((sums + per - 1) / per), 256, 0, stream>>>(phead, parts, p.nbits, p.W,
-                                                                                      gw, slots);
+            k_msm_bit_merge<<<dim3(p.nbits + 1, gw), 64, 0, stream>>>(qpart, parts, c, p.W, slots);
             ZK_CHECK(hipGetLastError());
         }
+    } else {
+        k_msm_reduce_fold<<<gw * (p.T1 / 64), 64, 0, stream>>>(buckets, offsets, p.B, p.T1, part);
+        ZK_CHECK(hipGetLastError());
+        k_msm_fold_sums<<<dim3(p.nbits + 1, gw), 64, 0, stream>>>(part, p.T1, p.nbits, c, p.W, slots);
+        ZK_CHECK(hipGetLastError());
     }
     ZK_CHECK(prof_mark(prof, PH_HEADER, stream));
-    k_slice_header<<<(count + 63) / 64, 64, 0, stream>>>(slots, count, c, p.W, p.nbits);
-    ZK_CHECK(hipGetLastError());
     ZK_CHECK(prof_mark(prof, PH_NUM, stream));
     if (slots_dev) *slots_dev = slots;
     return prof_finish(prof);
@@ -1523,7 +1729,7 @@ void host_tail_one(const uint8_t *blob, uint8_t *out96, bool split = false) {
     static_assert(sizeof(zkh::Xyzz) == sizeof(G1Xyzz), "host and device XYZZ layouts differ");
     static_assert((kL1 & (kL1 - 1)) == 0, "kL1 is a power of two");
     const zkh::Xyzz *q = reinterpret_cast<const zkh::Xyzz *>(blob + kSliceQ);
-    const uint32_t c = h->c, W = h->W, nb = h->nbits, l1 = (uint32_t)__builtin_ctz(kL1);
+    const uint32_t c = h->c, W = h->W, nb = h->nbits, l1 = h->l1;
     const int top = zkh::msm_tail_top(c, W, nb, l1), lo = top * 11 / 20;
     zkh::Jac res;
     if (!split || lo < 1) {
@@ -1925,7 +2131,7 @@ static hipError_t finish_batch(uint8_t *const *slices, uint8_t **slots_dev, uint
         ZK_CHECK(device_collect(slots_dev, count, stream));
         return check_markers(slices, count, stream);
     }
-    return host_collect(slices, count, stream);
+    return host_collect(slices, count, stream, ZK_MSM_OUT_BYTES);  // the outs' size
 }
 
 // One MSM with caller-owned scratch (no allocation): the result (Jacobian,

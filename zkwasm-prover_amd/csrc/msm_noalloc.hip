@@ -44,7 +44,7 @@ extern "C" {
 hipError_t zk_msm_noalloc(void *out, const void *points, const void *scalars, int n, int c, hipStream_t stream) {
     if (n <= 0 || !out || !points || !scalars || c < 0 || c == 1 || c > 17) return hipErrorInvalidValue;
     // sizes whose scratch exceeds the array are refused, never shrunk to fit
-    if (zk_msm_scratch_bytes(n, c) > (size_t)ZK_MSM_NOALLOC_SCRATCH_BYTES) return hipErrorInvalidValue;
+    if (zk::msm_noalloc_bytes((uint32_t)n, (uint32_t)c) > (size_t)ZK_MSM_NOALLOC_SCRATCH_BYTES) return hipErrorInvalidValue;
     return zk::guard([&]() -> hipError_t {
         void *ptr = nullptr;
         ZK_CHECK(scratch_address(&ptr));

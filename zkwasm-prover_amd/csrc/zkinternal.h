@@ -53,6 +53,7 @@ hipError_t ntt_batch_from(const void *const *src, void *const *buf, void *const 
 // server sets it to merge the MSMs of concurrent proofs. (prover_core.cpp)
 // One MSM through the pipeline with the device tail, enqueued on stream
 // without host waits or host allocation (msm.hip)
+size_t msm_noalloc_bytes(uint32_t n, uint32_t c);
 hipError_t msm_one_async(void *out, const void *points, const void *scalars, uint32_t n, uint32_t c, void *scratch,
                          size_t scratch_bytes, hipStream_t stream);
 
