@@ -375,6 +375,21 @@ __device__ __forceinline__ void f29_unpack(const F29 &a, uint32_t x[8]) {
         x[w] = v;
     }
 }
+// 32 a for a < 2^256 (normalised limbs): an operand in the 2^256 domain moved
+// to the 2^261 domain of a 29-bit product (64 r for a < 2r: times < 2r in bounds)
+__device__ __forceinline__ F29 f29_shl5(const F29 &a) {
+    F29 r;
+    r.l[0] = (a.l[0] << 5) & kM29;
+#pragma unroll
+    for (int i = 1; i < 9; i++) r.l[i] = ((a.l[i] << 5) | (a.l[i - 1] >> 24)) & kM29;
+    return r;
+}
+// a value below 2r in 29-bit limbs -> canonical 32-bit form (same domain)
+__device__ __forceinline__ Fr f29_to_fr(const F29 &a) {
+    Fr r;
+    f29_unpack(a, r.v);
+    return fe_reduce_once<FrParams>(r);
+}
 // a * w in Fr's 32-bit Montgomery form for a < r and w29 = f29_from32(w)
 // (w 2^261 mod r up to 32 r): the 29-bit product a w29 2^-261 is a w 2^256
 // mod r itself, < 2r, so repacking both ways and one conditional

@@ -4,252 +4,175 @@
 // `eval_logup_z_pure` (cuda/bn254.cu:19-220, :1914-1993; caller
 // src/lib.rs:590-745), plus zk_batch_invert.
 //
-// Batch inversion is Montgomery's trick in three launches over tiles of 4096
-// elements (prefix products into the caller's temp, every tile's total
-// inverted by its own thread of a small launch, then two products per
-// element on the way back; details at k_binv_up below).  Above 2^24 elements
-// a multi-level hierarchy takes over: level 0 thread t owns the m elements
-// t, t + T, t + 2T, ... (T = n/m, coalesced) and writes only their product;
-// the T products are inverted recursively the same way, the last <= 512 by
-// one workgroup with a product tree in LDS; on the way down each thread
-// rebuilds its prefix products in registers and emits the inverses.
+// Batch inversion is Montgomery's trick in one launch over tiles of 256 E
+// elements (details at k_binv below); the logup's z[i] = s[i] - m[i] / (t[i] +
+// beta) and its tile sums come out of the same pass.
 // A zero input stays zero and does not disturb the others (halo2
 // BatchInvert semantics); the reference's chunked kernel would zero its chunk
 // instead, a case its callers never produce (beta is random).
 //
 // The logup z scan (exclusive prefix sum with a carried start value) is a
-// three-kernel block scan: block totals, one-block scan of the totals with
-// the carry, then the in-block exclusive scan plus offset.
+// three-kernel block scan: block totals (from k_binv where that wrote z), a
+// one-block scan of the totals with the carry, then the in-block exclusive
+// scan plus offset.
+#include "ff29.h"
+#include "inv_dev.h"
 #include "zkcore.h"
 
 using namespace zk;
 
 namespace {
 
-constexpr int kM = 8;          // elements per thread at each level
-constexpr uint32_t kTop = 512;  // values inverted by the single-workgroup tree
 constexpr uint32_t kScanBlock = 2048;  // elements per scan block (256 threads x 8)
 
-enum ApplyMode { OUT_SET = 0, OUT_ADD = 1 };
+enum BinvMode {
+    OUT_SET = 0,   // out[i] = 1 / x'[i]
+    OUT_ADD = 1,   // out[i] += 1 / x'[i]
+    OUT_LOGUP = 2  // out[i] = s[i] - m[i] / x'[i], and x[tile start] = the tile's sum of out
+};
 
-__device__ __forceinline__ Fr load_plus(const Fr *x, size_t i, const Fr *beta, bool has_beta, const Fr &b) {
-    Fr v = fe_load<FrParams>(&x[i]);
-    return has_beta ? v + b : v;
+// ---- batch inversion ------------------------------------------------------
+// One workgroup per tile of 256 E elements, thread t owning the elements k *
+// 256 + t (k < E), so every access is coalesced.  Each thread forms its prefix
+// products in registers; the 256 thread products go through a product tree in
+// LDS; the first wave inverts the tile's product (inv_wave.h); the tree is
+// walked down, and each thread emits its elements' inverses backwards.  Three
+// products per element and one read (two of x, the second from cache) and one
+// write of each array.
+//
+// Why one launch: with the prefix products through memory and the tiles'
+// products inverted by a launch of their own it moved 5 x 32 B per element and
+// waited 70 us for the inversions with the device idle; here other tiles'
+// products run meanwhile (2^22 elements: 264 -> 191 us; 2^18: 160 -> 50).
+// The products are the 29-bit ones (ff29.h): running products stay in the
+// 256-bit Montgomery domain below 2r, and one operand of each product is
+// shifted into the 2^261 domain (f29_from32 of an element, f29_shl5 of a
+// product).  Four waves per SIMD (128 registers, nine per prefix) measured
+// best: 2^22 elements 225 us with three, 191 with four, 208 with five.
+constexpr uint32_t kBT = 256;
+
+struct BinvNode {
+    uint32_t l[9];  // stride of nine words: no bank conflicts
+};
+__device__ __forceinline__ F29 node_load(const BinvNode &n) {
+    F29 r;
+#pragma unroll
+    for (int i = 0; i < 9; i++) r.l[i] = n.l[i];
+    return r;
+}
+__device__ __forceinline__ void node_store(BinvNode &n, const F29 &v) {
+#pragma unroll
+    for (int i = 0; i < 9; i++) n.l[i] = v.l[i];
 }
 
-// fe_inv with the binary GCD inlined, so that its limb arrays stay in
-// registers (fe_inv's out-of-line call keeps them in scratch memory); the
-// exact one-bit extended Euclid should the product check fail, as fe_inv.
-// 0 -> 0.
-__device__ __forceinline__ Fr fr_inv_inline(const Fr &a) {
-    if (fe_is_zero<FrParams>(a)) return fe_zero<FrParams>();
-    uint32_t v[8];
-    const bool ok = zkinv::bingcd(v, a.v, FrParams::M, FrParams::INV);
-    const Fr r = fe_from_raw<FrParams>(v) * fe_from_raw<FrParams>(FrParams::INVC);
-    if (ok && fe_eq<FrParams>(a * r, fe_one<FrParams>())) return r;
-    return fe_inv_raw<FrParams>(a) * fe_from_raw<FrParams>(FrParams::R3);
-}
-
-// tot[t] = prod_k x'[t + k*T] (zeros skipped)
-__global__ __launch_bounds__(256) void k_binv_totals(const Fr *__restrict__ x, const Fr *__restrict__ beta, Fr *__restrict__ tot,
-                              uint32_t n, uint32_t T) {
-    uint32_t t = blockIdx.x * blockDim.x + threadIdx.x;
-    if (t >= T) return;
+template <int MODE, int E>
+__global__ __launch_bounds__(kBT, 4) void k_binv(Fr *x, const Fr *__restrict__ beta, Fr *out, uint32_t n, const Fr *s,
+                                                 const Fr *__restrict__ m) {
+    __shared__ BinvNode tree[2 * kBT];
+    __shared__ Fr part[kBT / 64];
+    const uint32_t t = threadIdx.x;
+    const uint64_t base = (uint64_t)blockIdx.x * (kBT * E) + t;
     const bool hb = beta != nullptr;
-    Fr b = hb ? fe_load<FrParams>(beta) : fe_zero<FrParams>();
-    Fr acc = fe_one<FrParams>();
-    for (uint32_t i = t; i < n; i += T) {
-        Fr v = load_plus(x, i, beta, hb, b);
-        if (!fe_is_zero<FrParams>(v)) acc = acc * v;
-    }
-    fe_store<FrParams>(&tot[t], acc);
-}
-
-// inverse of each element from the inverse of its thread's product
-template <int MODE>
-__global__ __launch_bounds__(256) void k_binv_apply(const Fr *__restrict__ x, const Fr *__restrict__ beta,
-                             const Fr *__restrict__ inv_tot, Fr *out, uint32_t n, uint32_t T) {
-    uint32_t t = blockIdx.x * blockDim.x + threadIdx.x;
-    if (t >= T) return;
-    const bool hb = beta != nullptr;
-    Fr b = hb ? fe_load<FrParams>(beta) : fe_zero<FrParams>();
-    Fr v[kM], pre[kM];
-    Fr acc = fe_one<FrParams>();
-#pragma unroll 8
-    for (int k = 0; k < kM; k++) {
-        uint32_t i = t + (uint32_t)k * T;
-        v[k] = i < n ? load_plus(x, i, beta, hb, b) : fe_zero<FrParams>();
+    const Fr b = hb ? fe_load<FrParams>(beta) : fe_zero<FrParams>();
+    F29 pre[E], acc = f29_repack(FrParams::ONE);
+    uint32_t live = 0;  // bit k: element k exists and is not zero
+#pragma clang loop unroll(full)
+    for (int k = 0; k < E; k++) {
+        const uint64_t i = base + (uint32_t)k * kBT;
         pre[k] = acc;
-        if (!fe_is_zero<FrParams>(v[k])) acc = acc * v[k];
-    }
-    Fr inv = fe_load<FrParams>(&inv_tot[t]);
-#pragma unroll 8
-    for (int k = kM - 1; k >= 0; k--) {
-        uint32_t i = t + (uint32_t)k * T;
-        Fr r;
-        if (fe_is_zero<FrParams>(v[k])) {
-            r = fe_zero<FrParams>();
-        } else {
-            r = inv * pre[k];
-            inv = inv * v[k];
-        }
         if (i < n) {
+            Fr v = fe_load<FrParams>(&x[i]);
+            if (hb) v = v + b;
+            if (!fe_is_zero<FrParams>(v)) {
+                live |= 1u << k;
+                acc = f29_mul<Fr29Mod>(acc, f29_from32(v));
+            }
+        }
+    }
+    node_store(tree[kBT + t], acc);
+    __syncthreads();
+    for (uint32_t w = kBT / 2; w >= 1; w >>= 1) {
+        if (t < w) {
+            const uint32_t p = w + t;
+            node_store(tree[p], f29_mul<Fr29Mod>(node_load(tree[2 * p]), f29_shl5(node_load(tree[2 * p + 1]))));
+        }
+        __syncthreads();
+    }
+    if (t < 64) {
+        const Fr inv = fr_inv_wave(f29_to_fr(node_load(tree[1])));
+        if (t == 0) node_store(tree[1], f29_repack(inv.v));
+    }
+    __syncthreads();
+    for (uint32_t w = 1; w < kBT; w <<= 1) {
+        if (t < w) {
+            const uint32_t p = w + t;
+            const F29 ip = f29_shl5(node_load(tree[p]));
+            const F29 l = node_load(tree[2 * p]), r = node_load(tree[2 * p + 1]);
+            node_store(tree[2 * p], f29_mul<Fr29Mod>(ip, r));
+            node_store(tree[2 * p + 1], f29_mul<Fr29Mod>(ip, l));
+        }
+        __syncthreads();
+    }
+    acc = node_load(tree[kBT + t]);
+    Fr sum = fe_zero<FrParams>();
+    // fully unrolled: the prefixes stay in registers
+#pragma clang loop unroll(full)
+    for (int k = E - 1; k >= 0; k--) {
+        const uint64_t i = base + (uint32_t)k * kBT;
+        if (i < n) {
+            Fr r = fe_zero<FrParams>();
+            if ((live >> k) & 1u) {
+                r = f29_to_fr(k ? f29_mul<Fr29Mod>(f29_shl5(acc), pre[k]) : acc);
+                if (k) {
+                    Fr v = fe_load<FrParams>(&x[i]);
+                    if (hb) v = v + b;
+                    acc = f29_mul<Fr29Mod>(acc, f29_from32(v));
+                }
+            }
             if (MODE == OUT_ADD) r = fe_load<FrParams>(&out[i]) + r;
+            if (MODE == OUT_LOGUP) {
+                r = fe_load<FrParams>(&s[i]) - fr_mul_w29(fe_load<FrParams>(&m[i]), f29_from32(r));
+                sum = sum + r;
+            }
             fe_store<FrParams>(&out[i], r);
         }
     }
+    if (MODE == OUT_LOGUP) {
+        // the tile's sum into x's slot of its first element, which only this
+        // workgroup has read
+#pragma unroll
+        for (int d = 32; d; d >>= 1) {
+            Fr o;
+#pragma unroll
+            for (int i = 0; i < 8; i++) o.v[i] = (uint32_t)__shfl_xor((int)sum.v[i], d);
+            sum = sum + o;
+        }
+        if ((t & 63) == 0) part[t >> 6] = sum;
+        __syncthreads();  // also: every read of x in this tile is done
+        if (t == 0) {
+            for (uint32_t w = 1; w < kBT / 64; w++) sum = sum + part[w];
+            fe_store<FrParams>(&x[base], sum);
+        }
+    }
 }
 
-// one workgroup: inverses of x'[i] = x[i] (+ beta) for i < N <= kTop (zeros stay
-// zero), stored (MODE OUT_SET) or added (OUT_ADD) to out
+// Elements per thread.  A tile costs a tree (about 27 wave products) and an
+// inversion's latency whatever its size, which eight elements per thread
+// amortise; small inputs take fewer so that more workgroups share the products
+// (2 / 4 / 8 per thread: 2^16 elements 44 / 49 / 60 us, 2^18 50 / 50 / 60, 2^20
+// 107 / 73 / 77, 2^22 370 / 257 / 191).
+int binv_elems(uint32_t n) { return n <= (1u << 17) ? 2 : n <= (1u << 20) ? 4 : 8; }
 template <int MODE>
-__global__ __launch_bounds__(256) void k_binv_top(const Fr *__restrict__ x, const Fr *__restrict__ beta, Fr *out,
-                                                  uint32_t N) {
-    __shared__ Fr tree[2 * kTop];
-    __shared__ uint32_t zero[kTop];
-    const uint32_t P = kTop;  // leaves at [P, 2P)
-    const bool hb = beta != nullptr;
-    Fr b = hb ? fe_load<FrParams>(beta) : fe_zero<FrParams>();
-    for (uint32_t i = threadIdx.x; i < P; i += blockDim.x) {
-        Fr v = i < N ? load_plus(x, i, beta, hb, b) : fe_one<FrParams>();
-        bool z = fe_is_zero<FrParams>(v);
-        zero[i] = z;
-        tree[P + i] = z ? fe_one<FrParams>() : v;
-    }
-    __syncthreads();
-    for (uint32_t w = P / 2; w >= 1; w >>= 1) {
-        for (uint32_t i = threadIdx.x; i < w; i += blockDim.x) tree[w + i] = tree[2 * (w + i)] * tree[2 * (w + i) + 1];
-        __syncthreads();
-    }
-    if (threadIdx.x == 0) tree[1] = fr_inv_inline(tree[1]);
-    __syncthreads();
-    for (uint32_t w = 1; w < P; w <<= 1) {
-        for (uint32_t i = threadIdx.x; i < w; i += blockDim.x) {
-            uint32_t p = w + i;
-            Fr ip = tree[p];
-            Fr l = tree[2 * p], r = tree[2 * p + 1];
-            tree[2 * p] = ip * r;
-            tree[2 * p + 1] = ip * l;
-        }
-        __syncthreads();
-    }
-    for (uint32_t i = threadIdx.x; i < N; i += blockDim.x) {
-        Fr r = zero[i] ? fe_zero<FrParams>() : tree[P + i];
-        if (MODE == OUT_ADD) r = fe_load<FrParams>(&out[i]) + r;
-        fe_store<FrParams>(&out[i], r);
-    }
-}
-
-// ---- batch inversion in three launches (n <= 2^24) ------------------------
-// Tile b = 4096 elements, 256 threads x 16; thread t owns the elements
-// b * 4096 + k * 256 + t (k < 16), so every load and store is coalesced.
-//   up:   each thread's exclusive prefix products go to pre[] (the slot of its
-//         first element is not needed: that prefix is 1), the 256 thread
-//         products into an LDS product tree; the tile's total goes into the
-//         free slot pre[b * 4096].
-//   tiles: one thread per tile inverts its total in place (T independent
-//         binary-GCD inversions side by side, no product tree over tiles).
-//   down: each tile rebuilds its thread products (pre of the last element
-//         times that element), the tree, walks it down from the tile's
-//         inverse, and each thread emits its elements' inverses backwards
-//         (two products per element).
-// Three Montgomery products per element in all; traffic 5 x 32 B per element
-// (x twice, pre written and read, out written).
-constexpr uint32_t kBT = 256;
-constexpr int kBM = 16;
-constexpr uint32_t kTile = kBT * kBM;
-constexpr uint32_t kTopMax = kBT * kBM;  // tiles up to which the tiled path runs (n <= 2^24)
-
-// LDS product tree over kBT leaves at [kBT, 2 kBT): tree[1] = their product
-__device__ __forceinline__ void tree_up(Fr *tree) {
-    for (uint32_t w = kBT / 2; w >= 1; w >>= 1) {
-        if (threadIdx.x < w) {
-            const uint32_t p = w + threadIdx.x;
-            tree[p] = tree[2 * p] * tree[2 * p + 1];
-        }
-        __syncthreads();
-    }
-}
-// from tree[1] = the inverse of the product: each leaf becomes its inverse
-__device__ __forceinline__ void tree_down(Fr *tree) {
-    for (uint32_t w = 1; w < kBT; w <<= 1) {
-        if (threadIdx.x < w) {
-            const uint32_t p = w + threadIdx.x;
-            const Fr ip = tree[p], l = tree[2 * p], r = tree[2 * p + 1];
-            tree[2 * p] = ip * r;
-            tree[2 * p + 1] = ip * l;
-        }
-        __syncthreads();
-    }
-}
-
-__global__ __launch_bounds__(kBT) void k_binv_up(const Fr *__restrict__ x, const Fr *__restrict__ beta,
-                                                 Fr *__restrict__ pre, uint32_t n) {
-    __shared__ Fr tree[2 * kBT];
-    const uint32_t t = threadIdx.x, base = blockIdx.x * kTile;
-    const bool hb = beta != nullptr;
-    const Fr b = hb ? fe_load<FrParams>(beta) : fe_zero<FrParams>();
-    Fr acc = fe_one<FrParams>();
-#pragma unroll 4
-    for (int k = 0; k < kBM; k++) {
-        const uint32_t i = base + (uint32_t)k * kBT + t;
-        if (i >= n) break;
-        const Fr v = load_plus(x, i, beta, hb, b);
-        if (k) fe_store<FrParams>(&pre[i], acc);
-        if (!fe_is_zero<FrParams>(v)) acc = acc * v;
-    }
-    tree[kBT + t] = acc;
-    __syncthreads();
-    tree_up(tree);
-    if (t == 0) fe_store<FrParams>(&pre[base], tree[1]);
-}
-
-// the T tile totals at pre[b * kTile] -> their inverses, in place: one
-// independent inversion per thread (a separate launch keeps the inversion's
-// registers out of the streaming kernels)
-__global__ __launch_bounds__(64) void k_binv_tiles(Fr *pre, uint32_t T) {
-    const uint32_t b = blockIdx.x * blockDim.x + threadIdx.x;
-    if (b >= T) return;
-    Fr *p = &pre[(size_t)b * kTile];
-    fe_store<FrParams>(p, fr_inv_inline(fe_load<FrParams>(p)));
-}
-
-template <int MODE>
-__global__ __launch_bounds__(kBT) void k_binv_down(const Fr *x, const Fr *__restrict__ beta,
-                                                   const Fr *__restrict__ pre, Fr *out, uint32_t n) {
-    __shared__ Fr tree[2 * kBT];
-    const uint32_t t = threadIdx.x, base = blockIdx.x * kTile;
-    const bool hb = beta != nullptr;
-    const Fr b = hb ? fe_load<FrParams>(beta) : fe_zero<FrParams>();
-    // this thread's elements: k < kl
-    int kl = 0;
-    while (kl < kBM && base + (uint32_t)kl * kBT + t < n) kl++;
-    Fr prod = fe_one<FrParams>();
-    if (kl) {
-        const uint32_t i = base + (uint32_t)(kl - 1) * kBT + t;
-        const Fr v = load_plus(x, i, beta, hb, b);
-        if (kl > 1) prod = fe_load<FrParams>(&pre[i]);
-        if (!fe_is_zero<FrParams>(v)) prod = prod * v;
-    }
-    tree[kBT + t] = prod;
-    __syncthreads();
-    const Fr inv_tile = fe_load<FrParams>(&pre[base]);
-    tree_up(tree);
-    if (t == 0) tree[1] = inv_tile;
-    __syncthreads();
-    tree_down(tree);
-    Fr acc = tree[kBT + t];
-    for (int k = kl - 1; k >= 0; k--) {
-        const uint32_t i = base + (uint32_t)k * kBT + t;
-        const Fr v = load_plus(x, i, beta, hb, b);
-        Fr r = fe_zero<FrParams>();
-        if (!fe_is_zero<FrParams>(v)) {
-            r = k ? acc * fe_load<FrParams>(&pre[i]) : acc;
-            acc = acc * v;
-        }
-        if (MODE == OUT_ADD) r = fe_load<FrParams>(&out[i]) + r;
-        fe_store<FrParams>(&out[i], r);
-    }
+hipError_t binv_launch(Fr *x, const Fr *beta, Fr *out, uint32_t n, const Fr *s, const Fr *m, hipStream_t stream) {
+    const int e = binv_elems(n);
+    const uint32_t tiles = (uint32_t)(((uint64_t)n + (uint64_t)kBT * e - 1) / ((uint64_t)kBT * e));
+    if (e == 2)
+        k_binv<MODE, 2><<<tiles, kBT, 0, stream>>>(x, beta, out, n, s, m);
+    else if (e == 4)
+        k_binv<MODE, 4><<<tiles, kBT, 0, stream>>>(x, beta, out, n, s, m);
+    else
+        k_binv<MODE, 8><<<tiles, kBT, 0, stream>>>(x, beta, out, n, s, m);
+    return hipGetLastError();
 }
 
 __global__ void k_logup_step2(Fr *__restrict__ z, const Fr *__restrict__ s, const Fr *__restrict__ tinv,
@@ -260,103 +183,97 @@ __global__ void k_logup_step2(Fr *__restrict__ z, const Fr *__restrict__ s, cons
         fe_store<FrParams>(&z[i], fe_load<FrParams>(&s[i]) - fe_load<FrParams>(&m[i]) * fe_load<FrParams>(&tinv[i]));
 }
 
-// ---- field prefix scans (add or mul) --------------------------------------
-template <bool MUL>
-__device__ __forceinline__ Fr op_combine(const Fr &a, const Fr &b) {
-    return MUL ? a * b : a + b;
-}
-template <bool MUL>
-__device__ __forceinline__ Fr op_identity() {
-    return MUL ? fe_one<FrParams>() : fe_zero<FrParams>();
-}
-
+// ---- additive prefix scan ---------------------------------------------------
 // block totals: 256 threads x 8 contiguous elements
-template <bool MUL>
 __global__ __launch_bounds__(256) void k_fscan_totals(const Fr *__restrict__ z, uint32_t n, Fr *__restrict__ tot) {
     __shared__ Fr sh[256];
     uint32_t base = blockIdx.x * kScanBlock + threadIdx.x * 8;
-    Fr acc = op_identity<MUL>();
+    Fr acc = fe_zero<FrParams>();
     for (uint32_t k = 0; k < 8; k++)
-        if (base + k < n) acc = op_combine<MUL>(acc, fe_load<FrParams>(&z[base + k]));
+        if (base + k < n) acc = acc + fe_load<FrParams>(&z[base + k]);
     sh[threadIdx.x] = acc;
     __syncthreads();
     for (uint32_t s = 128; s; s >>= 1) {
-        if (threadIdx.x < s) sh[threadIdx.x] = op_combine<MUL>(sh[threadIdx.x], sh[threadIdx.x + s]);
+        if (threadIdx.x < s) sh[threadIdx.x] = sh[threadIdx.x] + sh[threadIdx.x + s];
         __syncthreads();
     }
     if (threadIdx.x == 0) fe_store<FrParams>(&tot[blockIdx.x], sh[0]);
 }
 
-// one block: exclusive scan of nb totals in place, starting from *carry
-// (identity when carry == null)
-template <bool MUL>
-__global__ __launch_bounds__(256) void k_fscan_top(Fr *tot, uint32_t nb, const Fr *__restrict__ carry) {
-    __shared__ Fr sh[256];
-    __shared__ Fr run;
-    if (threadIdx.x == 0) run = carry ? fe_load<FrParams>(carry) : op_identity<MUL>();
+// exclusive scan over a workgroup of 256 threads: shuffles inside each wave,
+// the wave totals through LDS.  Returns the sum of the earlier threads'
+// values; total (every thread): the workgroup's.
+__device__ __forceinline__ Fr block_scan_add(const Fr &v, Fr *sh, Fr &total) {
+    const uint32_t lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+    Fr inc = v;
+#pragma unroll
+    for (int d = 1; d < 64; d <<= 1) {
+        Fr o;
+#pragma unroll
+        for (int i = 0; i < 8; i++) o.v[i] = (uint32_t)__shfl_up((int)inc.v[i], d, 64);
+        if (lane >= (uint32_t)d) inc = inc + o;
+    }
+    if (lane == 63) sh[wv] = inc;
     __syncthreads();
-    // each round covers 256 * 8 totals: thread-local serial part + LDS scan
+    Fr off = fe_zero<FrParams>();
+    total = fe_zero<FrParams>();
+    for (uint32_t w = 0; w < 4; w++) {
+        if (w < wv) off = off + sh[w];
+        total = total + sh[w];
+    }
+    __syncthreads();
+    return off + (inc - v);
+}
+
+// one block: exclusive scan of the nb totals at tot[b * stride] in place,
+// starting from *carry (zero when carry == null)
+__global__ __launch_bounds__(256) void k_fscan_top(Fr *tot, uint32_t nb, size_t stride, const Fr *__restrict__ carry) {
+    __shared__ Fr sh[4];
+    Fr run = carry ? fe_load<FrParams>(carry) : fe_zero<FrParams>();
+    // each round covers 256 * 8 totals: thread-local serial part + block scan
     for (uint32_t base = 0; base < nb; base += 256 * 8) {
         uint32_t b0 = base + threadIdx.x * 8;
         Fr loc[8];
-        Fr acc = op_identity<MUL>();
-#pragma unroll 8
+        Fr acc = fe_zero<FrParams>(), total;
+#pragma unroll
         for (uint32_t k = 0; k < 8; k++) {
-            loc[k] = b0 + k < nb ? fe_load<FrParams>(&tot[b0 + k]) : op_identity<MUL>();
-            acc = op_combine<MUL>(acc, loc[k]);
+            loc[k] = b0 + k < nb ? fe_load<FrParams>(&tot[(b0 + k) * stride]) : fe_zero<FrParams>();
+            acc = acc + loc[k];
         }
-        sh[threadIdx.x] = acc;
-        __syncthreads();
-        // Hillis-Steele inclusive scan of the 256 thread totals
-        for (uint32_t off = 1; off < 256; off <<= 1) {
-            Fr x = threadIdx.x >= off ? sh[threadIdx.x - off] : op_identity<MUL>();
-            __syncthreads();
-            sh[threadIdx.x] = op_combine<MUL>(sh[threadIdx.x], x);
-            __syncthreads();
-        }
-        Fr pre = op_combine<MUL>(run, threadIdx.x ? sh[threadIdx.x - 1] : op_identity<MUL>());
-#pragma unroll 8
+        Fr pre = run + block_scan_add(acc, sh, total);
+#pragma unroll
         for (uint32_t k = 0; k < 8; k++) {
-            if (b0 + k < nb) fe_store<FrParams>(&tot[b0 + k], pre);
-            pre = op_combine<MUL>(pre, loc[k]);
+            if (b0 + k < nb) fe_store<FrParams>(&tot[(b0 + k) * stride], pre);
+            pre = pre + loc[k];
         }
-        __syncthreads();
-        if (threadIdx.x == 255) run = op_combine<MUL>(run, sh[255]);
-        __syncthreads();
+        run = run + total;
     }
 }
 
-// z[i] = offset_block + exclusive in-block prefix; last_z gets z[last_index]
-template <bool MUL>
-__global__ __launch_bounds__(256) void k_fscan_apply(Fr *z, uint32_t n, const Fr *__restrict__ tot,
+// z[i] = offset of the block + exclusive in-block prefix; last_z gets
+// z[last_index].  Blocks of 256 E elements, thread t owning E consecutive
+// ones; block b's offset is at tot[b * stride].
+template <int E>
+__global__ __launch_bounds__(256) void k_fscan_apply(Fr *z, uint32_t n, const Fr *__restrict__ tot, size_t stride,
                                                      Fr *last_z, int64_t last_index) {
-    __shared__ Fr sh[256];
-    uint32_t base = blockIdx.x * kScanBlock + threadIdx.x * 8;
-    Fr loc[8];
-    Fr acc = op_identity<MUL>();
-#pragma unroll 8
-    for (uint32_t k = 0; k < 8; k++) {
-        loc[k] = base + k < n ? fe_load<FrParams>(&z[base + k]) : op_identity<MUL>();
-        acc = op_combine<MUL>(acc, loc[k]);
+    __shared__ Fr sh[4];
+    const uint64_t base = (uint64_t)blockIdx.x * (256 * E) + threadIdx.x * E;
+    Fr loc[E];
+    Fr acc = fe_zero<FrParams>(), total;
+#pragma unroll
+    for (uint32_t k = 0; k < E; k++) {
+        loc[k] = base + k < n ? fe_load<FrParams>(&z[base + k]) : fe_zero<FrParams>();
+        acc = acc + loc[k];
     }
-    sh[threadIdx.x] = acc;
-    __syncthreads();
-    for (uint32_t off = 1; off < 256; off <<= 1) {
-        Fr x = threadIdx.x >= off ? sh[threadIdx.x - off] : op_identity<MUL>();
-        __syncthreads();
-        sh[threadIdx.x] = op_combine<MUL>(sh[threadIdx.x], x);
-        __syncthreads();
-    }
-    Fr pre = op_combine<MUL>(fe_load<FrParams>(&tot[blockIdx.x]),
-                             threadIdx.x ? sh[threadIdx.x - 1] : op_identity<MUL>());
-#pragma unroll 8
-    for (uint32_t k = 0; k < 8; k++) {
-        uint32_t i = base + k;
+    Fr pre = fe_load<FrParams>(&tot[blockIdx.x * stride]) + block_scan_add(acc, sh, total);
+#pragma unroll
+    for (uint32_t k = 0; k < E; k++) {
+        const uint64_t i = base + k;
         if (i < n) {
             fe_store<FrParams>(&z[i], pre);
             if (last_z && (int64_t)i == last_index) fe_store<FrParams>(last_z, pre);
         }
-        pre = op_combine<MUL>(pre, loc[k]);
+        pre = pre + loc[k];
     }
 }
 
@@ -364,107 +281,27 @@ __global__ __launch_bounds__(256) void k_fscan_apply(Fr *z, uint32_t n, const Fr
 
 namespace zk {
 
-// scratch Fr needed by batch_invert_ex for n elements: n (the prefix
-// products) up to 2^24 elements, beyond that the multi-level hierarchy's
-size_t binv_scratch_elems(uint32_t n) {
-    if (n <= (size_t)kTopMax * kTile) return n;
-    size_t s = 0;
-    uint32_t cnt = n;
-    while (cnt > kTop) {
-        uint32_t T = (cnt + kM - 1) / kM;
-        s += 2 * (size_t)T;
-        cnt = T;
-    }
-    return s;
-}
-
 // out[i] = 1/(x[i] (+ beta)) (mode OUT_SET) or out[i] += that (OUT_ADD).
-// out may alias x.  temp must hold binv_scratch_elems(n) Fr.
-hipError_t batch_invert_ex(const Fr *x, const Fr *beta, Fr *out, int mode, uint32_t n, Fr *temp,
-                           hipStream_t stream) {
+// out may alias x.
+hipError_t batch_invert_ex(const Fr *x, const Fr *beta, Fr *out, int mode, uint32_t n, hipStream_t stream) {
     if (n == 0) return hipSuccess;
-    if (n <= (size_t)kTopMax * kTile) {
-        const uint32_t T = (n + kTile - 1) / kTile;
-        k_binv_up<<<T, kBT, 0, stream>>>(x, beta, temp, n);
-        ZK_CHECK(hipGetLastError());
-        k_binv_tiles<<<(T + 63) / 64, 64, 0, stream>>>(temp, T);
-        ZK_CHECK(hipGetLastError());
-        if (mode == OUT_ADD)
-            k_binv_down<OUT_ADD><<<T, kBT, 0, stream>>>(x, beta, temp, out, n);
-        else
-            k_binv_down<OUT_SET><<<T, kBT, 0, stream>>>(x, beta, temp, out, n);
-        return hipGetLastError();
-    }
-    if (n <= kTop) {
-        if (mode == OUT_ADD)
-            k_binv_top<OUT_ADD><<<1, 256, 0, stream>>>(x, beta, out, n);
-        else
-            k_binv_top<OUT_SET><<<1, 256, 0, stream>>>(x, beta, out, n);
-        return hipGetLastError();
-    }
-    const Fr *vals[16];
-    const Fr *betas[16];
-    Fr *tots[16], *invs[16];
-    uint32_t cnts[16], Ts[16];
-    int levels = 0;
-    const Fr *cur = x;
-    const Fr *cur_beta = beta;
-    uint32_t cnt = n;
-    Fr *tp = temp;
-    while (cnt > kTop && levels < 15) {
-        uint32_t T = (cnt + kM - 1) / kM;
-        vals[levels] = cur;
-        betas[levels] = cur_beta;
-        cnts[levels] = cnt;
-        Ts[levels] = T;
-        tots[levels] = tp;
-        invs[levels] = tp + T;
-        tp += 2 * (size_t)T;
-        k_binv_totals<<<(T + 255) / 256, 256, 0, stream>>>(cur, cur_beta, tots[levels], cnt, T);
-        ZK_CHECK(hipGetLastError());
-        cur = tots[levels];
-        cur_beta = nullptr;
-        cnt = T;
-        levels++;
-    }
-    if (cnt > kTop) return hipErrorInvalidValue;
-    k_binv_top<OUT_SET><<<1, 256, 0, stream>>>(tots[levels - 1], nullptr, invs[levels - 1], cnt);
-    ZK_CHECK(hipGetLastError());
-    for (int L = levels - 1; L >= 0; L--) {
-        uint32_t T = Ts[L];
-        uint32_t blocks = (T + 255) / 256;
-        if (L > 0)
-            k_binv_apply<OUT_SET><<<blocks, 256, 0, stream>>>(vals[L], nullptr, invs[L], invs[L - 1], cnts[L], T);
-        else if (mode == OUT_ADD)
-            k_binv_apply<OUT_ADD><<<blocks, 256, 0, stream>>>(vals[0], betas[0], invs[0], out, cnts[0], T);
-        else
-            k_binv_apply<OUT_SET><<<blocks, 256, 0, stream>>>(vals[0], betas[0], invs[0], out, cnts[0], T);
-        ZK_CHECK(hipGetLastError());
-    }
-    return hipSuccess;
+    Fr *xx = const_cast<Fr *>(x);  // written in OUT_LOGUP only
+    return mode == OUT_ADD ? binv_launch<OUT_ADD>(xx, beta, out, n, nullptr, nullptr, stream)
+                           : binv_launch<OUT_SET>(xx, beta, out, n, nullptr, nullptr, stream);
 }
 
-size_t fscan_scratch_elems(uint32_t n) { return (n + kScanBlock - 1) / kScanBlock + 1; }
-
-// exclusive scan in place; carry (device) = start value or null for the
-// identity; last_z (device, may be null) receives z[last_index].
-hipError_t field_scan(Fr *z, uint32_t n, bool mul, const Fr *carry, Fr *last_z, int64_t last_index, Fr *tot,
-                      hipStream_t stream) {
+// exclusive sum scan in place; carry (device) = start value or null for
+// zero; last_z (device, may be null) receives z[last_index].  tot: one Fr per
+// kScanBlock elements.
+static hipError_t field_scan(Fr *z, uint32_t n, const Fr *carry, Fr *last_z, int64_t last_index, Fr *tot,
+                             hipStream_t stream) {
     if (n == 0) return hipSuccess;
     uint32_t nb = (n + kScanBlock - 1) / kScanBlock;
-    if (mul) {
-        k_fscan_totals<true><<<nb, 256, 0, stream>>>(z, n, tot);
-        ZK_CHECK(hipGetLastError());
-        k_fscan_top<true><<<1, 256, 0, stream>>>(tot, nb, carry);
-        ZK_CHECK(hipGetLastError());
-        k_fscan_apply<true><<<nb, 256, 0, stream>>>(z, n, tot, last_z, last_index);
-    } else {
-        k_fscan_totals<false><<<nb, 256, 0, stream>>>(z, n, tot);
-        ZK_CHECK(hipGetLastError());
-        k_fscan_top<false><<<1, 256, 0, stream>>>(tot, nb, carry);
-        ZK_CHECK(hipGetLastError());
-        k_fscan_apply<false><<<nb, 256, 0, stream>>>(z, n, tot, last_z, last_index);
-    }
+    k_fscan_totals<<<nb, 256, 0, stream>>>(z, n, tot);
+    ZK_CHECK(hipGetLastError());
+    k_fscan_top<<<1, 256, 0, stream>>>(tot, nb, 1, carry);
+    ZK_CHECK(hipGetLastError());
+    k_fscan_apply<8><<<nb, 256, 0, stream>>>(z, n, tot, 1, last_z, last_index);
     return hipGetLastError();
 }
 
@@ -475,7 +312,7 @@ namespace zk {
 // out = (x + beta)^-1 element-wise (zeros stay zero); temp: n Fr
 hipError_t batch_invert_shifted(void *out, const void *x, const void *beta, void *temp, int n, hipStream_t stream) {
     if (n <= 0 || !out || !x || !beta || !temp) return hipErrorInvalidValue;
-    return batch_invert_ex((const Fr *)x, (const Fr *)beta, (Fr *)out, OUT_SET, (uint32_t)n, (Fr *)temp, stream);
+    return batch_invert_ex((const Fr *)x, (const Fr *)beta, (Fr *)out, OUT_SET, (uint32_t)n, stream);
 }
 
 // eval_logup_z_compose after its table inversion: z from the logup sum
@@ -490,7 +327,7 @@ hipError_t logup_z_inverted(void *z, void *input, const void *table_inv, const v
     k_logup_step2<<<blocks, 256, 0, stream>>>((Fr *)z, (const Fr *)input, (const Fr *)table_inv,
                                                (const Fr *)multiplicity, (uint32_t)n);
     ZK_CHECK(hipGetLastError());
-    return field_scan((Fr *)z, (uint32_t)n, false, (const Fr *)last_z, (Fr *)last_z, last_z_index, (Fr *)input,
+    return field_scan((Fr *)z, (uint32_t)n, (const Fr *)last_z, (Fr *)last_z, last_z_index, (Fr *)input,
                       stream);
 }
 
@@ -498,19 +335,19 @@ hipError_t logup_z_inverted(void *z, void *input, const void *table_inv, const v
 
 extern "C" {
 
-// In-place batch inversion; temp holds n Fr.
+// In-place batch inversion; temp (n Fr) is not needed by this implementation.
 hipError_t zk_batch_invert(void *a, void *temp, int n, hipStream_t stream) {
-    if (n < 0 || (n > 0 && !a) || (binv_scratch_elems((uint32_t)n) && !temp)) return hipErrorInvalidValue;
-    return batch_invert_ex((const Fr *)a, nullptr, (Fr *)a, OUT_SET, (uint32_t)n, (Fr *)temp, stream);
+    if (n < 0 || (n > 0 && (!a || !temp))) return hipErrorInvalidValue;
+    return batch_invert_ex((const Fr *)a, nullptr, (Fr *)a, OUT_SET, (uint32_t)n, stream);
 }
 
 // cuda/bn254.cu:1914-1934: sum[i] (=, or += when init != 0) 1/(input[i] + beta).
-// temp holds n Fr.
+// temp (n Fr) is not needed by this implementation.
 hipError_t logup_sum_input_inv(void *sum, const void *input, void *temp, const void *beta, int init, int n,
                                hipStream_t stream) {
-    if (n <= 0 || !sum || !input || !beta || (binv_scratch_elems((uint32_t)n) && !temp)) return hipErrorInvalidValue;
+    if (n <= 0 || !sum || !input || !beta || !temp) return hipErrorInvalidValue;
     return batch_invert_ex((const Fr *)input, (const Fr *)beta, (Fr *)sum, init ? OUT_ADD : OUT_SET, (uint32_t)n,
-                           (Fr *)temp, stream);
+                           stream);
 }
 
 // cuda/bn254.cu:1936-1966: z in place; input (n Fr) is scratch for the scan.
@@ -518,28 +355,36 @@ hipError_t eval_logup_z_pure(void *z, void *input, void *table, void *last_z, in
                              hipStream_t stream) {
     (void)table;
     if (n <= 0 || !z || !input || !last_z || last_z_index < 0 || last_z_index >= n) return hipErrorInvalidValue;
-    return field_scan((Fr *)z, (uint32_t)n, false, (const Fr *)last_z, (Fr *)last_z, last_z_index, (Fr *)input,
+    return field_scan((Fr *)z, (uint32_t)n, (const Fr *)last_z, (Fr *)last_z, last_z_index, (Fr *)input,
                       stream);
 }
 
-// cuda/bn254.cu:1968-1993.  As in the reference, table is inverted in place
-// (1/(table + beta)) with z as temporary storage, then
-// z[i] = input[i] - m[i] * table[i], then the exclusive scan with carry
-// last_z[0] using input as scratch; last_z[0] = z[last_z_index] at the end.
+// cuda/bn254.cu:1968-1993.  z[i] = input[i] - m[i] / (table[i] + beta), then
+// the exclusive scan with carry last_z[0]; last_z[0] = z[last_z_index] at the
+// end.  The inversion's pass writes z and its tiles' sums, the latter into
+// table (scratch, as input is: the reference inverts table in place with z as
+// temporary storage).
 hipError_t eval_logup_z_compose(void *z, void *input, void *table, const void *multiplicity, const void *beta,
                                 void *last_z, int last_z_index, int n, hipStream_t stream) {
     if (n <= 0 || !z || !input || !table || !multiplicity || !beta || !last_z || last_z_index < 0 ||
         last_z_index >= n)
         return hipErrorInvalidValue;
-    ZK_CHECK(batch_invert_ex((const Fr *)table, (const Fr *)beta, (Fr *)table, OUT_SET, (uint32_t)n, (Fr *)z,
-                             stream));
-    uint32_t blocks = ((uint32_t)n + 255) / 256;
-    if (blocks > 16384) blocks = 16384;
-    k_logup_step2<<<blocks, 256, 0, stream>>>((Fr *)z, (const Fr *)input, (const Fr *)table, (const Fr *)multiplicity,
-                                               (uint32_t)n);
+    const uint32_t un = (uint32_t)n;
+    const int e = binv_elems(un);
+    const size_t tile = (size_t)kBT * e;
+    const uint32_t nb = (uint32_t)((un + tile - 1) / tile);
+    Fr *zz = (Fr *)z, *tab = (Fr *)table, *lz = (Fr *)last_z;
+    ZK_CHECK(binv_launch<OUT_LOGUP>(tab, (const Fr *)beta, zz, un, (const Fr *)input, (const Fr *)multiplicity,
+                                    stream));
+    k_fscan_top<<<1, 256, 0, stream>>>(tab, nb, tile, lz);
     ZK_CHECK(hipGetLastError());
-    return field_scan((Fr *)z, (uint32_t)n, false, (const Fr *)last_z, (Fr *)last_z, last_z_index, (Fr *)input,
-                      stream);
+    if (e == 2)
+        k_fscan_apply<2><<<nb, 256, 0, stream>>>(zz, un, tab, tile, lz, last_z_index);
+    else if (e == 4)
+        k_fscan_apply<4><<<nb, 256, 0, stream>>>(zz, un, tab, tile, lz, last_z_index);
+    else
+        k_fscan_apply<8><<<nb, 256, 0, stream>>>(zz, un, tab, tile, lz, last_z_index);
+    return hipGetLastError();
 }
 
 }  // extern "C"
