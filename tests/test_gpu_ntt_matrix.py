@@ -1,0 +1,90 @@
+"""NTT passes on the matrix cores (degrees 6 to 8, launches of at least 2^19
+elements) against the CPU oracle, bit for bit: every pair of inner sizes as
+first, middle and last pass, batches just below and at the threshold, extreme
+inputs (the byte columns' bounds), iNTT scaling and coset extensions."""
+import ctypes
+
+import numpy as np
+import pytest
+from test_gpu_field_ntt import _CosetItem, _gpu_ntt, _ntt_batch, _omegas_dev
+
+pytestmark = pytest.mark.gpu
+
+R = 0x30644E72E131A029B85045B68181585D2833E84879B9709143E1F593F0000001
+TOP = np.array([[(R - 1) >> (64 * i) & (2**64 - 1) for i in range(4)]], dtype=np.uint64)
+
+
+def _pattern(zo, kind, n, seed):
+    if kind == "random":
+        return zo.rand_fr(n, seed)
+    x = np.zeros((n, 4), dtype=np.uint64)
+    if kind == "top":
+        x[:] = TOP
+    elif kind == "top_odd":
+        x[1::2] = TOP
+    elif kind == "top_half":
+        x[n // 2:] = TOP
+    else:  # one element, the last
+        x[-1:] = TOP
+    return x
+
+
+# plans: 2^19 = 7 6 6, 2^20 = 7 7 6, 2^21 = 7 7 7, 2^22 = 8 7 7
+@pytest.mark.parametrize("log_n,kind,inverse", [(19, "top", False), (19, "top_odd", True), (20, "top_half", False),
+                                                (21, "random", True), (21, "last", False), (22, "top_odd", True)])
+def test_single_transform(gpu, zo, log_n, kind, inverse):
+    n = 1 << log_n
+    x = _pattern(zo, kind, n, 40 + log_n)
+    w, n_inv = zo.root_of_unity(log_n), None
+    if inverse:
+        w, n_inv = zo.fr_inv(w), zo.fr_inv(zo.fr_from_u64(n))
+        exp = zo.ntt(x, log_n, w, n_inv)
+    else:
+        exp = zo.ntt(x, log_n, w)
+    assert (_gpu_ntt(zo, x, log_n, w, n_inv) == exp).all()
+
+
+# 2^16 = 8 8 at the threshold, one transform short of it, and with others
+# beside it; 2^15 = 8 7; 2^12 = 6 6 over several launches
+@pytest.mark.parametrize("logs", [[16] * 8, [16] * 7 + [12, 14], [16] * 8 + [15, 12, 3], [15] * 16, [12] * 128,
+                                  [18, 17, 18, 13]])
+def test_batch(gpu, zo, logs):
+    specs, exps = [], []
+    for m, k in enumerate(logs):
+        x, w = _pattern(zo, "top" if m % 5 == 4 else "random", 1 << k, 700 + m), zo.root_of_unity(k)
+        if m % 3 == 2:
+            w, n_inv = zo.fr_inv(w), zo.fr_inv(zo.fr_from_u64(1 << k))
+            specs.append((x, k, w, n_inv))
+            exps.append(zo.ntt(x, k, w, n_inv))
+        else:
+            specs.append((x, k, w, None))
+            exps.append(zo.ntt(x, k, w))
+    got = _ntt_batch(zo, specs)
+    assert [m for m in range(len(logs)) if not (got[m] == exps[m]).all()] == []
+
+
+@pytest.mark.parametrize("shapes", [[(18, 1)], [(17, 2), (16, 3)], [(12, 4)] * 8, [(19, 3)]])
+def test_coset_extension(gpu, zo, shapes):
+    from zkprover import device as dv
+    from zkprover._lib import lib
+    f = lib().zk_coset_extend_batch
+    f.argtypes = [ctypes.c_void_p, ctypes.c_int, ctypes.c_void_p, ctypes.c_int, ctypes.c_void_p, ctypes.c_void_p]
+    f.restype = ctypes.c_int
+    zeta = zo.to_mont([pow(7, (R - 1) // 3, R)])
+    cp = np.concatenate([zeta, zo.fr_mul(zeta, zeta)])
+    keep, items, exps = [], (_CosetItem * len(shapes))(), []
+    for m, (log_n, ext) in enumerate(shapes):
+        n, N = 1 << log_n, 1 << (log_n + ext)
+        coeffs = _pattern(zo, "top" if m % 2 else "random", n, 60 + m)
+        w = zo.root_of_unity(log_n + ext)
+        host = np.zeros((N, 4), dtype=np.uint64)
+        host[:n] = coeffs
+        exps.append(zo.ntt(zo.extended_prepare(host, cp, n, N, 0), log_n + ext, w))
+        om, src, buf, tmp = _omegas_dev(zo, log_n + ext, w), dv.to_dev(coeffs), dv.empty(N), dv.empty(N)
+        keep.append((om, src, buf, tmp))
+        items[m] = _CosetItem(src.data_ptr(), buf.data_ptr(), tmp.data_ptr(), om.data_ptr(), log_n, ext)
+    dcp = dv.to_dev(cp)
+    sw = (ctypes.c_ubyte * len(shapes))()
+    assert f(ctypes.addressof(items), len(shapes), dcp.data_ptr(), 3, sw, dv.stream_handle()) == 0
+    for m, (_, _, buf, tmp) in enumerate(keep):
+        assert (dv.from_dev(tmp if sw[m] else buf) == exps[m]).all(), shapes[m]

@@ -14,7 +14,8 @@
 // runs as well.  Pass twiddles are read from the natural-order w^i table that
 // `expand_omega_buffer` builds (one gather per element, no extra multiply);
 // the 2^(d-1) in-pass twiddles are staged once per workgroup in LDS.  The
-// n^-1 scaling of the iNTT is fused into the last pass.
+// n^-1 scaling of the iNTT is fused into the last pass.  Passes of degree 6 to
+// 8 with enough elements run on the matrix cores instead (k_ntt_mfma).
 #include <stdlib.h>
 #include <string.h>
 
@@ -23,6 +24,7 @@
 
 #include "ff29.h"
 #include "guard.h"
+#include "ntt_mfma.h"
 #include "zkcore.h"
 #include "zkinternal.h"
 
@@ -426,6 +428,200 @@ __global__ __launch_bounds__(kThreads) void k_ntt_pass(const NttPassArgs a) {
     }
 }
 
+// A pass of radix 2^(LA + LB) on the matrix cores (ntt_mfma.h).  A wave's
+// tile is 256 elements, whole columns (1, 2 or 4), so its exchange needs no
+// barrier.  Persistent, one workgroup of 16 waves per CU: a workgroup takes a
+// contiguous range of the launch's tiles, rebuilds the matrix and the twiddles
+// in LDS where the transform changes and deals the tiles to its waves one by
+// one.  Job block0 counts tiles.
+//
+// Bound by VALU issue (855 instructions per element of a 2^7 pass with
+// inter-pass twiddles, two 29-bit products of about 260 among them; the
+// radix-2 kernel has 1270 to 1580), then by the last pass's scattered reads of the
+// omegas.  2^22 elements: first pass 107 us, middle 157 us, last 187 us,
+// against 173 us each in the radix-2 kernel.  Tried: 32x32x32 products with
+// 512 elements per wave (two waves per SIMD: 140 and 220 us), 2048-element
+// tiles per workgroup with barriers in the exchange (111, 151 and 171 us at
+// 2^22, but batches 17% slower: the older of two workgroups ran ahead and left
+// the CU half empty).  Registers: 128 (four waves per SIMD), which the two
+// phases' fences below keep from spilling.
+template <int LA, int LB, bool FIRST>
+__global__ __launch_bounds__(kMfmaThreads) void k_ntt_mfma(const NttPassArgs a, uint32_t tiles) {
+    __shared__ __attribute__((aligned(16))) uint8_t mlds[MfmaLds::bytes(LA, LB)];
+    __shared__ uint32_t next_tile;
+    constexpr int deg = LA + LB, SA = 1 << LA, SB = 1 << LB, D = 1 << deg;
+    constexpr uint32_t kCols = kMfmaTile >> deg, kLogCols = 8 - deg;
+    uint8_t *mat = mlds;
+    uint32_t *tw = reinterpret_cast<uint32_t *>(mlds + MfmaLds::kMat);
+    const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    uint8_t *xch = mlds + MfmaLds::kMat + MfmaLds::twiddles(deg) + wave * MfmaLds::exchange(LA, LB);
+    const uint32_t t1 = (uint32_t)((uint64_t)tiles * (blockIdx.x + 1) / gridDim.x);
+    uint32_t q = 0;
+    for (uint32_t t0 = (uint32_t)((uint64_t)tiles * blockIdx.x / gridDim.x), end; t0 < t1; t0 = end) {
+        while (q + 1 < a.count && a.job[q + 1].block0 <= t0) q++;
+        end = q + 1 < a.count && a.job[q + 1].block0 < t1 ? a.job[q + 1].block0 : t1;
+        const NttJob &job = a.job[q];
+        const Fr *__restrict__ omegas = job.omegas;
+        const uint32_t log_n = job.log_n, log_p = job.log_p, log_t = log_n - deg;
+        {
+            uint32_t tid = threadIdx.x;
+            asm volatile("" : "+v"(tid));  // not hoisted out of the loop
+            __syncthreads();               // every wave is done with the previous tables
+            if (tid == 0) next_tile = t0;
+            // matrix: powers of w_16 = omegas[n / 16]
+            if (tid < 512)
+                mfma_matrix_entry(mat, tid >> 5, tid & 31, fe_load<FrParams>(&omegas[(size_t)(tid >> 5) << (log_n - 4)]));
+            // twiddles w_D^e (n^-1), reduced, in the 2^261 domain, by the other half
+            if (tid >= 512 && tid < 512 + D) {
+                const uint32_t e = tid - 512;
+                Fr w = fe_load<FrParams>(&omegas[(size_t)e << log_t]);
+                if (job.n_inv) w = fr_mul_w29(w, f29_from32(fe_load<FrParams>(job.n_inv)));
+                for (int k = 0; k < 5; k++) w = w + w;
+                const F29 f = f29_repack(w.v);
+#pragma clang loop unroll(full)
+                for (int i = 0; i < 9; i++) tw[e * kMfmaTwWords + i] = f.l[i];
+            }
+            __syncthreads();
+        }
+        const Fr *__restrict__ x = job.x;
+        Fr *__restrict__ y = job.y;
+        const uint32_t nz = job.nz, cn = job.cn, p = 1u << log_p;
+        // column and k1 of DFT d after the exchange: the first pass stores runs
+        // of k1, later ones runs of columns
+        auto col_b = [&](uint32_t d) { return FIRST ? d >> LA : d & (kCols - 1); };
+        auto k1_b = [&](uint32_t d) { return FIRST ? d & (SA - 1) : d >> kLogCols; };
+        // the lane, opaque to the optimiser: what follows from it is computed
+        // anew in each phase instead of being kept in registers (it spilled)
+        auto lane_now = [&]() {
+            uint32_t l = threadIdx.x & 63;
+            asm volatile("" : "+v"(l));
+            return l;
+        };
+        // a wave takes the next tile when it is done with one: of two workgroups
+        // with a fixed share each, the older one won every issue slot, ended
+        // early and left the CU half empty
+        for (;;) {
+            uint32_t tile = 0;
+            if ((threadIdx.x & 63) == 0) tile = atomicAdd(&next_tile, 1u);
+            tile = __builtin_amdgcn_readfirstlane(tile);
+            if (tile >= end) break;
+            const uint32_t index0 = (tile - job.block0) * kCols;
+            uint32_t v[4][8];
+            F29 w[4];
+            auto twiddle = [&](int s) {
+                __builtin_amdgcn_sched_barrier(0);
+                f29_unpack(f29_mul<Fr29Mod>(f29_repack(v[s]), w[s]), v[s]);
+                __builtin_amdgcn_sched_barrier(0);
+            };
+            {
+                // load, columns from lane to lane; the coset scale or the inter-pass twiddle
+                const uint32_t lane = lane_now(), n = lane & 15, h = lane >> 4;
+                uint32_t pos[4];
+                Fr o[4];
+#pragma clang loop unroll(full)
+                for (int s = 0; s < 4; s++) {
+                    const uint32_t d = mfma_dft_index<LA>(s, n), i = mfma_in<LA>(s, h) * SB + (d >> kLogCols);
+                    const uint32_t c = index0 + (d & (kCols - 1));
+                    pos[s] = c + (i << log_t);
+                    const bool in = !FIRST || !nz || pos[s] < nz;
+                    const Fr e = fe_load<FrParams>(&x[in ? pos[s] : 0]);
+#pragma clang loop unroll(full)
+                    for (int k = 0; k < 8; k++) v[s][k] = e.v[k];
+                    if constexpr (!FIRST) o[s] = fe_load<FrParams>(&omegas[((c & (p - 1)) * i) << (log_t - log_p)]);
+                }
+                if constexpr (!FIRST) {
+#pragma clang loop unroll(full)
+                    for (int s = 0; s < 4; s++) {
+                        w[s] = f29_from32(o[s]);
+                        twiddle(s);
+                    }
+                } else if (nz) {
+#pragma clang loop unroll(full)
+                    for (int s = 0; s < 4; s++) {
+#pragma clang loop unroll(full)
+                        for (int k = 0; k < 8; k++) v[s][k] = pos[s] < nz ? v[s][k] : 0u;
+                    }
+                    if (cn > 1) {
+                        uint32_t r[4];
+#pragma clang loop unroll(full)
+                        for (int s = 0; s < 4; s++) {
+                            r[s] = pos[s] % cn;
+                            o[s] = fe_load<FrParams>(&job.coset[r[s] ? r[s] - 1 : 0]);
+                        }
+#pragma clang loop unroll(full)
+                        for (int s = 0; s < 4; s++) {
+                            if (((mfma_in<LA>(s, 0) * SB) << log_t) >= nz) continue;  // all zero
+                            uint32_t u[8];
+#pragma clang loop unroll(full)
+                            for (int k = 0; k < 8; k++) u[k] = v[s][k];
+                            w[s] = f29_from32(o[s]);
+                            twiddle(s);
+#pragma clang loop unroll(full)
+                            for (int k = 0; k < 8; k++) v[s][k] = r[s] ? v[s][k] : u[k];
+                        }
+                    }
+                }
+            }
+            mfma_dft<LA>(v, mat, lane_now());
+            {
+                // exchange: (column, j1) DFTs to (column, k1) DFTs, 16 bytes of each element at a time
+                const uint32_t lane = lane_now(), n = lane & 15, h = lane >> 4;
+                uint4 lo[4];
+#pragma clang loop unroll(full)
+                for (int hw = 0; hw < 2; hw++) {
+#pragma clang loop unroll(full)
+                    for (int s = 0; s < 4; s++) {
+                        const uint32_t d = mfma_dft_index<LA>(s, n);
+                        uint4 *q4 = reinterpret_cast<uint4 *>(xch + (d * (SA + 1) + mfma_out<LA>(s, h)) * 16);
+                        *q4 = make_uint4(v[s][4 * hw], v[s][4 * hw + 1], v[s][4 * hw + 2], v[s][4 * hw + 3]);
+                    }
+                    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "workgroup"); __builtin_amdgcn_wave_barrier();
+#pragma clang loop unroll(full)
+                    for (int s = 0; s < 4; s++) {
+                        const uint32_t d = mfma_dft_index<LB>(s, n);
+                        const uint4 c = *reinterpret_cast<const uint4 *>(
+                            xch + (((mfma_in<LB>(s, h) << kLogCols) + col_b(d)) * (SA + 1) + k1_b(d)) * 16);
+                        if (hw == 0) {
+                            lo[s] = c;
+                        } else {
+                            v[s][4] = c.x, v[s][5] = c.y, v[s][6] = c.z, v[s][7] = c.w;
+                            v[s][0] = lo[s].x, v[s][1] = lo[s].y, v[s][2] = lo[s].z, v[s][3] = lo[s].w;
+                        }
+                    }
+                    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "workgroup"); __builtin_amdgcn_wave_barrier();
+                }
+            }
+            {
+                // twiddles w_D^(j1 k1)
+                const uint32_t lane = lane_now(), n = lane & 15, h = lane >> 4;
+#pragma clang loop unroll(full)
+                for (int s = 0; s < 4; s++) {
+                    const uint32_t e = mfma_in<LB>(s, h) * k1_b(mfma_dft_index<LB>(s, n));
+                    const uint4 *t = reinterpret_cast<const uint4 *>(tw + e * kMfmaTwWords);
+                    const uint4 ta = t[0], tb = t[1];
+                    w[s] = F29{{ta.x, ta.y, ta.z, ta.w, tb.x, tb.y, tb.z, tb.w, t[2].x}};
+                    twiddle(s);
+                }
+            }
+            mfma_dft<LB>(v, mat, lane_now());
+            // store: canonical after the last pass, else below 1.01 r
+            const uint32_t lane = lane_now(), n = lane & 15, h = lane >> 4;
+            const bool last = log_p + deg == log_n;
+#pragma clang loop unroll(full)
+            for (int s = 0; s < 4; s++) {
+                const uint32_t d = mfma_dft_index<LB>(s, n), index = index0 + col_b(d), kk = index & (p - 1);
+                const uint32_t addr = ((index - kk) << deg) + kk + ((k1_b(d) + SA * mfma_out<LB>(s, h)) << log_p);
+                fr_cond_sub(v[s]);
+                if (last) fr_cond_sub(v[s]);
+                Fr e;
+#pragma clang loop unroll(full)
+                for (int k = 0; k < 8; k++) e.v[k] = v[s][k];
+                fe_store<FrParams>(&y[addr], e);
+            }
+        }
+    }
+}
+
 // buf[i] = w^i for i in [2, n) given buf[1] = w (cuda/bn254.cu:1073-1094)
 __global__ void k_expand_omega(Fr *buf, uint32_t n, uint32_t chunk) {
     uint32_t t = blockIdx.x * blockDim.x + threadIdx.x;
@@ -508,6 +704,87 @@ static uint32_t register_rounds_enabled() {
     return on;
 }
 
+static void fill_job(NttJob &j, const NttSpec &sp, int r, int np, uint32_t logp, uint32_t deg, uint32_t block0) {
+    j.x = (r & 1) ? sp.b : sp.a;
+    j.y = (r & 1) ? sp.a : sp.b;
+    if (r == 0 && sp.src) {
+        j.x = sp.src;
+        j.nz = sp.nz;
+        j.coset = sp.coset;
+        j.cn = sp.cn;
+    }
+    j.omegas = sp.omegas;
+    j.n_inv = r == np - 1 ? sp.n_inv : nullptr;
+    j.block0 = block0;
+    j.log_n = (uint8_t)sp.log_n;
+    j.log_p = (uint8_t)logp;
+    j.deg = (uint8_t)deg;
+}
+
+// The degrees whose passes of round r go to the matrix cores: 6 to 8, where
+// the launch has at least 2^19 elements (two waves of 256 elements for each
+// SIMD).  Below that a pass is one tile's latency plus the tables, and the
+// radix-2 kernel with its shorter chains is as fast or faster (one transform,
+// both ways: 2^18 57 us here and 52 there, 2^19 79 and 87, 2^20 114 and 145;
+// eight transforms: 2^15 44 and 44, 2^16 61 and 65, 2^18 187 and 226).
+constexpr uint32_t kMfmaMinElems = 1u << 19;
+constexpr uint32_t kMfmaMinLog = 12;  // the tables of a smaller transform would cost more than its tiles
+static bool mfma_degree(const NttSpec &sp, uint32_t deg) { return sp.log_n >= kMfmaMinLog && deg >= 6 && deg <= 8; }
+static uint32_t mfma_degrees(const NttSpec *specs, uint32_t count, const uint32_t *degs, const int *np, int r) {
+    uint64_t elems[9] = {};
+    for (uint32_t m = 0; m < count; m++) {
+        if (r >= np[m]) continue;
+        const uint32_t deg = degs[(size_t)m * 32 + r];
+        if (mfma_degree(specs[m], deg)) elems[deg] += 1ull << specs[m].log_n;
+    }
+    uint32_t set = 0;
+    for (uint32_t d = 6; d <= 8; d++) set |= elems[d] >= kMfmaMinElems ? 1u << d : 0u;
+    return register_rounds_enabled() ? set : 0u;
+}
+
+// one workgroup (of four waves per SIMD) on each CU
+constexpr uint32_t kMfmaGrid = 256;
+
+// pass r of every transform whose degree is in set, one launch per degree and
+// kJobsPerLaunch transforms
+template <int LA, int LB, bool FIRST>
+static hipError_t mfma_launch(NttPassArgs &args, uint32_t &tiles, hipStream_t stream) {
+    if (args.count) {
+        const uint32_t blocks = (tiles + 3) / 4;
+        k_ntt_mfma<LA, LB, FIRST><<<blocks < kMfmaGrid ? blocks : kMfmaGrid, kMfmaThreads, 0, stream>>>(args, tiles);
+        ZK_CHECK(hipGetLastError());
+    }
+    memset(&args, 0, sizeof(args));
+    tiles = 0;
+    return hipSuccess;
+}
+static hipError_t mfma_round(const NttSpec *specs, uint32_t count, const uint32_t *degs, const int *np,
+                             const uint32_t *logp, int r, uint32_t set, hipStream_t stream) {
+    for (uint32_t d = 6; d <= 8; d++) {
+        if (!(set >> d & 1)) continue;
+        auto launch = [&](NttPassArgs &args, uint32_t &tiles) {
+            if (r == 0)
+                return d == 8   ? mfma_launch<4, 4, true>(args, tiles, stream)
+                       : d == 7 ? mfma_launch<4, 3, true>(args, tiles, stream)
+                                : mfma_launch<3, 3, true>(args, tiles, stream);
+            return d == 8   ? mfma_launch<4, 4, false>(args, tiles, stream)
+                   : d == 7 ? mfma_launch<4, 3, false>(args, tiles, stream)
+                            : mfma_launch<3, 3, false>(args, tiles, stream);
+        };
+        NttPassArgs args;
+        memset(&args, 0, sizeof(args));
+        uint32_t tiles = 0;
+        for (uint32_t m = 0; m < count; m++) {
+            if (r >= np[m] || degs[(size_t)m * 32 + r] != d || !mfma_degree(specs[m], d)) continue;
+            fill_job(args.job[args.count++], specs[m], r, np[m], logp[m], d, tiles);
+            tiles += 1u << (specs[m].log_n - 8);
+            if (args.count == kJobsPerLaunch) ZK_CHECK(launch(args, tiles));
+        }
+        ZK_CHECK(launch(args, tiles));
+    }
+    return hipSuccess;
+}
+
 hipError_t ntt_run_batch(const NttSpec *specs, uint32_t count, hipStream_t stream, int *passes) {
     std::vector<uint32_t> degs((size_t)count * 32);
     std::vector<int> np(count);
@@ -519,6 +796,8 @@ hipError_t ntt_run_batch(const NttSpec *specs, uint32_t count, hipStream_t strea
         if (passes) passes[m] = np[m];
     }
     for (int r = 0; r < rounds; r++) {
+        const uint32_t mfma = mfma_degrees(specs, count, degs.data(), np.data(), r);
+        ZK_CHECK(mfma_round(specs, count, degs.data(), np.data(), logp.data(), r, mfma, stream));
         NttPassArgs args;
         memset(&args, 0, sizeof(args));
         args.reg_rounds = register_rounds_enabled();
@@ -539,25 +818,16 @@ hipError_t ntt_run_batch(const NttSpec *specs, uint32_t count, hipStream_t strea
             const NttSpec &sp = specs[m];
             const uint32_t n = 1u << sp.log_n;
             const uint32_t deg = degs[(size_t)m * 32 + r];
+            if (mfma >> deg & 1 && mfma_degree(sp, deg)) {
+                logp[m] += deg;
+                continue;
+            }
             uint32_t tile = n < kTile ? n : kTile;
             uint32_t log_tile = log2_exact(tile);
             uint32_t log_g = log_tile > deg ? log_tile - deg : 0;
             uint32_t tile_elems = (1u << deg) << log_g;
             NttJob &j = args.job[args.count++];
-            j.x = (r & 1) ? sp.b : sp.a;
-            j.y = (r & 1) ? sp.a : sp.b;
-            if (r == 0 && sp.src) {
-                j.x = sp.src;
-                j.nz = sp.nz;
-                j.coset = sp.coset;
-                j.cn = sp.cn;
-            }
-            j.omegas = sp.omegas;
-            j.n_inv = r == np[m] - 1 ? sp.n_inv : nullptr;
-            j.block0 = blocks;
-            j.log_n = (uint8_t)sp.log_n;
-            j.log_p = (uint8_t)logp[m];
-            j.deg = (uint8_t)deg;
+            fill_job(j, sp, r, np[m], logp[m], deg, blocks);
             j.log_g = (uint8_t)log_g;
             blocks += n / tile_elems;
             // the tile, then D/2 twiddles (29-bit form: 36 B each)
