@@ -13,6 +13,7 @@
 // staged once per workgroup in LDS instead of being re-read per row.
 #include <string.h>
 
+#include "ff29.h"
 #include "zkcore.h"
 
 using namespace zk;
@@ -29,6 +30,60 @@ uint32_t grid_for(uint32_t n) {
 
 __device__ __forceinline__ Fr ld(const Fr *p) { return fe_load<FrParams>(p); }
 __device__ __forceinline__ void st(Fr *p, const Fr &v) { fe_store<FrParams>(p, v); }
+
+// Row arithmetic of the folds in lazy 29-bit limbs.  With 32-bit products
+// they were bound by VALU issue; here a fold t y + a b is one f29_mul2, two
+// products under one reduction, and nothing is reduced below r before the
+// store.  2^22 rows: logup fold 358 -> 291 us, shuffle 360 -> 267, first
+// permutation fold 209 -> 169 (273, 210 and 157 us of traffic), permutation
+// product of four columns 723 -> 660 (18 products a row, still VALU-bound).
+// The term list of k_batch_mul_sum stays in 32-bit products: it is bound by
+// its loads (384 us, 400 with these).
+//
+// An operand of a product enters as it is (lo) or times 2^5 (hi): lo x hi
+// stays in the stored 2^256 domain, hi x hi in the 2^261 domain.  Bounds: a
+// product is below (1 + sum a b / (169 r^2)) r, stored values are below r,
+// every product of lo and hi here below 2 r; one operand of a pair may have limbs up
+// to 2^30.6 (sums without carries).
+__device__ __forceinline__ F29 lo(const Fr &x) { return f29_repack(x.v); }
+__device__ __forceinline__ F29 hi(const Fr &x) { return f29_from32(x); }
+__device__ __forceinline__ F29 mul(const F29 &a, const F29 &b) { return f29_mul<Fr29Mod>(a, b); }
+__device__ __forceinline__ F29 mul2(const F29 &a, const F29 &b, const F29 &c, const F29 &d) {
+    return f29_mul2<Fr29Mod>(a, b, c, d);
+}
+__device__ __forceinline__ F29 add_nc(const F29 &a, const F29 &b) {
+    F29 r;
+#pragma unroll
+    for (int i = 0; i < 9; i++) r.l[i] = a.l[i] + b.l[i];
+    return r;
+}
+// 4 r, every limb but the top raised by 2^29 that is taken from the next: no
+// limb of a difference is negative
+constexpr uint32_t kR4x29[9] = {0x20000004u, 0x3c3eb27du, 0x39709142u, 0x3f4243ccu, 0x36174a0bu,
+                                0x2b6d0301u, 0x229b8503u, 0x397098cfu, 0x00c19138u};
+__device__ __forceinline__ F29 sub_nc(const F29 &a, const F29 &b) {  // a + 4 r - b, b < 3 r
+    F29 r;
+#pragma unroll
+    for (int i = 0; i < 9; i++) r.l[i] = a.l[i] + kR4x29[i] - b.l[i];
+    return r;
+}
+// a + r - b (< 2 r) and r - b
+__device__ __forceinline__ Fr sub_lazy(const Fr &a, const Fr &b) {
+    Fr t;
+    uint32_t c = 0, br = 0;
+#pragma unroll
+    for (int i = 0; i < 8; i++) t.v[i] = add_cc(a.v[i], FrParams::M[i], c);
+#pragma unroll
+    for (int i = 0; i < 8; i++) t.v[i] = sub_bb(t.v[i], b.v[i], br);
+    return t;
+}
+__device__ __forceinline__ Fr neg_lazy(const Fr &b) {
+    Fr t;
+    uint32_t br = 0;
+#pragma unroll
+    for (int i = 0; i < 8; i++) t.v[i] = sub_bb(FrParams::M[i], b.v[i], br);
+    return t;
+}
 
 #define GRID_LOOP(i, n)                                                \
     for (uint32_t i = blockIdx.x * blockDim.x + threadIdx.x; i < (n); \
@@ -123,30 +178,26 @@ __global__ void k_field_mul_zip(Fr *buf, const Fr *__restrict__ coeff, uint32_t 
 __global__ void k_perm_p1(Fr *res, const Fr *__restrict__ first, const Fr *__restrict__ last,
                           const Fr *__restrict__ l0, const Fr *__restrict__ l_last, const Fr *__restrict__ yp,
                           uint32_t n) {
-    Fr y = ld(yp), one = fe_one<FrParams>();
+    const F29 y = hi(ld(yp));
+    const Fr one = fe_one<FrParams>();
     GRID_LOOP(i, n) {
-        Fr t1 = ld(&res[i]) * y;
-        t1 = t1 + (one - ld(&first[i])) * ld(&l0[i]);
-        t1 = t1 * y;
-        Fr ls = ld(&last[i]);
-        t1 = t1 + (fe_sqr<FrParams>(ls) - ls) * ld(&l_last[i]);
-        st(&res[i], t1);
+        F29 t = mul2(lo(ld(&res[i])), y, lo(sub_lazy(one, ld(&first[i]))), hi(ld(&l0[i])));
+        const Fr ls = ld(&last[i]);
+        t = mul2(t, y, mul(lo(ls), hi(sub_lazy(ls, one))), hi(ld(&l_last[i])));
+        st(&res[i], f29_to_fr(t));
     }
 }
 
 // cuda/bn254.cu:704-739 (also logup_eval_h_z_set)
 __global__ void k_perm_p2(Fr *res, const Fr *const *__restrict__ set, const Fr *__restrict__ l0,
                           const Fr *__restrict__ yp, int n_set, int rot, uint32_t n) {
-    Fr y = ld(yp);
+    const F29 y = hi(ld(yp));
     GRID_LOOP(i, n) {
         uint32_t rp = (i + n + (uint32_t)rot) & (n - 1);
-        Fr t1 = ld(&res[i]);
-        Fr l = ld(&l0[i]);
-        for (int j = 1; j < n_set; j++) {
-            t1 = t1 * y;
-            t1 = t1 + (ld(&set[j][i]) - ld(&set[j - 1][rp])) * l;
-        }
-        st(&res[i], t1);
+        F29 t = lo(ld(&res[i]));
+        const F29 l = hi(ld(&l0[i]));
+        for (int j = 1; j < n_set; j++) t = mul2(t, y, lo(sub_lazy(ld(&set[j][i]), ld(&set[j - 1][rp]))), l);
+        st(&res[i], f29_to_fr(t));
     }
 }
 
@@ -166,36 +217,27 @@ __global__ void k_logup_eval_h(Fr *res, const Fr *__restrict__ ip, const Fr *__r
                                const Fr *__restrict__ table, const Fr *__restrict__ m, const Fr *__restrict__ zf,
                                const Fr *__restrict__ zl, const Fr *__restrict__ l0, const Fr *__restrict__ l_last,
                                const Fr *__restrict__ l_active, const Fr *__restrict__ yp, int rot, uint32_t n) {
-    Fr y = ld(yp);
+    const F29 y = hi(ld(yp));
     GRID_LOOP(i, n) {
         uint32_t rn = (i + (uint32_t)rot) & (n - 1);
-        Fr t = ld(&res[i]) * y;
-        Fr z = ld(&zf[i]);
-        t = t + ld(&l0[i]) * z;
-        t = t * y;
-        t = t + ld(&l_last[i]) * ld(&zl[i]);
-        t = t * y;
-        Fr tb = ld(&table[i]);
-        Fr u = (ld(&zf[rn]) - z) * tb;
-        u = u + ld(&m[i]);
-        u = u * ld(&ip[i]);
-        u = u - tb * ld(&ips[i]);
-        u = u * ld(&l_active[i]);
-        st(&res[i], t + u);
+        const Fr z = ld(&zf[i]);
+        F29 t = mul2(lo(ld(&res[i])), y, lo(ld(&l0[i])), hi(z));
+        t = mul2(t, y, lo(ld(&l_last[i])), hi(ld(&zl[i])));
+        const F29 tb = lo(ld(&table[i]));
+        F29 u = add_nc(mul(lo(sub_lazy(ld(&zf[rn]), z)), f29_shl5(tb)), lo(ld(&m[i])));  // < 2.4 r
+        u = mul2(u, hi(ld(&ip[i])), tb, hi(neg_lazy(ld(&ips[i]))));
+        st(&res[i], f29_to_fr(mul2(t, y, u, hi(ld(&l_active[i])))));
     }
 }
 
 // cuda/bn254.cu:920-949
 __global__ void k_logup_extra(Fr *res, const Fr *__restrict__ ip, const Fr *__restrict__ ips, const Fr *__restrict__ zp,
                               const Fr *__restrict__ l_active, const Fr *__restrict__ yp, int rot, uint32_t n) {
-    Fr y = ld(yp);
+    const F29 y = hi(ld(yp));
     GRID_LOOP(i, n) {
         uint32_t rn = (i + (uint32_t)rot) & (n - 1);
-        Fr t = ld(&res[i]) * y;
-        Fr u = (ld(&zp[rn]) - ld(&zp[i])) * ld(&ip[i]);
-        u = u - ld(&ips[i]);
-        u = u * ld(&l_active[i]);
-        st(&res[i], t + u);
+        const F29 u = add_nc(mul(lo(sub_lazy(ld(&zp[rn]), ld(&zp[i]))), hi(ld(&ip[i]))), lo(neg_lazy(ld(&ips[i]))));
+        st(&res[i], f29_to_fr(mul2(u, hi(ld(&l_active[i])), lo(ld(&res[i])), y)));
     }
 }
 
@@ -218,26 +260,23 @@ __global__ void k_inputs_product_sum(Fr *__restrict__ prod, Fr *__restrict__ psu
     }
 }
 
-// shared tail of the two shuffle kernels (cuda/bn254.cu:990-1013, :1049-1068)
-__device__ __forceinline__ Fr shuffle_fold(const Fr &res, const Fr &lhs, const Fr &rhs, const Fr &z, const Fr &zn,
-                                           const Fr &l0, const Fr &l_last, const Fr &l_active, const Fr &y) {
-    Fr one = fe_one<FrParams>();
-    Fr t = res * y;
-    t = t + l0 * (one - z);
-    t = t * y;
-    t = t + l_last * (z * z - z);
-    t = t * y;
-    Fr u = rhs * zn - lhs * z;
-    return t + u * l_active;
+// shared tail of the two shuffle kernels (cuda/bn254.cu:990-1013, :1049-1068);
+// lhs, rhs < 2 r
+__device__ __forceinline__ Fr shuffle_fold(const Fr &res, const F29 &lhs, const F29 &rhs, const Fr &z, const Fr &zn,
+                                           const Fr &l0, const Fr &l_last, const Fr &l_active, const F29 &y) {
+    const Fr one = fe_one<FrParams>();
+    F29 t = mul2(lo(res), y, lo(l0), hi(sub_lazy(one, z)));
+    t = mul2(t, y, mul(lo(z), hi(sub_lazy(z, one))), hi(l_last));
+    return f29_to_fr(mul2(t, y, mul2(rhs, hi(zn), lhs, hi(neg_lazy(z))), hi(l_active)));
 }
 
 __global__ void k_shuffle(Fr *res, const Fr *__restrict__ input, const Fr *__restrict__ table, const Fr *__restrict__ zp,
                           const Fr *__restrict__ l0, const Fr *__restrict__ l_last, const Fr *__restrict__ l_active,
                           const Fr *__restrict__ yp, int rot, uint32_t n) {
-    Fr y = ld(yp);
+    const F29 y = hi(ld(yp));
     GRID_LOOP(i, n) {
         uint32_t rn = (i + (uint32_t)rot) & (n - 1);
-        st(&res[i], shuffle_fold(ld(&res[i]), ld(&input[i]), ld(&table[i]), ld(&zp[i]), ld(&zp[rn]), ld(&l0[i]),
+        st(&res[i], shuffle_fold(ld(&res[i]), lo(ld(&input[i])), lo(ld(&table[i])), ld(&zp[i]), ld(&zp[rn]), ld(&l0[i]),
                                  ld(&l_last[i]), ld(&l_active[i]), y));
     }
 }
@@ -246,16 +285,16 @@ __global__ void k_shuffle_v2(Fr *res, const Fr *const *__restrict__ inputs, cons
                              const Fr *__restrict__ betas, int group_len, const Fr *__restrict__ zp,
                              const Fr *__restrict__ l0, const Fr *__restrict__ l_last, const Fr *__restrict__ l_active,
                              const Fr *__restrict__ yp, int rot, uint32_t n) {
-    Fr y = ld(yp);
+    const F29 y = hi(ld(yp));
     GRID_LOOP(i, n) {
         uint32_t rn = (i + (uint32_t)rot) & (n - 1);
         Fr b0 = ld(&betas[0]);
-        Fr l = ld(&inputs[0][i]) + b0;
-        Fr r = ld(&tables[0][i]) + b0;
+        F29 l = lo(ld(&inputs[0][i]) + b0);
+        F29 r = lo(ld(&tables[0][i]) + b0);
         for (int j = 1; j < group_len; j++) {
-            Fr bj = ld(&betas[j]);
-            l = l * (ld(&inputs[j][i]) + bj);
-            r = r * (ld(&tables[j][i]) + bj);
+            const F29 bj = hi(ld(&betas[j]));
+            l = mul(add_nc(hi(ld(&inputs[j][i])), bj), l);  // factors < 64 r
+            r = mul(add_nc(hi(ld(&tables[j][i])), bj), r);
         }
         st(&res[i], shuffle_fold(ld(&res[i]), l, r, ld(&zp[i]), ld(&zp[rn]), ld(&l0[i]), ld(&l_last[i]),
                                  ld(&l_active[i]), y));
@@ -340,22 +379,27 @@ __global__ void k_perm_set_eval(Fr *h, const Fr *__restrict__ z, const Fr *const
                                 const Fr *__restrict__ gamma, const Fr *__restrict__ bd, const Fr *__restrict__ X,
                                 const Fr *__restrict__ l_active, const Fr *__restrict__ yp, int rot, uint32_t n) {
     __shared__ const Fr *sv[kMaxPermCols], *ss[kMaxPermCols];
+    __shared__ F29 sb[kMaxPermCols];
     if (threadIdx.x < (unsigned)nc) {
         sv[threadIdx.x] = v[threadIdx.x];
         ss[threadIdx.x] = sig[threadIdx.x];
+        sb[threadIdx.x] = hi(ld(&bd[threadIdx.x]));
     }
     __syncthreads();
-    const Fr b = ld(beta), g = ld(gamma), y = ld(yp);
+    const F29 b = hi(ld(beta)), y = hi(ld(yp));
+    const Fr g = ld(gamma);
     GRID_LOOP(i, n) {
         const uint32_t rn = (i + (uint32_t)rot) & (n - 1);
-        const Fr x = ld(&X[i]);
-        Fr l = ld(&z[rn]), r = ld(&z[i]);
+        const F29 x = hi(ld(&X[i]));
+        F29 l = lo(ld(&z[rn])), r = lo(ld(&z[i]));
         for (int c = 0; c < nc; c++) {
-            const Fr vg = ld(&sv[c][i]) + g;
-            l = l * (vg + b * ld(&ss[c][i]));
-            r = r * (vg + ld(&bd[c]) * x);
+            // factors in the 2^261 domain: 32 (v + gamma) < 32 r and a product of
+            // two hi operands < 7.1 r; l and r stay below 1.4 r
+            const F29 vg = hi(ld(&sv[c][i]) + g);
+            l = mul(add_nc(vg, mul(b, hi(ld(&ss[c][i])))), l);
+            r = mul(add_nc(vg, mul(sb[c], x)), r);
         }
-        st(&h[i], ld(&h[i]) * y + ld(&l_active[i]) * (l - r));
+        st(&h[i], f29_to_fr(mul2(sub_nc(l, r), hi(ld(&l_active[i])), lo(ld(&h[i])), y)));
     }
 }
 
@@ -375,12 +419,14 @@ struct GateArgs {
 };
 __global__ __launch_bounds__(kThreads) void k_gate_eval(Fr *__restrict__ h, const GateArgs g,
                                                         const Fr *__restrict__ yp, uint32_t n) {
-    const Fr y = ld(yp);
+    const F29 y = hi(ld(yp));
     GRID_LOOP(i, n) {
-        const Fr a = ld(&g.a[i]);
-        Fr acc = a * ld(&g.b[i]) + ld(&g.c[i]) - ld(&g.d[i]);
-        for (int k = 0; k < g.ng; k++) acc = acc * y + (ld(&g.f[k][i]) * a - ld(&g.e[k][i]));
-        st(&h[i], ld(&g.q[i]) * acc);
+        const F29 a = hi(ld(&g.a[i]));
+        // acc < 3.3 r
+        F29 acc = add_nc(mul(lo(ld(&g.b[i])), a), lo(sub_lazy(ld(&g.c[i]), ld(&g.d[i]))));
+        for (int k = 0; k < g.ng; k++)
+            acc = add_nc(mul2(acc, y, lo(ld(&g.f[k][i])), a), lo(neg_lazy(ld(&g.e[k][i]))));
+        st(&h[i], f29_to_fr(mul(acc, hi(ld(&g.q[i])))));
     }
 }
 

@@ -127,6 +127,7 @@ __device__ __forceinline__ F29 f29_mul(const F29 &a, const F29 &b) {
 // products (the sum of the two a*b-type terms and the m*p terms of a column
 // is at most 27 values < 2^58); valid for a * b + c * d < 2^261 * p, e.g. all
 // four < 2p
+template <class Q = Fp29Mod>
 __device__ __forceinline__ F29 f29_mul2(const F29 &a, const F29 &b, const F29 &c, const F29 &d) {
     uint32_t m[9];
     F29 r;
@@ -143,11 +144,11 @@ __device__ __forceinline__ F29 f29_mul2(const F29 &a, const F29 &b, const F29 &c
         uint64_t u = 0;
 #pragma unroll
         for (int i = lo; i <= hi; i++)
-            if (i < k) u += (uint64_t)m[i] * kP29[k - i];
+            if (i < k) u += (uint64_t)m[i] * Q::P[k - i];
         acc += t0 + t1 + u;
         if (k < 9) {
-            m[k] = ((uint32_t)acc * kPInv29) & kM29;
-            acc += (uint64_t)m[k] * kP29[0];
+            m[k] = ((uint32_t)acc * Q::PINV) & kM29;
+            acc += (uint64_t)m[k] * Q::P[0];
         } else {
             r.l[k - 9] = (uint32_t)acc & kM29;
         }
