@@ -435,16 +435,16 @@ __global__ __launch_bounds__(kThreads) void k_ntt_pass(const NttPassArgs a) {
 // in LDS where the transform changes and deals the tiles to its waves one by
 // one.  Job block0 counts tiles.
 //
-// Bound by VALU issue (855 instructions per element of a 2^7 pass with
-// inter-pass twiddles, two 29-bit products of about 260 among them; the
-// radix-2 kernel has 1270 to 1580), then by the last pass's scattered reads of the
-// omegas.  2^22 elements: first pass 107 us, middle 157 us, last 187 us,
-// against 173 us each in the radix-2 kernel.  Tried: 32x32x32 products with
-// 512 elements per wave (two waves per SIMD: 140 and 220 us), 2048-element
-// tiles per workgroup with barriers in the exchange (111, 151 and 171 us at
-// 2^22, but batches 17% slower: the older of two workgroups ran ahead and left
-// the CU half empty).  Registers: 128 (four waves per SIMD), which the two
-// phases' fences below keep from spilling.
+// Bound by VALU issue (about 800 instructions per element of a 2^7 pass with
+// inter-pass twiddles, two 29-bit products of 260 among them; the radix-2
+// kernel has 1270 to 1580), then by the last pass's scattered reads of the
+// omegas.  2^22 elements: first pass 98 us, middle 157 us, last 184 us, against
+// 173 us each in the radix-2 kernel.  Tried: 32x32x32 products with 512
+// elements per wave (two waves per SIMD: 140 and 220 us), 2048-element tiles
+// per workgroup with barriers in the exchange (batches 17% slower: the older
+// of two workgroups ran ahead and left the CU half empty).  Registers: 128
+// (four waves per SIMD), which the phases' separate lane values and the
+// scheduling barriers below keep from spilling.
 template <int LA, int LB, bool FIRST>
 __global__ __launch_bounds__(kMfmaThreads) void k_ntt_mfma(const NttPassArgs a, uint32_t tiles) {
     __shared__ __attribute__((aligned(16))) uint8_t mlds[MfmaLds::bytes(LA, LB)];
@@ -604,14 +604,13 @@ __global__ __launch_bounds__(kMfmaThreads) void k_ntt_mfma(const NttPassArgs a, 
                 }
             }
             mfma_dft<LB>(v, mat, lane_now());
-            // store: canonical after the last pass, else below 1.01 r
+            // store: canonical after the last pass, else below 1.001 r
             const uint32_t lane = lane_now(), n = lane & 15, h = lane >> 4;
             const bool last = log_p + deg == log_n;
 #pragma clang loop unroll(full)
             for (int s = 0; s < 4; s++) {
                 const uint32_t d = mfma_dft_index<LB>(s, n), index = index0 + col_b(d), kk = index & (p - 1);
                 const uint32_t addr = ((index - kk) << deg) + kk + ((k1_b(d) + SA * mfma_out<LB>(s, h)) << log_p);
-                fr_cond_sub(v[s]);
                 if (last) fr_cond_sub(v[s]);
                 Fr e;
 #pragma clang loop unroll(full)

@@ -35,8 +35,8 @@
 //
 // Bounds: matrix entries are at most r / 2 in size and bytes 2^7, so a column
 // sum of 8 x 32 terms is at most 2^22 and a value 2^14 r; the fold returns
-// values in (0.99 r, 2.01 r), the twiddle product (reduced twiddle, 2^261 >
-// 169 r) 1.02 r, inter-pass twiddled input 1.2 r: u stays below 2.64 r < 2^255.
+// values in (0, 1.001 r), the twiddle product (reduced twiddle, 2^261 >
+// 169 r) 1.01 r, inter-pass twiddled input 1.2 r: u stays below 2.4 r < 2^255.
 #pragma once
 #include "ff29.h"
 #include "zkcore.h"
@@ -100,23 +100,23 @@ __device__ __forceinline__ void mfma_matrix_entry(uint8_t *mat, uint32_t e, uint
 }
 
 // One output from its 32 byte columns, added in pairs (z_j = y_2j + 2^8
-// y_2j+1, |y| <= 2^22): sum z_j 2^(16j) reduced into (0.99 r, 2.01 r).  The
-// quotient comes from the top two pairs.
+// y_2j+1, |y| <= 2^22): V = sum z_j 2^(16j) less q r, in (0, 1.001 r).  The
+// quotient comes from the top two pairs: with T = z15 2^16 + z14 in units of
+// 2^224, m = floor(floor(T / 2^15) 2^60 / (r / 2^224) / 2^32) is 2^13 V / r to
+// within (-0.3, 1.6) (the pairs below add 0.2, the two floors 0.4 and 1, the
+// constant 0.1), so q = floor((m - 2) / 2^13) never exceeds V / r.
 __device__ __forceinline__ void mfma_fold(uint32_t out[8], const int32_t (&z)[16]) {
-    // T = z15 2^16 + z14 in units of 2^224; q = floor(T / (r / 2^224)) to
-    // within one, from T / 2^15 times 2^(15 + 32 + 13) / (r / 2^224) / 2^15
     const int32_t t15 = (int32_t)((uint32_t)z[15] << 1) + (z[14] >> 15);
     // 2^60 / 811880050.88 = 1420063842.4
-    const int32_t q = __mulhi(t15, 1420063842) >> 13;
-    const int32_t nq = 1 - q;
-    int64_t acc = 0;
+    const int32_t nq = -((__mulhi(t15, 1420063842) - 2) >> 13);
+    int32_t carry = 0;  // below 2^16 in size: fits beside an even pair
 #pragma clang loop unroll(full)
     for (int j = 0; j < 8; j++) {
+        int64_t acc = z[2 * j] + carry;
         acc += (int64_t)z[2 * j + 1] * 65536;
         acc += (int64_t)nq * kRho[j];
-        acc += z[2 * j];
         out[j] = (uint32_t)acc;
-        acc >>= 32;
+        carry = (int32_t)(acc >> 32);
     }
 }
 
