@@ -1,7 +1,7 @@
 """NTT passes on the matrix cores (degrees 6 to 8, launches of at least 2^19
-elements) against the CPU oracle, bit for bit: every pair of inner sizes as
-first, middle and last pass, batches just below and at the threshold, extreme
-inputs (the byte columns' bounds), iNTT scaling and coset extensions."""
+elements) against the CPU oracle, bit for bit: the degrees in first,
+middle and last passes (degree 8: first only), batches just below and at the threshold, extreme
+inputs (the byte columns' bounds), iNTT scaling, coset extensions and capture."""
 import ctypes
 
 import numpy as np
@@ -88,3 +88,41 @@ def test_coset_extension(gpu, zo, shapes):
     assert f(ctypes.addressof(items), len(shapes), dcp.data_ptr(), 3, sw, dv.stream_handle()) == 0
     for m, (_, _, buf, tmp) in enumerate(keep):
         assert (dv.from_dev(tmp if sw[m] else buf) == exps[m]).all(), shapes[m]
+
+
+def test_captured_batch_replays(gpu, zo):
+    """a captured batch replays to the oracle's bytes, with its buffers cleared
+    and other eager work between the replays"""
+    import torch
+    from test_gpu_graph import _NttItem
+    from zkprover import device as dv
+    from zkprover._lib import call
+    stream = torch.cuda.Stream()
+    sh = stream.cuda_stream
+    logs = [18, 18, 16]
+    xs = [zo.rand_fr(1 << k, 90 + m) for m, k in enumerate(logs)]
+    ws = [zo.root_of_unity(k) for k in logs]
+    oms = [_omegas_dev(zo, k, w) for k, w in zip(logs, ws)]
+    orig = [dv.to_dev(x) for x in xs]
+    bufs, tmps = [dv.empty(1 << k) for k in logs], [dv.empty(1 << k) for k in logs]
+    items = (_NttItem * len(logs))(*[_NttItem(bufs[m].data_ptr(), tmps[m].data_ptr(), oms[m].data_ptr(), None, k, 0)
+                                     for m, k in enumerate(logs)])
+    swapped, exec_ = (ctypes.c_ubyte * len(logs))(), ctypes.c_void_p()
+    torch.cuda.synchronize()
+    call("zk_graph_begin", sh)
+    for m, k in enumerate(logs):
+        call("zk_copy", bufs[m].data_ptr(), orig[m].data_ptr(), (1 << k) * 32, sh)
+    call("zk_ntt_batch", ctypes.addressof(items), len(logs), ctypes.addressof(swapped), sh)
+    call("zk_graph_end", sh, ctypes.byref(exec_))
+    exps = [zo.ntt(x, k, w) for x, k, w in zip(xs, logs, ws)]
+    try:
+        for rep in range(3):
+            for b in bufs + tmps:
+                b.zero_()
+            torch.cuda.synchronize()
+            call("zk_graph_launch", exec_, sh)
+            torch.cuda.synchronize()
+            for m in range(len(logs)):
+                assert (dv.from_dev(tmps[m] if swapped[m] else bufs[m]) == exps[m]).all(), (rep, m)
+    finally:
+        call("zk_graph_destroy", exec_)

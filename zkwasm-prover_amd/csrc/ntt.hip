@@ -720,21 +720,25 @@ static void fill_job(NttJob &j, const NttSpec &sp, int r, int np, uint32_t logp,
     j.deg = (uint8_t)deg;
 }
 
-// The degrees whose passes of round r go to the matrix cores: 6 to 8, where
-// the launch has at least 2^19 elements (two waves of 256 elements for each
-// SIMD).  Below that a pass is one tile's latency plus the tables, and the
+// The degrees whose passes of round r go to the matrix cores: 6 and 7, and 8
+// in the first round (later its one column per wave would be loaded and stored
+// in runs of 32 bytes: 2^24 elements 880 and 1100 us per pass against 690 with the
+// radix-2 kernel), where the launch has at least 2^19 elements (two waves of
+// 256 elements for each SIMD).  Below that a pass is one tile's latency plus the tables, and the
 // radix-2 kernel with its shorter chains is as fast or faster (one transform,
 // both ways: 2^18 57 us here and 52 there, 2^19 79 and 87, 2^20 114 and 145;
 // eight transforms: 2^15 44 and 44, 2^16 61 and 65, 2^18 187 and 226).
 constexpr uint32_t kMfmaMinElems = 1u << 19;
 constexpr uint32_t kMfmaMinLog = 12;  // the tables of a smaller transform would cost more than its tiles
-static bool mfma_degree(const NttSpec &sp, uint32_t deg) { return sp.log_n >= kMfmaMinLog && deg >= 6 && deg <= 8; }
+static bool mfma_degree(const NttSpec &sp, uint32_t deg, int r) {
+    return sp.log_n >= kMfmaMinLog && deg >= 6 && deg <= (r ? 7 : 8);
+}
 static uint32_t mfma_degrees(const NttSpec *specs, uint32_t count, const uint32_t *degs, const int *np, int r) {
     uint64_t elems[9] = {};
     for (uint32_t m = 0; m < count; m++) {
         if (r >= np[m]) continue;
         const uint32_t deg = degs[(size_t)m * 32 + r];
-        if (mfma_degree(specs[m], deg)) elems[deg] += 1ull << specs[m].log_n;
+        if (mfma_degree(specs[m], deg, r)) elems[deg] += 1ull << specs[m].log_n;
     }
     uint32_t set = 0;
     for (uint32_t d = 6; d <= 8; d++) set |= elems[d] >= kMfmaMinElems ? 1u << d : 0u;
@@ -766,15 +770,14 @@ static hipError_t mfma_round(const NttSpec *specs, uint32_t count, const uint32_
                 return d == 8   ? mfma_launch<4, 4, true>(args, tiles, stream)
                        : d == 7 ? mfma_launch<4, 3, true>(args, tiles, stream)
                                 : mfma_launch<3, 3, true>(args, tiles, stream);
-            return d == 8   ? mfma_launch<4, 4, false>(args, tiles, stream)
-                   : d == 7 ? mfma_launch<4, 3, false>(args, tiles, stream)
-                            : mfma_launch<3, 3, false>(args, tiles, stream);
+            return d == 7 ? mfma_launch<4, 3, false>(args, tiles, stream)
+                          : mfma_launch<3, 3, false>(args, tiles, stream);
         };
         NttPassArgs args;
         memset(&args, 0, sizeof(args));
         uint32_t tiles = 0;
         for (uint32_t m = 0; m < count; m++) {
-            if (r >= np[m] || degs[(size_t)m * 32 + r] != d || !mfma_degree(specs[m], d)) continue;
+            if (r >= np[m] || degs[(size_t)m * 32 + r] != d || !mfma_degree(specs[m], d, r)) continue;
             fill_job(args.job[args.count++], specs[m], r, np[m], logp[m], d, tiles);
             tiles += 1u << (specs[m].log_n - 8);
             if (args.count == kJobsPerLaunch) ZK_CHECK(launch(args, tiles));
@@ -817,7 +820,7 @@ hipError_t ntt_run_batch(const NttSpec *specs, uint32_t count, hipStream_t strea
             const NttSpec &sp = specs[m];
             const uint32_t n = 1u << sp.log_n;
             const uint32_t deg = degs[(size_t)m * 32 + r];
-            if (mfma >> deg & 1 && mfma_degree(sp, deg)) {
+            if (mfma >> deg & 1 && mfma_degree(sp, deg, r)) {
                 logp[m] += deg;
                 continue;
             }
