@@ -660,17 +660,26 @@ __global__ void k_coset_scale(Fr *s, const Fr *__restrict__ cp, uint32_t cn, uin
 
 namespace zk {
 
+// elements a launch of matrix-core passes must have, see mfma_degrees
+constexpr uint32_t kMfmaMinElems = 1u << 19;
+
 // Largest pass degree per transform size; 0 = kMaxDeg.  Set by the
 // autotuner (zk_ntt_set_max_deg), read by every plan, possibly from other
 // threads: atomic (the plan changes only the speed, never the result).
 std::atomic<uint8_t> g_max_deg[31];
 
 // Radix plan: ceil(log_n / max_deg) passes, bits spread evenly (larger first).
+// Where every pass of a large transform would have degree 8 (2^24: 8 8 8) one
+// pass more is faster: all of them have degrees that run on the matrix cores, of
+// degree 8 only the first does (2^24, one transform 1970 us as 8 8 8 and 1789
+// as 6 6 6 6; four 7986 and 6654; with one degree below 8, 2^23 = 8 8 7, 937
+// and 942, four 3451 and 3584).
 int ntt_plan(uint32_t log_n, uint32_t *degs) {
     if (log_n == 0) return 0;
     const uint8_t tuned = log_n < 31 ? g_max_deg[log_n].load(std::memory_order_relaxed) : 0;
     const uint32_t md = tuned ? tuned : kMaxDeg;
     uint32_t passes = (log_n + md - 1) / md;
+    if (!tuned && (1ull << log_n) >= kMfmaMinElems && log_n % kMaxDeg == 0) passes++;
     uint32_t rem = log_n;
     for (uint32_t i = 0; i < passes; i++) {
         uint32_t left = passes - i;
@@ -728,7 +737,6 @@ static void fill_job(NttJob &j, const NttSpec &sp, int r, int np, uint32_t logp,
 // radix-2 kernel with its shorter chains is as fast or faster (one transform,
 // both ways: 2^18 57 us here and 52 there, 2^19 79 and 87, 2^20 114 and 145;
 // eight transforms: 2^15 44 and 44, 2^16 61 and 65, 2^18 187 and 226).
-constexpr uint32_t kMfmaMinElems = 1u << 19;
 constexpr uint32_t kMfmaMinLog = 12;  // the tables of a smaller transform would cost more than its tiles
 static bool mfma_degree(const NttSpec &sp, uint32_t deg, int r) {
     return sp.log_n >= kMfmaMinLog && deg >= 6 && deg <= (r ? 7 : 8);
