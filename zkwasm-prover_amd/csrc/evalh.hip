@@ -13,7 +13,7 @@
 // staged once per workgroup in LDS instead of being re-read per row.
 #include <string.h>
 
-#include "ff29.h"
+#include "evalh_rows.h"
 #include "zkcore.h"
 
 using namespace zk;
@@ -28,62 +28,7 @@ uint32_t grid_for(uint32_t n) {
     return b > 32768 ? 32768 : (b ? b : 1);
 }
 
-__device__ __forceinline__ Fr ld(const Fr *p) { return fe_load<FrParams>(p); }
 __device__ __forceinline__ void st(Fr *p, const Fr &v) { fe_store<FrParams>(p, v); }
-
-// Row arithmetic of the folds in lazy 29-bit limbs.  With 32-bit products
-// they were bound by VALU issue; here a fold t y + a b is one f29_mul2, two
-// products under one reduction, and nothing is reduced below r before the
-// store.  2^22 rows: logup fold 358 -> 291 us, shuffle 360 -> 267, first
-// permutation fold 209 -> 169 (273, 210 and 157 us of traffic), permutation
-// product of four columns 723 -> 660 (18 products a row, still VALU-bound).
-// The term list of k_batch_mul_sum stays in 32-bit products: it is bound by
-// its loads (384 us, 400 with these).
-//
-// An operand of a product enters as it is (lo) or times 2^5 (hi): lo x hi
-// stays in the stored 2^256 domain, hi x hi in the 2^261 domain.  Bounds: a
-// product is below (1 + sum a b / (169 r^2)) r, stored values are below r,
-// every product of lo and hi here below 2 r; one operand of a pair may have limbs up
-// to 2^30.6 (sums without carries).
-__device__ __forceinline__ F29 lo(const Fr &x) { return f29_repack(x.v); }
-__device__ __forceinline__ F29 hi(const Fr &x) { return f29_from32(x); }
-__device__ __forceinline__ F29 mul(const F29 &a, const F29 &b) { return f29_mul<Fr29Mod>(a, b); }
-__device__ __forceinline__ F29 mul2(const F29 &a, const F29 &b, const F29 &c, const F29 &d) {
-    return f29_mul2<Fr29Mod>(a, b, c, d);
-}
-__device__ __forceinline__ F29 add_nc(const F29 &a, const F29 &b) {
-    F29 r;
-#pragma unroll
-    for (int i = 0; i < 9; i++) r.l[i] = a.l[i] + b.l[i];
-    return r;
-}
-// 4 r, every limb but the top raised by 2^29 that is taken from the next: no
-// limb of a difference is negative
-constexpr uint32_t kR4x29[9] = {0x20000004u, 0x3c3eb27du, 0x39709142u, 0x3f4243ccu, 0x36174a0bu,
-                                0x2b6d0301u, 0x229b8503u, 0x397098cfu, 0x00c19138u};
-__device__ __forceinline__ F29 sub_nc(const F29 &a, const F29 &b) {  // a + 4 r - b, b < 3 r
-    F29 r;
-#pragma unroll
-    for (int i = 0; i < 9; i++) r.l[i] = a.l[i] + kR4x29[i] - b.l[i];
-    return r;
-}
-// a + r - b (< 2 r) and r - b
-__device__ __forceinline__ Fr sub_lazy(const Fr &a, const Fr &b) {
-    Fr t;
-    uint32_t c = 0, br = 0;
-#pragma unroll
-    for (int i = 0; i < 8; i++) t.v[i] = add_cc(a.v[i], FrParams::M[i], c);
-#pragma unroll
-    for (int i = 0; i < 8; i++) t.v[i] = sub_bb(t.v[i], b.v[i], br);
-    return t;
-}
-__device__ __forceinline__ Fr neg_lazy(const Fr &b) {
-    Fr t;
-    uint32_t br = 0;
-#pragma unroll
-    for (int i = 0; i < 8; i++) t.v[i] = sub_bb(FrParams::M[i], b.v[i], br);
-    return t;
-}
 
 #define GRID_LOOP(i, n)                                                \
     for (uint32_t i = blockIdx.x * blockDim.x + threadIdx.x; i < (n); \
@@ -180,12 +125,7 @@ __global__ void k_perm_p1(Fr *res, const Fr *__restrict__ first, const Fr *__res
                           uint32_t n) {
     const F29 y = hi(ld(yp));
     const Fr one = fe_one<FrParams>();
-    GRID_LOOP(i, n) {
-        F29 t = mul2(lo(ld(&res[i])), y, lo(sub_lazy(one, ld(&first[i]))), hi(ld(&l0[i])));
-        const Fr ls = ld(&last[i]);
-        t = mul2(t, y, mul(lo(ls), hi(sub_lazy(ls, one))), hi(ld(&l_last[i])));
-        st(&res[i], f29_to_fr(t));
-    }
+    GRID_LOOP(i, n) st(&res[i], perm_p1_row(res, first, last, l0, l_last, i, one, y));
 }
 
 // cuda/bn254.cu:704-739 (also logup_eval_h_z_set)
@@ -196,7 +136,7 @@ __global__ void k_perm_p2(Fr *res, const Fr *const *__restrict__ set, const Fr *
         uint32_t rp = (i + n + (uint32_t)rot) & (n - 1);
         F29 t = lo(ld(&res[i]));
         const F29 l = hi(ld(&l0[i]));
-        for (int j = 1; j < n_set; j++) t = mul2(t, y, lo(sub_lazy(ld(&set[j][i]), ld(&set[j - 1][rp]))), l);
+        for (int j = 1; j < n_set; j++) t = perm_p2_step(t, ld(&set[j][i]), ld(&set[j - 1][rp]), l, y);
         st(&res[i], f29_to_fr(t));
     }
 }
@@ -220,13 +160,7 @@ __global__ void k_logup_eval_h(Fr *res, const Fr *__restrict__ ip, const Fr *__r
     const F29 y = hi(ld(yp));
     GRID_LOOP(i, n) {
         uint32_t rn = (i + (uint32_t)rot) & (n - 1);
-        const Fr z = ld(&zf[i]);
-        F29 t = mul2(lo(ld(&res[i])), y, lo(ld(&l0[i])), hi(z));
-        t = mul2(t, y, lo(ld(&l_last[i])), hi(ld(&zl[i])));
-        const F29 tb = lo(ld(&table[i]));
-        F29 u = add_nc(mul(lo(sub_lazy(ld(&zf[rn]), z)), f29_shl5(tb)), lo(ld(&m[i])));  // < 2.4 r
-        u = mul2(u, hi(ld(&ip[i])), tb, hi(neg_lazy(ld(&ips[i]))));
-        st(&res[i], f29_to_fr(mul2(t, y, u, hi(ld(&l_active[i])))));
+        st(&res[i], logup_row(res, ip, ips, table, m, zf, zl, l0, l_last, l_active, i, rn, y));
     }
 }
 
@@ -236,8 +170,7 @@ __global__ void k_logup_extra(Fr *res, const Fr *__restrict__ ip, const Fr *__re
     const F29 y = hi(ld(yp));
     GRID_LOOP(i, n) {
         uint32_t rn = (i + (uint32_t)rot) & (n - 1);
-        const F29 u = add_nc(mul(lo(sub_lazy(ld(&zp[rn]), ld(&zp[i]))), hi(ld(&ip[i]))), lo(neg_lazy(ld(&ips[i]))));
-        st(&res[i], f29_to_fr(mul2(u, hi(ld(&l_active[i])), lo(ld(&res[i])), y)));
+        st(&res[i], logup_extra_row(res, ip, ips, zp, l_active, i, rn, y));
     }
 }
 
@@ -258,16 +191,6 @@ __global__ void k_inputs_product_sum(Fr *__restrict__ prod, Fr *__restrict__ psu
         }
         st(&psum[i], sum);
     }
-}
-
-// shared tail of the two shuffle kernels (cuda/bn254.cu:990-1013, :1049-1068);
-// lhs, rhs < 2 r
-__device__ __forceinline__ Fr shuffle_fold(const Fr &res, const F29 &lhs, const F29 &rhs, const Fr &z, const Fr &zn,
-                                           const Fr &l0, const Fr &l_last, const Fr &l_active, const F29 &y) {
-    const Fr one = fe_one<FrParams>();
-    F29 t = mul2(lo(res), y, lo(l0), hi(sub_lazy(one, z)));
-    t = mul2(t, y, mul(lo(z), hi(sub_lazy(z, one))), hi(l_last));
-    return f29_to_fr(mul2(t, y, mul2(rhs, hi(zn), lhs, hi(neg_lazy(z))), hi(l_active)));
 }
 
 __global__ void k_shuffle(Fr *res, const Fr *__restrict__ input, const Fr *__restrict__ table, const Fr *__restrict__ zp,
@@ -293,8 +216,8 @@ __global__ void k_shuffle_v2(Fr *res, const Fr *const *__restrict__ inputs, cons
         F29 r = lo(ld(&tables[0][i]) + b0);
         for (int j = 1; j < group_len; j++) {
             const F29 bj = hi(ld(&betas[j]));
-            l = mul(add_nc(hi(ld(&inputs[j][i])), bj), l);  // factors < 64 r
-            r = mul(add_nc(hi(ld(&tables[j][i])), bj), r);
+            l = shuffle_factor(l, ld(&inputs[j][i]), bj);
+            r = shuffle_factor(r, ld(&tables[j][i]), bj);
         }
         st(&res[i], shuffle_fold(ld(&res[i]), l, r, ld(&zp[i]), ld(&zp[rn]), ld(&l0[i]), ld(&l_last[i]),
                                  ld(&l_active[i]), y));
@@ -373,8 +296,9 @@ __global__ void k_lookup_eval_h(Fr *res, const Fr *__restrict__ input, const Fr 
 // same term from field_op / permutation_eval_h_l and one extended NTT per
 // side and column (src/eval_h.rs:700-840); here sigma_c and X stay resident as
 // coset evaluations and one pass reads each operand once.
+// Five waves per SIMD asked for: 97 registers without it, one too many.
 constexpr int kMaxPermCols = 16;
-__global__ void k_perm_set_eval(Fr *h, const Fr *__restrict__ z, const Fr *const *__restrict__ v,
+__global__ __launch_bounds__(kThreads, 5) void k_perm_set_eval(Fr *h, const Fr *__restrict__ z, const Fr *const *__restrict__ v,
                                 const Fr *const *__restrict__ sig, int nc, const Fr *__restrict__ beta,
                                 const Fr *__restrict__ gamma, const Fr *__restrict__ bd, const Fr *__restrict__ X,
                                 const Fr *__restrict__ l_active, const Fr *__restrict__ yp, int rot, uint32_t n) {
@@ -393,13 +317,11 @@ __global__ void k_perm_set_eval(Fr *h, const Fr *__restrict__ z, const Fr *const
         const F29 x = hi(ld(&X[i]));
         F29 l = lo(ld(&z[rn])), r = lo(ld(&z[i]));
         for (int c = 0; c < nc; c++) {
-            // factors in the 2^261 domain: 32 (v + gamma) < 32 r and a product of
-            // two hi operands < 7.1 r; l and r stay below 1.4 r
             const F29 vg = hi(ld(&sv[c][i]) + g);
-            l = mul(add_nc(vg, mul(b, hi(ld(&ss[c][i])))), l);
-            r = mul(add_nc(vg, mul(sb[c], x)), r);
+            l = perm_set_factor(l, vg, b, hi(ld(&ss[c][i])));
+            r = perm_set_factor(r, vg, sb[c], x);
         }
-        st(&h[i], f29_to_fr(mul2(sub_nc(l, r), hi(ld(&l_active[i])), lo(ld(&h[i])), y)));
+        st(&h[i], perm_set_fold(ld(&h[i]), l, r, ld(&l_active[i]), y));
     }
 }
 
@@ -422,11 +344,9 @@ __global__ __launch_bounds__(kThreads) void k_gate_eval(Fr *__restrict__ h, cons
     const F29 y = hi(ld(yp));
     GRID_LOOP(i, n) {
         const F29 a = hi(ld(&g.a[i]));
-        // acc < 3.3 r
-        F29 acc = add_nc(mul(lo(ld(&g.b[i])), a), lo(sub_lazy(ld(&g.c[i]), ld(&g.d[i]))));
-        for (int k = 0; k < g.ng; k++)
-            acc = add_nc(mul2(acc, y, lo(ld(&g.f[k][i])), a), lo(neg_lazy(ld(&g.e[k][i]))));
-        st(&h[i], f29_to_fr(mul(acc, hi(ld(&g.q[i])))));
+        F29 acc = gate_first(a, ld(&g.b[i]), ld(&g.c[i]), ld(&g.d[i]));
+        for (int k = 0; k < g.ng; k++) acc = gate_step(acc, a, ld(&g.f[k][i]), ld(&g.e[k][i]), y);
+        st(&h[i], gate_last(acc, ld(&g.q[i])));
     }
 }
 

@@ -183,20 +183,31 @@ __device__ __forceinline__ Fe<P> fe_mul_cios(const Fe<P> &a, const Fe<P> &b) {
 // (acc:t) += x * y as a 96-bit accumulator: acc is a 64-bit VGPR pair and t
 // the third word.  v_mad_u64_u32 writes its 64-bit carry-out to an SGPR lane
 // mask, which v_addc_co_u32 folds into t (two VALU instructions, no moves).
+// (Host builds of this header take the same sum in C.)
 __device__ __forceinline__ void mac96(uint64_t &acc, uint32_t &t, uint32_t x, uint32_t y) {
+#if defined(__HIP_DEVICE_COMPILE__)
     uint64_t cc;
     asm("v_mad_u64_u32 %0, %1, %3, %4, %0\n\t"
         "v_addc_co_u32_e64 %2, %1, %2, 0, %1"
         : "+v"(acc), "=&s"(cc), "+v"(t)
         : "v"(x), "v"(y));
+#else
+    const uint64_t p = (uint64_t)x * y;
+    acc += p;
+    t += acc < p;
+#endif
 }
 // same with an SGPR second operand (the modulus words are uniform constants)
 __device__ __forceinline__ void mac96s(uint64_t &acc, uint32_t &t, uint32_t x, uint32_t y) {
+#if defined(__HIP_DEVICE_COMPILE__)
     uint64_t cc;
     asm("v_mad_u64_u32 %0, %1, %3, %4, %0\n\t"
         "v_addc_co_u32_e64 %2, %1, %2, 0, %1"
         : "+v"(acc), "=&s"(cc), "+v"(t)
         : "v"(x), "s"(y));
+#else
+    mac96(acc, t, x, y);
+#endif
 }
 
 // Montgomery multiplication by product scanning with the reduction folded
