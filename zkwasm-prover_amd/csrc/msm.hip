@@ -89,17 +89,16 @@ constexpr uint32_t kMagic = 0x4d534d32u;  // "MSM2": masked sums present in the 
 //   then            S[w]: W Jacobian window sums (device tail only)
 constexpr size_t kSliceQ = 128;
 // bytes of a slice the layout above can use: W * (nbits + 1) masked sums and
-// W window sums stay below 34300 B for every window 2 <= c <= 17
-constexpr size_t kSliceReserve = 36 * 1024;
+// W window sums take at most 33568 B over the windows 2 <= c <= 17 (at c = 14)
+constexpr size_t kSliceReserve = 33 * 1024;
 
 // Arrays placed into caller memory, in two lifetimes: phase 1 (the sort) and
-// phase 2 (accumulation and reduction).  offsets, entries and the long-bucket
-// list live across both;
+// phase 2 (accumulation and reduction).  offsets and entries live across both;
 // the phase-1 temporaries (tmp, hist, starts, scan) are free again in phase 2.
 enum MsmArr {
-    A_ITEMS, A_SLOTS, A_OFFSETS, A_ENTRIES, A_LONG,                // both phases
+    A_ITEMS, A_SLOTS, A_OFFSETS, A_ENTRIES,                        // both phases
     A_TMP, A_HIST, A_STARTS, A_SCAN,                               // phase 1
-    A_BUCKETS, A_PHEAD, A_PTAIL, A_TB, A_PART,                     // phase 2
+    A_BUCKETS, A_PHEAD, A_PTAIL, A_TB, A_LONG, A_PART,             // phase 2
     A_COUNT
 };
 constexpr int kFirstPhase2 = A_BUCKETS;
@@ -175,7 +174,8 @@ inline uint32_t plain_hi_bits(uint32_t c) {
     return hi;
 }
 
-constexpr uint32_t kBitParts = 5;   // k_msm_bits: T and four masked sums per 16 buckets
+constexpr uint32_t kBitSpan = 16;   // k_msm_bits: buckets of a wave, whose first five places take T and four masked sums
+constexpr uint32_t kBitPart = 8;    // the place of a span that k_msm_bit_sums may write a part to
 constexpr uint32_t kFoldParts = 8;  // k_msm_reduce_fold: T, six masked sums and A per 64 segments
 
 // workgroups per output of k_msm_bit_sums (B <= 2^17: at most 16, see kQuadBuckets)
@@ -264,10 +264,8 @@ MsmPlan make_plan(const uint32_t *ns, uint32_t count, uint32_t c, bool fixed = f
     p.size[A_BUCKETS] = (size_t)p.NB * sizeof(X29S);
     p.size[A_PHEAD] = (size_t)p.chunks * sizeof(X29S);
     p.size[A_PTAIL] = (size_t)p.chunks * sizeof(X29S);
-    const uint32_t hw = (p.B + 15) / 16;
     p.size[A_TB] = (size_t)p.chunks * 4;
-    p.size[A_PART] = p.quads ? (size_t)count * p.W * (hw * kBitParts + (p.nbits + 1) * bit_sum_parts(hw)) * sizeof(X29S)
-                             : (size_t)count * p.W * (p.T1 / 64) * kFoldParts * sizeof(X29S);
+    p.size[A_PART] = p.quads ? 0 : (size_t)count * p.W * (p.T1 / 64) * kFoldParts * sizeof(X29S);
     // [count, (bucket, first chunk, last chunk) per bucket spanning > kWalk chunks]
     p.size[A_LONG] = (size_t)(1 + 3 * (p.chunks / kWalk + 1)) * 4;
     return p;
@@ -400,13 +398,11 @@ struct ItemPack {
     uint32_t first, k;
 };
 __global__ __launch_bounds__(256) void k_msm_put_items(ItemPack pk, MsmItemDev *__restrict__ items,
-                                                       uint8_t **__restrict__ slots, uint32_t *__restrict__ long_count,
-                                                       uint32_t *__restrict__ wcount, uint32_t nw) {
+                                                       uint8_t **__restrict__ slots, uint32_t *__restrict__ wcount,
+                                                       uint32_t nw) {
     uint32_t j = threadIdx.x;
-    if (pk.first == 0) {
-        if (j == 0) *long_count = 0;
+    if (pk.first == 0)
         for (uint32_t k = j; k < nw; k += blockDim.x) wcount[k] = 0;
-    }
     if (j >= pk.k) return;
     items[pk.first + j] = pk.it[j];
     slots[pk.first + j] = pk.slot[j];
@@ -904,9 +900,11 @@ __global__ __launch_bounds__(256) void k_msm_accumulate(const uint32_t *__restri
                                                         const MsmItemDev *__restrict__ items,
                                                         X29S *__restrict__ buckets, X29S *__restrict__ phead,
                                                         X29S *__restrict__ ptail, uint32_t *__restrict__ tb,
-                                                        uint64_t nchunks, uint32_t cmin) {
+                                                        uint32_t *__restrict__ long_count, uint64_t nchunks,
+                                                        uint32_t cmin) {
     uint64_t t = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (t >= nchunks) return;
+    if (t == 0) *long_count = 0;  // of the fixup's list, which follows
     const uint32_t total = off[NB], chunk = chunk_of(total, cmin);
     const uint64_t s64 = t * chunk;
     uint32_t tail_bucket = kNone;
@@ -1212,20 +1210,22 @@ __global__ __launch_bounds__(64) void k_msm_fold_sums(const X29S *__restrict__ p
 }
 
 // Bucket reduction by quads of lanes, one wave per 16 consecutive buckets b =
-// 16 h + i of an item window g (padded with empty ones when B < 16): S_w =
+// 16 h + i of an item window g (fewer when B < 16): S_w =
 // sum_b (b + 1) B_b = T + sum_k 2^k Q_k with T the sum of all buckets and Q_k
 // that of the buckets with bit k of b set.  Four butterfly steps over the
 // quads: at step k a quad with bit k of i clear adds its partner's value;
-// afterwards quad 0 holds the wave's T and quad 2^k its Q_k (k < 4).  They go
-// to part[(g * hw + h) * kBitParts + {0, 1 + k}] for k_msm_bit_sums.
-__global__ __launch_bounds__(256) void k_msm_bits(const X29S *__restrict__ buckets, const uint32_t *__restrict__ off,
-                                                  uint32_t B, uint32_t hw, uint32_t nwaves,
-                                                  X29S *__restrict__ part) {
+// afterwards quad 0 holds the wave's T and quad 2^k its Q_k (2^k < B, k < 4).
+// They go to places 0 and 1 + k of the wave's own buckets, which it has read
+// (no other wave does), for k_msm_bit_sums: 1 + log2 B places of B < 16
+// buckets, five of 16.  An array of their own made the smallest scratch of a
+// small MSM up to twice what callers had kept for it.
+__global__ __launch_bounds__(256) void k_msm_bits(X29S *buckets, const uint32_t *__restrict__ off, uint32_t B,
+                                                  uint32_t hw, uint32_t nwaves) {
     const uint32_t gh = (blockIdx.x * blockDim.x + threadIdx.x) >> 6;
     if (gh >= nwaves) return;
     const uint32_t g = gh / hw, h = gh % hw;
     const uint32_t i = (threadIdx.x & 63) >> 2, q = threadIdx.x & 3;
-    const uint32_t b = h * 16 + i, idx = g * B + b;
+    const uint32_t b = h * kBitSpan + i, idx = g * B + b;
     Q29 p{};
     bool pe = true;
     if (b < B && off[idx + 1] != off[idx]) p = q29_load(&buckets[idx], pe, q);
@@ -1235,10 +1235,10 @@ __global__ __launch_bounds__(256) void k_msm_bits(const X29S *__restrict__ bucke
         const Q29 o = q29_shfl_xor(p, pe, oe, 4 << k);
         if (!((i >> k) & 1u)) q29_add(p, pe, o, oe, q);
     }
-    X29S *dst = part + (size_t)gh * kBitParts;
+    X29S *dst = buckets + (size_t)g * B + h * kBitSpan;
     if (i == 0)
         q29_store(&dst[0], p, pe, q);
-    else if ((i & (i - 1)) == 0)
+    else if ((i & (i - 1)) == 0 && i < B)
         q29_store(&dst[1 + __builtin_ctz(i)], p, pe, q);
 }
 
@@ -1257,25 +1257,24 @@ __device__ __forceinline__ void q29_slot_store(uint8_t *const *slots, uint32_t g
 // the partials of k_msm_bits.  o < nbits: Q_k for k = o + 1 (k < 4: the sum of
 // the waves' Q_k; else the sum of T_h over the waves with bit k - 4 of h set);
 // o = nbits: T + Q_0.  With several parts (wide windows: up to 256 waves
-// each), part z's sum goes to qpart[(g * (nbits + 1) + o) * parts + z] for
-// k_msm_bit_merge.
-__global__ __launch_bounds__(256) void k_msm_bit_sums(const X29S *__restrict__ part, uint32_t hw, uint32_t c,
-                                                      uint32_t W, uint8_t *const *__restrict__ slots,
-                                                      X29S *__restrict__ qpart) {
+// each), part z's sum goes to place kBitPart of span o * parts + z for
+// k_msm_bit_merge (there are hw >= (nbits + 1) * parts spans).
+__global__ __launch_bounds__(256) void k_msm_bit_sums(X29S *buckets, uint32_t hw, uint32_t c, uint32_t W,
+                                                      uint8_t *const *__restrict__ slots) {
     __shared__ X29S sh[4];
     const uint32_t o = blockIdx.x, g = blockIdx.y, nbits = c - 2, k = o + 1, parts = gridDim.z;
     const uint32_t q = threadIdx.x & 3, span = (hw + parts - 1) / parts, h0 = blockIdx.z * span;
     const uint32_t h1 = h0 + span < hw ? h0 + span : hw;
-    const X29S *src = part + (size_t)g * hw * kBitParts;
+    X29S *src = buckets + ((size_t)g << (c - 1));
     Q29 acc{};
     bool ae = true, ve;
     for (uint32_t h = h0 + (threadIdx.x >> 2); h < h1; h += blockDim.x >> 2) {
         if (o == nbits || k < 4 || ((h >> (k - 4)) & 1u)) {
-            const Q29 v = q29_load(&src[h * kBitParts + (o < nbits && k < 4 ? 1 + k : 0)], ve, q);
+            const Q29 v = q29_load(&src[h * kBitSpan + (o < nbits && k < 4 ? 1 + k : 0)], ve, q);
             q29_add(acc, ae, v, ve, q);
         }
         if (o == nbits) {
-            const Q29 v = q29_load(&src[h * kBitParts + 1], ve, q);
+            const Q29 v = q29_load(&src[h * kBitSpan + 1], ve, q);
             q29_add(acc, ae, v, ve, q);
         }
     }
@@ -1284,17 +1283,17 @@ __global__ __launch_bounds__(256) void k_msm_bit_sums(const X29S *__restrict__ p
         if (parts == 1)
             q29_slot_store(slots, g, c, W, o, acc, ae, q);
         else
-            q29_store(&qpart[((size_t)g * (nbits + 1) + o) * parts + blockIdx.z], acc, ae, q);
+            q29_store(&src[(o * parts + blockIdx.z) * kBitSpan + kBitPart], acc, ae, q);
     }
 }
 
 // grid (nbits + 1, gw), one wave: adds the parts (at most 16) of each sum
-__global__ __launch_bounds__(64) void k_msm_bit_merge(const X29S *__restrict__ qpart, uint32_t parts, uint32_t c,
+__global__ __launch_bounds__(64) void k_msm_bit_merge(const X29S *__restrict__ buckets, uint32_t parts, uint32_t c,
                                                       uint32_t W, uint8_t *const *__restrict__ slots) {
     const uint32_t o = blockIdx.x, g = blockIdx.y, z = threadIdx.x >> 2, q = threadIdx.x & 3;
     Q29 p{};
     bool pe = true;
-    if (z < parts) p = q29_load(&qpart[((size_t)g * (c - 1) + o) * parts + z], pe, q);
+    if (z < parts) p = q29_load(&buckets[((size_t)g << (c - 1)) + (o * parts + z) * kBitSpan + kBitPart], pe, q);
     q29_wave_sum(p, pe, q);
     if (threadIdx.x < 4) q29_slot_store(slots, g, c, W, o, p, pe, q);
 }
@@ -1616,8 +1615,7 @@ hipError_t msm_run(const MsmJob *jobs, uint32_t count, size_t slice_bytes, uint3
                 tile += it.ntiles;
                 dig += (uint64_t)jb.n * p.Wd;
             }
-            k_msm_put_items<<<1, 256, 0, stream>>>(pk, items, slots, longs, hist,
-                                                   p.window_sort ? (uint32_t)p.nhist : 0u);
+            k_msm_put_items<<<1, 256, 0, stream>>>(pk, items, slots, hist, p.window_sort ? (uint32_t)p.nhist : 0u);
             ZK_CHECK(hipGetLastError());
         }
     }
@@ -1674,7 +1672,7 @@ hipError_t msm_run(const MsmJob *jobs, uint32_t count, size_t slice_bytes, uint3
     ZK_CHECK(prof_mark(prof, PH_ACCUMULATE, stream));
     const uint32_t cblocks = (uint32_t)((p.chunks + 255) / 256);
     k_msm_accumulate<<<cblocks, 256, 0, stream>>>(entries, offsets, (uint32_t)p.NB, p.W * p.B, items, buckets,
-                                                  phead, ptail, tb, p.chunks, p.chunk);
+                                                  phead, ptail, tb, longs, p.chunks, p.chunk);
     ZK_CHECK(hipGetLastError());
     ZK_CHECK(prof_mark(prof, PH_FIXUP, stream));
     const uint64_t fquads = p.NB > p.chunks ? p.NB : p.chunks;
@@ -1690,18 +1688,16 @@ hipError_t msm_run(const MsmJob *jobs, uint32_t count, size_t slice_bytes, uint3
     ZK_CHECK(prof_mark(prof, PH_REDUCE, stream));
     const uint32_t gw = count * p.W;
     if (p.quads) {
-        const uint32_t hw = (p.B + 15) / 16, nwaves = gw * hw;
-        k_msm_bits<<<(nwaves + 3) / 4, 256, 0, stream>>>(buckets, offsets, p.B, hw, nwaves, part);
+        const uint32_t hw = (p.B + kBitSpan - 1) / kBitSpan, nwaves = gw * hw;
+        k_msm_bits<<<(nwaves + 3) / 4, 256, 0, stream>>>(buckets, offsets, p.B, hw, nwaves);
         ZK_CHECK(hipGetLastError());
         // at most 256 waves' partials per workgroup: a chain of 4 to 8
         // additions before its tree
         const uint32_t parts = bit_sum_parts(hw);
-        X29S *qpart = part + (size_t)nwaves * kBitParts;
-        k_msm_bit_sums<<<dim3(p.nbits + 1, gw, parts), hw > 16 ? 256 : 64, 0, stream>>>(part, hw, c, p.W, slots,
-                                                                                     qpart);
+        k_msm_bit_sums<<<dim3(p.nbits + 1, gw, parts), hw > 16 ? 256 : 64, 0, stream>>>(buckets, hw, c, p.W, slots);
         ZK_CHECK(hipGetLastError());
         if (parts > 1) {
-            k_msm_bit_merge<<<dim3(p.nbits + 1, gw), 64, 0, stream>>>(qpart, parts, c, p.W, slots);
+            k_msm_bit_merge<<<dim3(p.nbits + 1, gw), 64, 0, stream>>>(buckets, parts, c, p.W, slots);
             ZK_CHECK(hipGetLastError());
         }
     } else {
