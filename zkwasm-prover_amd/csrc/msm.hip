@@ -198,8 +198,10 @@ inline uint32_t min_chunk(uint64_t max_entries) {
 }
 
 // chunk: smallest chunk of the accumulation (the partial sums' arrays are
-// sized for it), 0 = what the pass would like
-MsmPlan make_plan(const uint32_t *ns, uint32_t count, uint32_t c, bool fixed = false, uint32_t chunk = 0) {
+// sized for it), 0 = what the pass would like; small_tiles = false: large sort
+// tiles, whose histogram is a quarter
+MsmPlan make_plan(const uint32_t *ns, uint32_t count, uint32_t c, bool fixed = false, uint32_t chunk = 0,
+                  bool small_tiles = true) {
     MsmPlan p;
     memset(&p, 0, sizeof(p));
     p.count = count;
@@ -215,7 +217,7 @@ MsmPlan make_plan(const uint32_t *ns, uint32_t count, uint32_t c, bool fixed = f
         p.ntiles += (ns[m] + kSortTile - 1) / kSortTile;
     }
     p.tile = kSortTile;
-    if (p.ntiles < kFewTiles) {
+    if (small_tiles && p.ntiles < kFewTiles) {
         p.tile = kSmallTile;
         p.ntiles = 0;
         for (uint32_t m = 0; m < count; m++) p.ntiles += (ns[m] + p.tile - 1) / p.tile;
@@ -1520,18 +1522,26 @@ bool choose_plan(const uint32_t *ns, uint32_t count, size_t slice_bytes, uint32_
         for (uint32_t cc = c0 + 1; cc <= 17; cc++) order[norder++] = cc;
         for (uint32_t cc = c0 - 1; cc >= 2; cc--) order[norder++] = cc;
     }
-    for (int k = 0; k < norder; k++) {
-        // the chunk the pass would like first, larger ones (fewer partial
-        // sums) while they do not fit
+    // order[k] with the chunk the pass would like first, then larger ones
+    // (fewer partial sums) while they do not fit
+    auto fits = [&](int k, bool small_tiles) {
         for (uint32_t ch = 0;; ch = p.chunk + p.chunk / 2 < kChunk ? p.chunk + p.chunk / 2 : kChunk) {
-            p = make_plan(ns, count, order[k], fixed, ch);
+            p = make_plan(ns, count, order[k], fixed, ch, small_tiles);
             // entry positions are u32 and the masked-sum grid's y is < 2^16
             if (p.max_entries < 0x80000000ull && (uint64_t)count * p.W < 65536 &&
                 slice_bytes_needed(p.W, p.nbits) <= slice_bytes && place(p, regions, region_bytes, nreg))
                 return true;
-            if (p.chunk >= kChunk) break;
+            if (p.chunk >= kChunk) return false;
         }
-    }
+    };
+    // The wanted window is not given up for small sort tiles, whose histogram
+    // is four times the large ones' (the drop-in's buffers of 241001 points: 840
+    // us at c = 15 with large tiles, 1285 at c = 14 with small ones); another
+    // window is taken with large tiles only when none fits with small ones.
+    if (fits(0, true) || fits(0, false)) return true;
+    for (bool small_tiles : {true, false})
+        for (int k = 1; k < norder; k++)
+            if (fits(k, small_tiles)) return true;
     return false;
 }
 
