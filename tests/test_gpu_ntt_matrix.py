@@ -1,7 +1,8 @@
 """NTT passes on the matrix cores (degrees 6 to 8, launches of at least 2^19
 elements) against the CPU oracle, bit for bit: the degrees in first,
-middle and last passes (degree 8: first only), batches just below and at the threshold, extreme
-inputs (the byte columns' bounds), iNTT scaling, coset extensions and capture."""
+middle and last passes (degree 8: first only), batches just below and at the threshold (which counts
+the transforms of one launch, at most 48, of 2^15 elements or more), workgroups
+with a part of their tiles, extreme inputs (the byte columns' bounds), iNTT scaling, coset extensions and capture."""
 import ctypes
 
 import numpy as np
@@ -45,9 +46,11 @@ def test_single_transform(gpu, zo, log_n, kind, inverse):
 
 
 # 2^16 = 8 8 at the threshold, one transform short of it, and with others
-# beside it; 2^15 = 8 7; 2^12 = 6 6 over several launches
+# beside it; 2^15 = 8 7, in one launch and with one transform in a second, which
+# stays below the threshold; 2^12 = 6 6, radix-2 passes in several launches;
+# transforms whose tiles don't divide evenly among their workgroups
 @pytest.mark.parametrize("logs", [[16] * 8, [16] * 7 + [12, 14], [16] * 8 + [15, 12, 3], [15] * 16, [12] * 128,
-                                  [18, 17, 18, 13]])
+                                  [18, 17, 18, 13], [15] * 49, [18] * 3, [17, 15, 19, 16, 15, 15]])
 def test_batch(gpu, zo, logs):
     specs, exps = [], []
     for m, k in enumerate(logs):
@@ -63,7 +66,8 @@ def test_batch(gpu, zo, logs):
     assert [m for m in range(len(logs)) if not (got[m] == exps[m]).all()] == []
 
 
-@pytest.mark.parametrize("shapes", [[(18, 1)], [(17, 2), (16, 3)], [(12, 4)] * 8, [(19, 3)]])
+@pytest.mark.parametrize("shapes", [[(18, 1)], [(17, 2), (16, 3)], [(12, 4)] * 8, [(19, 3)],
+                                    [(16, 2)] * 3])
 def test_coset_extension(gpu, zo, shapes):
     from zkprover import device as dv
     from zkprover._lib import lib

@@ -430,10 +430,11 @@ __global__ __launch_bounds__(kThreads) void k_ntt_pass(const NttPassArgs a) {
 
 // A pass of radix 2^(LA + LB) on the matrix cores (ntt_mfma.h).  A wave's
 // tile is 256 elements, whole columns (1, 2 or 4), so its exchange needs no
-// barrier.  Persistent, one workgroup of 16 waves per CU: a workgroup takes a
-// contiguous range of the launch's tiles, rebuilds the matrix and the twiddles
-// in LDS where the transform changes and deals the tiles to its waves one by
-// one.  Job block0 counts tiles.
+// barrier.  Persistent, one workgroup of 16 waves per CU: it builds the matrix
+// and the twiddles of one transform in LDS and deals up to `tiles` of its tiles
+// to its waves one by one.  Ranges that crossed from one transform to the next
+// built the tables twice, with the waves waiting in between (three transforms
+// of 2^18, both ways: 104 and 87 us; 24 of 2^14 to 2^20 602 and 555).
 //
 // Bound by VALU issue (about 800 instructions per element of a 2^7 pass with
 // inter-pass twiddles, two 29-bit products of 260 among them; the radix-2
@@ -443,8 +444,8 @@ __global__ __launch_bounds__(kThreads) void k_ntt_pass(const NttPassArgs a) {
 // elements per wave (two waves per SIMD: 140 and 220 us), 2048-element tiles
 // per workgroup with barriers in the exchange (batches 17% slower: the older
 // of two workgroups ran ahead and left the CU half empty).  Registers: 128
-// (four waves per SIMD), which the phases' separate lane values and the
-// scheduling barriers below keep from spilling.
+// (four waves per SIMD), for which the phases have separate lane values and the
+// scheduling barriers below stand; the <4, 4> pass still spills 8 B per lane.
 template <int LA, int LB, bool FIRST>
 __global__ __launch_bounds__(kMfmaThreads) void k_ntt_mfma(const NttPassArgs a, uint32_t tiles) {
     __shared__ __attribute__((aligned(16))) uint8_t mlds[MfmaLds::bytes(LA, LB)];
@@ -455,168 +456,164 @@ __global__ __launch_bounds__(kMfmaThreads) void k_ntt_mfma(const NttPassArgs a, 
     uint32_t *tw = reinterpret_cast<uint32_t *>(mlds + MfmaLds::kMat);
     const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     uint8_t *xch = mlds + MfmaLds::kMat + MfmaLds::twiddles(deg) + wave * MfmaLds::exchange(LA, LB);
-    const uint32_t t1 = (uint32_t)((uint64_t)tiles * (blockIdx.x + 1) / gridDim.x);
     uint32_t q = 0;
-    for (uint32_t t0 = (uint32_t)((uint64_t)tiles * blockIdx.x / gridDim.x), end; t0 < t1; t0 = end) {
-        while (q + 1 < a.count && a.job[q + 1].block0 <= t0) q++;
-        end = q + 1 < a.count && a.job[q + 1].block0 < t1 ? a.job[q + 1].block0 : t1;
-        const NttJob &job = a.job[q];
-        const Fr *__restrict__ omegas = job.omegas;
-        const uint32_t log_n = job.log_n, log_p = job.log_p, log_t = log_n - deg;
-        {
-            uint32_t tid = threadIdx.x;
-            asm volatile("" : "+v"(tid));  // not hoisted out of the loop
-            __syncthreads();               // every wave is done with the previous tables
-            if (tid == 0) next_tile = t0;
-            // matrix: powers of w_16 = omegas[n / 16]
-            if (tid < 512)
-                mfma_matrix_entry(mat, tid >> 5, tid & 31, fe_load<FrParams>(&omegas[(size_t)(tid >> 5) << (log_n - 4)]));
-            // twiddles w_D^e (n^-1), reduced, in the 2^261 domain, by the other half
-            if (tid >= 512 && tid < 512 + D) {
-                const uint32_t e = tid - 512;
-                Fr w = fe_load<FrParams>(&omegas[(size_t)e << log_t]);
-                if (job.n_inv) w = fr_mul_w29(w, f29_from32(fe_load<FrParams>(job.n_inv)));
-                for (int k = 0; k < 5; k++) w = w + w;
-                const F29 f = f29_repack(w.v);
+    while (q + 1 < a.count && a.job[q + 1].block0 <= blockIdx.x) q++;
+    const NttJob &job = a.job[q];
+    const uint32_t t0 = (blockIdx.x - job.block0) * tiles;
+    const uint32_t log_n = job.log_n, log_p = job.log_p, log_t = log_n - deg;
+    const uint32_t all = 1u << (log_n - 8), end = all - t0 < tiles ? all : t0 + tiles;
+    const Fr *__restrict__ omegas = job.omegas;
+    {
+        const uint32_t tid = threadIdx.x;
+        if (tid == 0) next_tile = t0;
+        // matrix: powers of w_16 = omegas[n / 16]
+        if (tid < 512)
+            mfma_matrix_entry(mat, tid >> 5, tid & 31, fe_load<FrParams>(&omegas[(size_t)(tid >> 5) << (log_n - 4)]));
+        // twiddles w_D^e (n^-1), reduced, in the 2^261 domain, by the other half
+        if (tid >= 512 && tid < 512 + D) {
+            const uint32_t e = tid - 512;
+            Fr w = fe_load<FrParams>(&omegas[(size_t)e << log_t]);
+            if (job.n_inv) w = fr_mul_w29(w, f29_from32(fe_load<FrParams>(job.n_inv)));
+            for (int k = 0; k < 5; k++) w = w + w;
+            const F29 f = f29_repack(w.v);
 #pragma clang loop unroll(full)
-                for (int i = 0; i < 9; i++) tw[e * kMfmaTwWords + i] = f.l[i];
-            }
-            __syncthreads();
+            for (int i = 0; i < 9; i++) tw[e * kMfmaTwWords + i] = f.l[i];
         }
-        const Fr *__restrict__ x = job.x;
-        Fr *__restrict__ y = job.y;
-        const uint32_t nz = job.nz, cn = job.cn, p = 1u << log_p;
-        // column and k1 of DFT d after the exchange: the first pass stores runs
-        // of k1, later ones runs of columns
-        auto col_b = [&](uint32_t d) { return FIRST ? d >> LA : d & (kCols - 1); };
-        auto k1_b = [&](uint32_t d) { return FIRST ? d & (SA - 1) : d >> kLogCols; };
-        // the lane, opaque to the optimiser: what follows from it is computed
-        // anew in each phase instead of being kept in registers (it spilled)
-        auto lane_now = [&]() {
-            uint32_t l = threadIdx.x & 63;
-            asm volatile("" : "+v"(l));
-            return l;
+        __syncthreads();
+    }
+    const Fr *__restrict__ x = job.x;
+    Fr *__restrict__ y = job.y;
+    const uint32_t nz = job.nz, cn = job.cn, p = 1u << log_p;
+    // column and k1 of DFT d after the exchange: the first pass stores runs
+    // of k1, later ones runs of columns
+    auto col_b = [&](uint32_t d) { return FIRST ? d >> LA : d & (kCols - 1); };
+    auto k1_b = [&](uint32_t d) { return FIRST ? d & (SA - 1) : d >> kLogCols; };
+    // the lane, opaque to the optimiser: what follows from it is computed
+    // anew in each phase instead of being kept in registers (it spilled)
+    auto lane_now = [&]() {
+        uint32_t l = threadIdx.x & 63;
+        asm volatile("" : "+v"(l));
+        return l;
+    };
+    // a wave takes the next tile when it is done with one: of two workgroups
+    // with a fixed share each, the older one won every issue slot, ended
+    // early and left the CU half empty
+    for (;;) {
+        uint32_t tile = 0;
+        if ((threadIdx.x & 63) == 0) tile = atomicAdd(&next_tile, 1u);
+        tile = __builtin_amdgcn_readfirstlane(tile);
+        if (tile >= end) break;
+        const uint32_t index0 = tile * kCols;
+        uint32_t v[4][8];
+        F29 w[4];
+        auto twiddle = [&](int s) {
+            __builtin_amdgcn_sched_barrier(0);
+            f29_unpack(f29_mul<Fr29Mod>(f29_repack(v[s]), w[s]), v[s]);
+            __builtin_amdgcn_sched_barrier(0);
         };
-        // a wave takes the next tile when it is done with one: of two workgroups
-        // with a fixed share each, the older one won every issue slot, ended
-        // early and left the CU half empty
-        for (;;) {
-            uint32_t tile = 0;
-            if ((threadIdx.x & 63) == 0) tile = atomicAdd(&next_tile, 1u);
-            tile = __builtin_amdgcn_readfirstlane(tile);
-            if (tile >= end) break;
-            const uint32_t index0 = (tile - job.block0) * kCols;
-            uint32_t v[4][8];
-            F29 w[4];
-            auto twiddle = [&](int s) {
-                __builtin_amdgcn_sched_barrier(0);
-                f29_unpack(f29_mul<Fr29Mod>(f29_repack(v[s]), w[s]), v[s]);
-                __builtin_amdgcn_sched_barrier(0);
-            };
-            {
-                // load, columns from lane to lane; the coset scale or the inter-pass twiddle
-                const uint32_t lane = lane_now(), n = lane & 15, h = lane >> 4;
-                uint32_t pos[4];
-                Fr o[4];
-#pragma clang loop unroll(full)
-                for (int s = 0; s < 4; s++) {
-                    const uint32_t d = mfma_dft_index<LA>(s, n), i = mfma_in<LA>(s, h) * SB + (d >> kLogCols);
-                    const uint32_t c = index0 + (d & (kCols - 1));
-                    pos[s] = c + (i << log_t);
-                    const bool in = !FIRST || !nz || pos[s] < nz;
-                    const Fr e = fe_load<FrParams>(&x[in ? pos[s] : 0]);
-#pragma clang loop unroll(full)
-                    for (int k = 0; k < 8; k++) v[s][k] = e.v[k];
-                    if constexpr (!FIRST) o[s] = fe_load<FrParams>(&omegas[((c & (p - 1)) * i) << (log_t - log_p)]);
-                }
-                if constexpr (!FIRST) {
-#pragma clang loop unroll(full)
-                    for (int s = 0; s < 4; s++) {
-                        w[s] = f29_from32(o[s]);
-                        twiddle(s);
-                    }
-                } else if (nz) {
-#pragma clang loop unroll(full)
-                    for (int s = 0; s < 4; s++) {
-#pragma clang loop unroll(full)
-                        for (int k = 0; k < 8; k++) v[s][k] = pos[s] < nz ? v[s][k] : 0u;
-                    }
-                    if (cn > 1) {
-                        uint32_t r[4];
-#pragma clang loop unroll(full)
-                        for (int s = 0; s < 4; s++) {
-                            r[s] = pos[s] % cn;
-                            o[s] = fe_load<FrParams>(&job.coset[r[s] ? r[s] - 1 : 0]);
-                        }
-#pragma clang loop unroll(full)
-                        for (int s = 0; s < 4; s++) {
-                            if (((mfma_in<LA>(s, 0) * SB) << log_t) >= nz) continue;  // all zero
-                            uint32_t u[8];
-#pragma clang loop unroll(full)
-                            for (int k = 0; k < 8; k++) u[k] = v[s][k];
-                            w[s] = f29_from32(o[s]);
-                            twiddle(s);
-#pragma clang loop unroll(full)
-                            for (int k = 0; k < 8; k++) v[s][k] = r[s] ? v[s][k] : u[k];
-                        }
-                    }
-                }
-            }
-            mfma_dft<LA>(v, mat, lane_now());
-            {
-                // exchange: (column, j1) DFTs to (column, k1) DFTs, 16 bytes of each element at a time
-                const uint32_t lane = lane_now(), n = lane & 15, h = lane >> 4;
-                uint4 lo[4];
-#pragma clang loop unroll(full)
-                for (int hw = 0; hw < 2; hw++) {
-#pragma clang loop unroll(full)
-                    for (int s = 0; s < 4; s++) {
-                        const uint32_t d = mfma_dft_index<LA>(s, n);
-                        uint4 *q4 = reinterpret_cast<uint4 *>(xch + (d * (SA + 1) + mfma_out<LA>(s, h)) * 16);
-                        *q4 = make_uint4(v[s][4 * hw], v[s][4 * hw + 1], v[s][4 * hw + 2], v[s][4 * hw + 3]);
-                    }
-                    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "workgroup"); __builtin_amdgcn_wave_barrier();
-#pragma clang loop unroll(full)
-                    for (int s = 0; s < 4; s++) {
-                        const uint32_t d = mfma_dft_index<LB>(s, n);
-                        const uint4 c = *reinterpret_cast<const uint4 *>(
-                            xch + (((mfma_in<LB>(s, h) << kLogCols) + col_b(d)) * (SA + 1) + k1_b(d)) * 16);
-                        if (hw == 0) {
-                            lo[s] = c;
-                        } else {
-                            v[s][4] = c.x, v[s][5] = c.y, v[s][6] = c.z, v[s][7] = c.w;
-                            v[s][0] = lo[s].x, v[s][1] = lo[s].y, v[s][2] = lo[s].z, v[s][3] = lo[s].w;
-                        }
-                    }
-                    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "workgroup"); __builtin_amdgcn_wave_barrier();
-                }
-            }
-            {
-                // twiddles w_D^(j1 k1)
-                const uint32_t lane = lane_now(), n = lane & 15, h = lane >> 4;
-#pragma clang loop unroll(full)
-                for (int s = 0; s < 4; s++) {
-                    const uint32_t e = mfma_in<LB>(s, h) * k1_b(mfma_dft_index<LB>(s, n));
-                    const uint4 *t = reinterpret_cast<const uint4 *>(tw + e * kMfmaTwWords);
-                    const uint4 ta = t[0], tb = t[1];
-                    w[s] = F29{{ta.x, ta.y, ta.z, ta.w, tb.x, tb.y, tb.z, tb.w, t[2].x}};
-                    twiddle(s);
-                }
-            }
-            mfma_dft<LB>(v, mat, lane_now());
-            // store: canonical after the last pass, else below 1.001 r
+        {
+            // load, columns from lane to lane; the coset scale or the inter-pass twiddle
             const uint32_t lane = lane_now(), n = lane & 15, h = lane >> 4;
-            const bool last = log_p + deg == log_n;
+            uint32_t pos[4];
+            Fr o[4];
 #pragma clang loop unroll(full)
             for (int s = 0; s < 4; s++) {
-                const uint32_t d = mfma_dft_index<LB>(s, n), index = index0 + col_b(d), kk = index & (p - 1);
-                const uint32_t addr = ((index - kk) << deg) + kk + ((k1_b(d) + SA * mfma_out<LB>(s, h)) << log_p);
-                if (last) fr_cond_sub(v[s]);
-                Fr e;
+                const uint32_t d = mfma_dft_index<LA>(s, n), i = mfma_in<LA>(s, h) * SB + (d >> kLogCols);
+                const uint32_t c = index0 + (d & (kCols - 1));
+                pos[s] = c + (i << log_t);
+                const bool in = !FIRST || !nz || pos[s] < nz;
+                const Fr e = fe_load<FrParams>(&x[in ? pos[s] : 0]);
 #pragma clang loop unroll(full)
-                for (int k = 0; k < 8; k++) e.v[k] = v[s][k];
-                fe_store<FrParams>(&y[addr], e);
+                for (int k = 0; k < 8; k++) v[s][k] = e.v[k];
+                if constexpr (!FIRST) o[s] = fe_load<FrParams>(&omegas[((c & (p - 1)) * i) << (log_t - log_p)]);
             }
+            if constexpr (!FIRST) {
+#pragma clang loop unroll(full)
+                for (int s = 0; s < 4; s++) {
+                    w[s] = f29_from32(o[s]);
+                    twiddle(s);
+                }
+            } else if (nz) {
+#pragma clang loop unroll(full)
+                for (int s = 0; s < 4; s++) {
+#pragma clang loop unroll(full)
+                    for (int k = 0; k < 8; k++) v[s][k] = pos[s] < nz ? v[s][k] : 0u;
+                }
+                if (cn > 1) {
+                    uint32_t r[4];
+#pragma clang loop unroll(full)
+                    for (int s = 0; s < 4; s++) {
+                        r[s] = pos[s] % cn;
+                        o[s] = fe_load<FrParams>(&job.coset[r[s] ? r[s] - 1 : 0]);
+                    }
+#pragma clang loop unroll(full)
+                    for (int s = 0; s < 4; s++) {
+                        if (((mfma_in<LA>(s, 0) * SB) << log_t) >= nz) continue;  // all zero
+                        uint32_t u[8];
+#pragma clang loop unroll(full)
+                        for (int k = 0; k < 8; k++) u[k] = v[s][k];
+                        w[s] = f29_from32(o[s]);
+                        twiddle(s);
+#pragma clang loop unroll(full)
+                        for (int k = 0; k < 8; k++) v[s][k] = r[s] ? v[s][k] : u[k];
+                    }
+                }
+            }
+        }
+        mfma_dft<LA>(v, mat, lane_now());
+        {
+            // exchange: (column, j1) DFTs to (column, k1) DFTs, 16 bytes of each element at a time
+            const uint32_t lane = lane_now(), n = lane & 15, h = lane >> 4;
+            uint4 lo[4];
+#pragma clang loop unroll(full)
+            for (int hw = 0; hw < 2; hw++) {
+#pragma clang loop unroll(full)
+                for (int s = 0; s < 4; s++) {
+                    const uint32_t d = mfma_dft_index<LA>(s, n);
+                    uint4 *q4 = reinterpret_cast<uint4 *>(xch + (d * (SA + 1) + mfma_out<LA>(s, h)) * 16);
+                    *q4 = make_uint4(v[s][4 * hw], v[s][4 * hw + 1], v[s][4 * hw + 2], v[s][4 * hw + 3]);
+                }
+                __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "workgroup"); __builtin_amdgcn_wave_barrier();
+#pragma clang loop unroll(full)
+                for (int s = 0; s < 4; s++) {
+                    const uint32_t d = mfma_dft_index<LB>(s, n);
+                    const uint4 c = *reinterpret_cast<const uint4 *>(
+                        xch + (((mfma_in<LB>(s, h) << kLogCols) + col_b(d)) * (SA + 1) + k1_b(d)) * 16);
+                    if (hw == 0) {
+                        lo[s] = c;
+                    } else {
+                        v[s][4] = c.x, v[s][5] = c.y, v[s][6] = c.z, v[s][7] = c.w;
+                        v[s][0] = lo[s].x, v[s][1] = lo[s].y, v[s][2] = lo[s].z, v[s][3] = lo[s].w;
+                    }
+                }
+                __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "workgroup"); __builtin_amdgcn_wave_barrier();
+            }
+        }
+        {
+            // twiddles w_D^(j1 k1)
+            const uint32_t lane = lane_now(), n = lane & 15, h = lane >> 4;
+#pragma clang loop unroll(full)
+            for (int s = 0; s < 4; s++) {
+                const uint32_t e = mfma_in<LB>(s, h) * k1_b(mfma_dft_index<LB>(s, n));
+                const uint4 *t = reinterpret_cast<const uint4 *>(tw + e * kMfmaTwWords);
+                const uint4 ta = t[0], tb = t[1];
+                w[s] = F29{{ta.x, ta.y, ta.z, ta.w, tb.x, tb.y, tb.z, tb.w, t[2].x}};
+                twiddle(s);
+            }
+        }
+        mfma_dft<LB>(v, mat, lane_now());
+        // store: canonical after the last pass, else below 1.001 r
+        const uint32_t lane = lane_now(), n = lane & 15, h = lane >> 4;
+        const bool last = log_p + deg == log_n;
+#pragma clang loop unroll(full)
+        for (int s = 0; s < 4; s++) {
+            const uint32_t d = mfma_dft_index<LB>(s, n), index = index0 + col_b(d), kk = index & (p - 1);
+            const uint32_t addr = ((index - kk) << deg) + kk + ((k1_b(d) + SA * mfma_out<LB>(s, h)) << log_p);
+            if (last) fr_cond_sub(v[s]);
+            Fr e;
+#pragma clang loop unroll(full)
+            for (int k = 0; k < 8; k++) e.v[k] = v[s][k];
+            fe_store<FrParams>(&y[addr], e);
         }
     }
 }
@@ -732,37 +729,70 @@ static void fill_job(NttJob &j, const NttSpec &sp, int r, int np, uint32_t logp,
 // The degrees whose passes of round r go to the matrix cores: 6 and 7, and 8
 // in the first round (later its one column per wave would be loaded and stored
 // in runs of 32 bytes: 2^24 elements 880 and 1100 us per pass against 690 with the
-// radix-2 kernel), where the launch has at least 2^19 elements (two waves of
-// 256 elements for each SIMD).  Below that a pass is one tile's latency plus the tables, and the
+// radix-2 kernel), where the launch (at most kJobsPerLaunch transforms, not the
+// whole batch) has at least 2^19 elements (two waves of 256 elements for each
+// SIMD).  Below that a pass is one tile's latency plus the tables, and the
 // radix-2 kernel with its shorter chains is as fast or faster (one transform,
-// both ways: 2^18 57 us here and 52 there, 2^19 79 and 87, 2^20 114 and 145;
-// eight transforms: 2^15 44 and 44, 2^16 61 and 65, 2^18 187 and 226).
-constexpr uint32_t kMfmaMinLog = 12;  // the tables of a smaller transform would cost more than its tiles
+// both ways: 2^18 57 us here and 52 there, 2^19 68 and 86, 2^20 98 and 142;
+// eight of 2^16 51 and 60).  Transforms below 2^15 stay there too: the tables
+// cost as much as their few tiles (2^14, both ways: 32 transforms 53 and 56 us,
+// 48 75 and 72, 64 114 and 107; 256 of 2^12 297 and 199).
+constexpr uint32_t kMfmaMinLog = 15;
 static bool mfma_degree(const NttSpec &sp, uint32_t deg, int r) {
     return sp.log_n >= kMfmaMinLog && deg >= 6 && deg <= (r ? 7 : 8);
 }
-static uint32_t mfma_degrees(const NttSpec *specs, uint32_t count, const uint32_t *degs, const int *np, int r) {
-    uint64_t elems[9] = {};
-    for (uint32_t m = 0; m < count; m++) {
-        if (r >= np[m]) continue;
-        const uint32_t deg = degs[(size_t)m * 32 + r];
-        if (mfma_degree(specs[m], deg, r)) elems[deg] += 1ull << specs[m].log_n;
+// on[m]: transform m's pass of round r goes to the matrix cores, decided
+// launch by launch as mfma_round forms them
+static void mfma_choose(const NttSpec *specs, uint32_t count, const uint32_t *degs, const int *np, int r,
+                        std::vector<uint8_t> &on) {
+    on.assign(count, 0);
+    if (!register_rounds_enabled()) return;
+    for (uint32_t d = 6; d <= 8; d++) {
+        uint32_t first = 0, jobs = 0;  // of the launch being filled, from transform `first`
+        uint64_t elems = 0;
+        for (uint32_t m = 0; m <= count; m++) {
+            const bool mine = m < count && r < np[m] && degs[(size_t)m * 32 + r] == d && mfma_degree(specs[m], d, r);
+            if (mine && !jobs++) first = m;
+            if (mine) elems += 1ull << specs[m].log_n;
+            if (jobs < kJobsPerLaunch && m < count) continue;
+            if (elems >= kMfmaMinElems)
+                for (uint32_t q = first; q <= m && q < count; q++)
+                    if (r < np[q] && degs[(size_t)q * 32 + r] == d && mfma_degree(specs[q], d, r)) on[q] = 1;
+            jobs = 0;
+            elems = 0;
+        }
     }
-    uint32_t set = 0;
-    for (uint32_t d = 6; d <= 8; d++) set |= elems[d] >= kMfmaMinElems ? 1u << d : 0u;
-    return register_rounds_enabled() ? set : 0u;
 }
 
 // one workgroup (of four waves per SIMD) on each CU
 constexpr uint32_t kMfmaGrid = 256;
 
-// pass r of every transform whose degree is in set, one launch per degree and
+// pass r of the transforms that are on, one launch per degree and
 // kJobsPerLaunch transforms
 template <int LA, int LB, bool FIRST>
 static hipError_t mfma_launch(NttPassArgs &args, uint32_t &tiles, hipStream_t stream) {
     if (args.count) {
-        const uint32_t blocks = (tiles + 3) / 4;
-        k_ntt_mfma<LA, LB, FIRST><<<blocks < kMfmaGrid ? blocks : kMfmaGrid, kMfmaThreads, 0, stream>>>(args, tiles);
+        // the fewest tiles per workgroup with which the jobs' own workgroups fit
+        // the grid (block0 counts them)
+        auto number = [&](uint32_t per) {
+            uint32_t blocks = 0;
+            for (uint32_t q = 0; q < args.count; q++) {
+                args.job[q].block0 = blocks;
+                blocks += ((1u << (args.job[q].log_n - 8)) + per - 1) / per;
+            }
+            return blocks;
+        };
+        uint32_t lo = (tiles + kMfmaGrid - 1) / kMfmaGrid, per = tiles;  // per fits: one workgroup a job
+        if (lo < 4) lo = 4;
+        while (lo < per) {
+            const uint32_t mid = (lo + per) / 2;
+            if (number(mid) <= kMfmaGrid)
+                per = mid;
+            else
+                lo = mid + 1;
+        }
+        const uint32_t blocks = number(per);
+        k_ntt_mfma<LA, LB, FIRST><<<blocks, kMfmaThreads, 0, stream>>>(args, per);
         ZK_CHECK(hipGetLastError());
     }
     memset(&args, 0, sizeof(args));
@@ -770,9 +800,8 @@ static hipError_t mfma_launch(NttPassArgs &args, uint32_t &tiles, hipStream_t st
     return hipSuccess;
 }
 static hipError_t mfma_round(const NttSpec *specs, uint32_t count, const uint32_t *degs, const int *np,
-                             const uint32_t *logp, int r, uint32_t set, hipStream_t stream) {
+                             const uint32_t *logp, int r, const std::vector<uint8_t> &on, hipStream_t stream) {
     for (uint32_t d = 6; d <= 8; d++) {
-        if (!(set >> d & 1)) continue;
         auto launch = [&](NttPassArgs &args, uint32_t &tiles) {
             if (r == 0)
                 return d == 8   ? mfma_launch<4, 4, true>(args, tiles, stream)
@@ -785,8 +814,8 @@ static hipError_t mfma_round(const NttSpec *specs, uint32_t count, const uint32_
         memset(&args, 0, sizeof(args));
         uint32_t tiles = 0;
         for (uint32_t m = 0; m < count; m++) {
-            if (r >= np[m] || degs[(size_t)m * 32 + r] != d || !mfma_degree(specs[m], d, r)) continue;
-            fill_job(args.job[args.count++], specs[m], r, np[m], logp[m], d, tiles);
+            if (!on[m] || degs[(size_t)m * 32 + r] != d) continue;
+            fill_job(args.job[args.count++], specs[m], r, np[m], logp[m], d, 0);
             tiles += 1u << (specs[m].log_n - 8);
             if (args.count == kJobsPerLaunch) ZK_CHECK(launch(args, tiles));
         }
@@ -799,6 +828,7 @@ hipError_t ntt_run_batch(const NttSpec *specs, uint32_t count, hipStream_t strea
     std::vector<uint32_t> degs((size_t)count * 32);
     std::vector<int> np(count);
     std::vector<uint32_t> logp(count, 0);
+    std::vector<uint8_t> mfma;
     int rounds = 0;
     for (uint32_t m = 0; m < count; m++) {
         np[m] = ntt_plan(specs[m].log_n, &degs[(size_t)m * 32]);
@@ -806,7 +836,7 @@ hipError_t ntt_run_batch(const NttSpec *specs, uint32_t count, hipStream_t strea
         if (passes) passes[m] = np[m];
     }
     for (int r = 0; r < rounds; r++) {
-        const uint32_t mfma = mfma_degrees(specs, count, degs.data(), np.data(), r);
+        mfma_choose(specs, count, degs.data(), np.data(), r, mfma);
         ZK_CHECK(mfma_round(specs, count, degs.data(), np.data(), logp.data(), r, mfma, stream));
         NttPassArgs args;
         memset(&args, 0, sizeof(args));
@@ -828,7 +858,7 @@ hipError_t ntt_run_batch(const NttSpec *specs, uint32_t count, hipStream_t strea
             const NttSpec &sp = specs[m];
             const uint32_t n = 1u << sp.log_n;
             const uint32_t deg = degs[(size_t)m * 32 + r];
-            if (mfma >> deg & 1 && mfma_degree(sp, deg, r)) {
+            if (mfma[m]) {
                 logp[m] += deg;
                 continue;
             }
