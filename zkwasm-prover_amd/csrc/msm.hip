@@ -104,9 +104,13 @@ enum MsmArr {
 constexpr int kFirstPhase2 = A_BUCKETS;
 
 // scalars per histogram / scatter tile: 4096, or 1024 while that leaves fewer
-// than kFewTiles tiles (one workgroup each: 2^17 points had 25 workgroups,
-// digits and histogram 51 us against 18)
-constexpr uint32_t kSortTile = 4096, kSmallTile = 1024, kFewTiles = 512;
+// than kFewTiles tiles, one workgroup of 1024 threads per CU (2^17 points had
+// 32, digits and histogram 51 us against 18).  With more the small tiles only
+// cost: their histogram and its scan are four times as long (2^20 zeros 235 and
+// 210 us, 2000001 uniform scalars 3330 and 3084).
+constexpr uint32_t kSortTile = 4096, kSmallTile = 1024, kFewTiles = 256;
+// workgroups the low-level sort should have
+constexpr uint32_t kFewGroups = 512;
 // Items of at most this many scalars are sorted by one workgroup per (item,
 // window) straight from the digits (k_msm_sort_window): no histogram, no
 // scan, no scatter.  Needs the window's buckets as LDS counters.
@@ -233,7 +237,7 @@ MsmPlan make_plan(const uint32_t *ns, uint32_t count, uint32_t c, bool fixed = f
         uint32_t hi = c - 1 > lo_most ? c - 1 - lo_most : 0;
         const uint64_t per = (uint64_t)nmax * (fixed ? p.Wd : 1);  // an item's entries in one bucket set
         while (hi < most && ((per >> hi) > kGroupWant ||
-                             ((uint64_t)count * p.W << hi) < kFewTiles && (per >> hi) > 2048))
+                             ((uint64_t)count * p.W << hi) < kFewGroups && (per >> hi) > 2048))
             hi++;
         p.hi_bits = hi;
     }
