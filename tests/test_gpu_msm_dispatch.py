@@ -69,3 +69,29 @@ def test_msm_opposite_buckets(gpu, zo):
     pts[0::2], pts[1::2] = half.reshape(n // 2, -1), neg.reshape(n // 2, -1)
     for vals in ([1] * n, [1 + k % 2 for k in range(n)], [1 + k // 2 for k in range(n)]):
         _check(zo, pts, np.concatenate([zo.fr_from_u64(v) for v in vals]), 8)
+
+
+# one to a few heavy buckets: up to 256 heads after the first chunk go to one
+# workgroup, more to one for each 256 (chunks of 8 here: 2056 entries are a tail
+# and 256 heads when the run starts a chunk)
+@pytest.mark.parametrize("n", [2040, 2048, 2056, 2057, 2064, 2065, 4105, 30000, 70001])
+def test_msm_heavy_buckets(gpu, zo, n):
+    pts = zo.gen_bases_random(n, 77)
+    one = zo.fr_from_u64(1)
+    _check(zo, pts, np.repeat(one, n, axis=0), 8)
+    rm1 = zo.to_mont([R - 1])
+    sc = np.repeat(rm1, n, axis=0)
+    sc[:: 3] = zo.fr_from_u64(200)
+    sc[1:: 101] = zo.rand_fr(len(sc[1:: 101]), 78)
+    _check(zo, pts, sc, 0)
+
+
+def test_msm_heavy_bucket_equal_points(gpu, zo):
+    """equal parts of one bucket (doublings when the parts are added) and parts
+    that cancel"""
+    n = 8 * 256 * 4
+    pts = np.repeat(zo.gen_bases_random(1, 9).reshape(1, -1), n, axis=0)
+    sc = np.repeat(zo.fr_from_u64(1), n, axis=0)
+    _check(zo, pts, sc, 9)
+    pts[n // 2:] = _negated(pts[n // 2:].reshape(n // 2, -1)).reshape(n // 2, -1)
+    _check(zo, pts, sc, 9)

@@ -73,8 +73,10 @@ constexpr uint32_t kRoundThreads = 256 * 256;
 constexpr uint32_t kMinRounds = 3;
 constexpr uint32_t kMinChunk = 8;
 // Buckets whose run spans more chunks than this go to a workgroup each
-// (k_msm_fixup_long), the others to one quad of lanes, a serial chain.
-constexpr uint32_t kWalk = 12;
+// (k_msm_fixup_long), or to one for each kPartHeads of them, the others to one
+// quad of lanes, a serial chain.
+constexpr uint32_t kWalk = 12, kPartHeads = 256;
+constexpr uint32_t kLongWords = 5;  // of a list entry, see k_msm_fixup_long
 // Bucket reduction: up to this many buckets in the pass by quads of lanes
 // (k_msm_bits: a chain of 4 + B / 1024 + 6 additions), above it by one lane
 // per 8 buckets (k_msm_reduce_fold: 22 additions, a third less lane work).
@@ -201,6 +203,10 @@ inline uint32_t min_chunk(uint64_t max_entries) {
     return ch < kChunk ? ch : kChunk;
 }
 
+// entries the list of long buckets can have: such a bucket owns kWalk whole
+// chunks at least, and has one entry more than full parts
+inline uint64_t long_parts(uint64_t chunks) { return chunks / kWalk + chunks / kPartHeads + 2; }
+
 // chunk: smallest chunk of the accumulation (the partial sums' arrays are
 // sized for it), 0 = what the pass would like; small_tiles = false: large sort
 // tiles, whose histogram is a quarter
@@ -272,8 +278,8 @@ MsmPlan make_plan(const uint32_t *ns, uint32_t count, uint32_t c, bool fixed = f
     p.size[A_PTAIL] = (size_t)p.chunks * sizeof(X29S);
     p.size[A_TB] = (size_t)p.chunks * 4;
     p.size[A_PART] = p.quads ? 0 : (size_t)count * p.W * (p.T1 / 64) * kFoldParts * sizeof(X29S);
-    // [count, (bucket, first chunk, last chunk) per bucket spanning > kWalk chunks]
-    p.size[A_LONG] = (size_t)(1 + 3 * (p.chunks / kWalk + 1)) * 4;
+    // [count, an entry per kPartHeads chunks of a bucket spanning > kWalk chunks]
+    p.size[A_LONG] = (size_t)(1 + kLongWords * long_parts(p.chunks)) * 4;
     return p;
 }
 
@@ -994,8 +1000,8 @@ __global__ __launch_bounds__(256) void k_msm_accumulate(const uint32_t *__restri
 // bucket, 112 by chunk; 16 columns of 2^18, a third of a chunk per bucket: 36 us
 // by chunk, 176 by bucket).  Spans of more than kWalk chunks (few: their
 // count is at most nchunks / kWalk) are listed for k_msm_fixup_long, one
-// workgroup each, so a heavy bucket (e.g. the multiplicities of a lookup, all
-// in a handful of buckets) never becomes a serial chain.  The chains are what
+// workgroup or more each, so a heavy bucket (e.g. the multiplicities of a
+// lookup, all in a handful of buckets) never becomes a serial chain.  The chains are what
 // this takes (the additions themselves are few), hence quads.
 __global__ __launch_bounds__(256) void k_msm_fixup(X29S *__restrict__ buckets, const X29S *__restrict__ phead,
                                                    const X29S *__restrict__ ptail, const uint32_t *__restrict__ tb,
@@ -1016,10 +1022,15 @@ __global__ __launch_bounds__(256) void k_msm_fixup(X29S *__restrict__ buckets, c
     if (t == last) return;  // one chunk owned the whole run and stored it
     if (last - t > kWalk) {
         if (q == 0) {
-            const uint32_t k = atomicAdd(&longs[0], 1u);
-            longs[1 + 3 * k] = b;
-            longs[2 + 3 * k] = t;
-            longs[3 + 3 * k] = last;
+            const uint32_t parts = (last - t + kPartHeads - 1) / kPartHeads, k0 = atomicAdd(&longs[0], parts);
+            for (uint32_t k = k0; k < k0 + parts; k++) {
+                uint32_t *e = longs + 1 + kLongWords * k;
+                e[0] = b;
+                e[1] = t;
+                e[2] = last;
+                e[3] = k0;
+                e[4] = 0;
+            }
         }
         return;
     }
@@ -1063,24 +1074,45 @@ __device__ __forceinline__ void q29_block_sum(Q29 &p, bool &pe, uint32_t q, X29S
     __syncthreads();
 }
 
-// one workgroup of 64 quads per listed long bucket: ptail[t] + sum of
-// phead[t+1..last]
-__global__ __launch_bounds__(256) void k_msm_fixup_long(X29S *__restrict__ buckets,
-                                                        const X29S *__restrict__ phead,
-                                                        const X29S *__restrict__ ptail,
-                                                        const uint32_t *__restrict__ longs) {
+// ptail[t] + sum of phead[t+1..last] for the listed buckets, one workgroup of
+// 64 quads for each kPartHeads of a bucket's heads.  Entry k of the list:
+// (bucket, t, last, the bucket's first entry k0, workgroups that are done).
+// With several parts each leaves its sum at its own first head, and the one
+// that finishes last (it waits for none) adds them: with one workgroup per
+// bucket, chunks chosen for many threads made one heavy bucket a chain (300000
+// scalars of 1, 23 k partial sums: 1005 us, whole MSM 2050 and 1105 us).
+__global__ __launch_bounds__(256) void k_msm_fixup_long(X29S *__restrict__ buckets, X29S *phead,
+                                                        const X29S *__restrict__ ptail, uint32_t *longs) {
     __shared__ X29S sh[4];
+    __shared__ uint32_t done;
     const uint32_t count = longs[0], q = threadIdx.x & 3, quad = threadIdx.x >> 2;
-    for (uint32_t i = blockIdx.x; i < count; i += gridDim.x) {
-        const uint32_t b = longs[1 + 3 * i], t = longs[2 + 3 * i], last = longs[3 + 3 * i];
+    for (uint32_t k = blockIdx.x; k < count; k += gridDim.x) {
+        const uint32_t *e = longs + 1 + kLongWords * k;
+        const uint32_t b = e[0], t = e[1], last = e[2], k0 = e[3];
+        const uint32_t parts = (last - t + kPartHeads - 1) / kPartHeads, u0 = t + 1 + (k - k0) * kPartHeads;
+        const uint32_t u1 = last - u0 < kPartHeads ? last : u0 + kPartHeads - 1;
         bool ae = true, qe;
         Q29 acc{};
-        if (quad == 0) acc = q29_load(&ptail[t], ae, q);
-        for (uint32_t u = t + 1 + quad; u <= last; u += blockDim.x / 4) {
+        if (k == k0 && quad == 0) acc = q29_load(&ptail[t], ae, q);
+        for (uint32_t u = u0 + quad; u <= u1; u += blockDim.x / 4) {
             const Q29 v = q29_load(&phead[u], qe, q);
             q29_add(acc, ae, v, qe, q);
         }
         q29_block_sum(acc, ae, q, sh);
+        if (parts > 1) {
+            if (threadIdx.x < 4) q29_store(&phead[u0], acc, ae, q);
+            __threadfence();
+            if (threadIdx.x == 0) done = atomicAdd(&longs[1 + kLongWords * k0 + 4], 1u);
+            __syncthreads();
+            if (done + 1 < parts) continue;
+            __threadfence();
+            ae = true;
+            for (uint32_t p = quad; p < parts; p += blockDim.x / 4) {
+                const Q29 v = q29_load(&phead[t + 1 + p * kPartHeads], qe, q);
+                q29_add(acc, ae, v, qe, q);
+            }
+            q29_block_sum(acc, ae, q, sh);
+        }
         if (threadIdx.x < 4) q29_store(&buckets[b], acc, ae, q);
     }
 }
@@ -1694,7 +1726,7 @@ hipError_t msm_run(const MsmJob *jobs, uint32_t count, size_t slice_bytes, uint3
                                                                    longs, (uint32_t)p.chunks, p.chunk);
     ZK_CHECK(hipGetLastError());
     {
-        const uint64_t max_long = p.chunks / kWalk + 1;
+        const uint64_t max_long = long_parts(p.chunks);
         k_msm_fixup_long<<<(uint32_t)(max_long < 1024 ? max_long : 1024), 256, 0, stream>>>(buckets, phead, ptail,
                                                                                            longs);
         ZK_CHECK(hipGetLastError());
