@@ -71,10 +71,10 @@ def test_msm_opposite_buckets(gpu, zo):
         _check(zo, pts, np.concatenate([zo.fr_from_u64(v) for v in vals]), 8)
 
 
-# one to a few heavy buckets: up to 256 heads after the first chunk go to one
-# workgroup, more to one for each 256 (chunks of 8 here: 2056 entries are a tail
-# and 256 heads when the run starts a chunk)
-@pytest.mark.parametrize("n", [2040, 2048, 2056, 2057, 2064, 2065, 4105, 30000, 70001])
+# one to a few heavy buckets: up to 1024 heads after the first chunk go to one
+# workgroup, more to one for each 512 (chunks of 8 here: 8200 entries are a tail
+# and 1024 heads when the run starts a chunk)
+@pytest.mark.parametrize("n", [2048, 8192, 8200, 8201, 8209, 12297, 12305, 30000, 70001])
 def test_msm_heavy_buckets(gpu, zo, n):
     pts = zo.gen_bases_random(n, 77)
     one = zo.fr_from_u64(1)
@@ -89,7 +89,7 @@ def test_msm_heavy_buckets(gpu, zo, n):
 def test_msm_heavy_bucket_equal_points(gpu, zo):
     """equal parts of one bucket (doublings when the parts are added) and parts
     that cancel"""
-    n = 8 * 256 * 4
+    n = 8 * 512 * 4
     pts = np.repeat(zo.gen_bases_random(1, 9).reshape(1, -1), n, axis=0)
     sc = np.repeat(zo.fr_from_u64(1), n, axis=0)
     _check(zo, pts, sc, 9)

@@ -73,10 +73,11 @@ constexpr uint32_t kRoundThreads = 256 * 256;
 constexpr uint32_t kMinRounds = 3;
 constexpr uint32_t kMinChunk = 8;
 // Buckets whose run spans more chunks than this go to a workgroup each
-// (k_msm_fixup_long), or to one for each kPartHeads of them, the others to one
-// quad of lanes, a serial chain.
-constexpr uint32_t kWalk = 12, kPartHeads = 256;
+// (k_msm_fixup_long), the others to one quad of lanes, a serial chain.  More
+// than kSplitHeads chunks go to a workgroup for each kPartHeads of them.
+constexpr uint32_t kWalk = 12, kSplitHeads = 1024, kPartHeads = 512;
 constexpr uint32_t kLongWords = 5;  // of a list entry, see k_msm_fixup_long
+__host__ __device__ inline uint32_t heads_per_part(uint32_t heads) { return heads > kSplitHeads ? kPartHeads : heads; }
 // Bucket reduction: up to this many buckets in the pass by quads of lanes
 // (k_msm_bits: a chain of 4 + B / 1024 + 6 additions), above it by one lane
 // per 8 buckets (k_msm_reduce_fold: 22 additions, a third less lane work).
@@ -278,7 +279,7 @@ MsmPlan make_plan(const uint32_t *ns, uint32_t count, uint32_t c, bool fixed = f
     p.size[A_PTAIL] = (size_t)p.chunks * sizeof(X29S);
     p.size[A_TB] = (size_t)p.chunks * 4;
     p.size[A_PART] = p.quads ? 0 : (size_t)count * p.W * (p.T1 / 64) * kFoldParts * sizeof(X29S);
-    // [count, an entry per kPartHeads chunks of a bucket spanning > kWalk chunks]
+    // [count, an entry per part of a bucket spanning > kWalk chunks]
     p.size[A_LONG] = (size_t)(1 + kLongWords * long_parts(p.chunks)) * 4;
     return p;
 }
@@ -1022,7 +1023,8 @@ __global__ __launch_bounds__(256) void k_msm_fixup(X29S *__restrict__ buckets, c
     if (t == last) return;  // one chunk owned the whole run and stored it
     if (last - t > kWalk) {
         if (q == 0) {
-            const uint32_t parts = (last - t + kPartHeads - 1) / kPartHeads, k0 = atomicAdd(&longs[0], parts);
+            const uint32_t per = heads_per_part(last - t), parts = (last - t + per - 1) / per;
+            const uint32_t k0 = atomicAdd(&longs[0], parts);
             for (uint32_t k = k0; k < k0 + parts; k++) {
                 uint32_t *e = longs + 1 + kLongWords * k;
                 e[0] = b;
@@ -1075,12 +1077,17 @@ __device__ __forceinline__ void q29_block_sum(Q29 &p, bool &pe, uint32_t q, X29S
 }
 
 // ptail[t] + sum of phead[t+1..last] for the listed buckets, one workgroup of
-// 64 quads for each kPartHeads of a bucket's heads.  Entry k of the list:
-// (bucket, t, last, the bucket's first entry k0, workgroups that are done).
-// With several parts each leaves its sum at its own first head, and the one
-// that finishes last (it waits for none) adds them: with one workgroup per
-// bucket, chunks chosen for many threads made one heavy bucket a chain (300000
-// scalars of 1, 23 k partial sums: 1005 us, whole MSM 2050 and 1105 us).
+// 64 quads for each part of a bucket's heads.  Entry k of the list: (bucket, t,
+// last, the bucket's first entry k0, workgroups that are done).  With several
+// parts each leaves its sum at its own first head, and the one that finishes
+// last (it waits for none) adds them: with one workgroup per bucket, chunks
+// chosen for many threads made one heavy bucket a chain (300000 scalars of 1,
+// 23 k partial sums: 1007 us, now 64; 60000 uniform scalars, whose top window
+// has four buckets of 1.9 k: whole MSM 681 and 556).  The trees and the cache
+// write-back of each part cost where there are many long buckets as it is (16
+// columns of 2^18 r - 1 against a table, 240 buckets of 2731 heads: 176 us in
+// one part each, 268 in parts of 512, 464 in parts of 256), so up to
+// kSplitHeads stay whole.
 __global__ __launch_bounds__(256) void k_msm_fixup_long(X29S *__restrict__ buckets, X29S *phead,
                                                         const X29S *__restrict__ ptail, uint32_t *longs) {
     __shared__ X29S sh[4];
@@ -1089,8 +1096,8 @@ __global__ __launch_bounds__(256) void k_msm_fixup_long(X29S *__restrict__ bucke
     for (uint32_t k = blockIdx.x; k < count; k += gridDim.x) {
         const uint32_t *e = longs + 1 + kLongWords * k;
         const uint32_t b = e[0], t = e[1], last = e[2], k0 = e[3];
-        const uint32_t parts = (last - t + kPartHeads - 1) / kPartHeads, u0 = t + 1 + (k - k0) * kPartHeads;
-        const uint32_t u1 = last - u0 < kPartHeads ? last : u0 + kPartHeads - 1;
+        const uint32_t per = heads_per_part(last - t), parts = (last - t + per - 1) / per;
+        const uint32_t u0 = t + 1 + (k - k0) * per, u1 = last - u0 < per ? last : u0 + per - 1;
         bool ae = true, qe;
         Q29 acc{};
         if (k == k0 && quad == 0) acc = q29_load(&ptail[t], ae, q);
@@ -1100,15 +1107,17 @@ __global__ __launch_bounds__(256) void k_msm_fixup_long(X29S *__restrict__ bucke
         }
         q29_block_sum(acc, ae, q, sh);
         if (parts > 1) {
-            if (threadIdx.x < 4) q29_store(&phead[u0], acc, ae, q);
-            __threadfence();
-            if (threadIdx.x == 0) done = atomicAdd(&longs[1 + kLongWords * k0 + 4], 1u);
+            if (threadIdx.x < 64) {  // the wave that has the sum
+                if (threadIdx.x < 4) q29_store(&phead[u0], acc, ae, q);
+                __threadfence();
+                if (threadIdx.x == 0) done = atomicAdd(&longs[1 + kLongWords * k0 + 4], 1u);
+            }
             __syncthreads();
             if (done + 1 < parts) continue;
             __threadfence();
             ae = true;
             for (uint32_t p = quad; p < parts; p += blockDim.x / 4) {
-                const Q29 v = q29_load(&phead[t + 1 + p * kPartHeads], qe, q);
+                const Q29 v = q29_load(&phead[t + 1 + p * per], qe, q);
                 q29_add(acc, ae, v, qe, q);
             }
             q29_block_sum(acc, ae, q, sh);
