@@ -333,7 +333,8 @@ hipError_t zk_coset_extend_batch(const zk_coset_item *items, int count, const vo
                                  int coset_powers_n, unsigned char *swapped, hipStream_t stream);
 
 /* Radix choice per size (autotuner hook): largest pass degree for 2^log_n
- * transforms, 1..8 (0 = default 8). */
+ * transforms, 1..8; 0 = the default plan (8, or 6 for 2^24, which the getter
+ * then returns: set again, it gives the same plan). */
 hipError_t zk_ntt_set_max_deg(int log_n, int max_deg);
 int zk_ntt_get_max_deg(int log_n);
 /* Autotuner: times each distinct radix plan (largest pass degree 4..8) for

@@ -247,6 +247,15 @@ def test_msm_fits_reference_buffers(lib, count):
             assert c == lib.zk_msm_default_window(n), (n, count, c)
 
 
+def test_ntt_default_degree_read_and_set_back(lib):
+    """the degree read for an untuned size names the default plan (2^24 runs as
+    four passes of degree 6), so a table that is read and restored changes none"""
+    lib.zk_ntt_get_max_deg.restype = ctypes.c_int
+    for k in range(1, 31):
+        passes = -(-k // 8) + (1 if k == 24 else 0)
+        assert -(-k // lib.zk_ntt_get_max_deg(k)) == passes, k
+
+
 def test_prover_core_sizing_host_only(lib):
     """footprints and commitment counts come from a host-side layout pass;
     inconsistent circuits are rejected with 0"""

@@ -657,26 +657,31 @@ __global__ void k_coset_scale(Fr *s, const Fr *__restrict__ cp, uint32_t cn, uin
 
 namespace zk {
 
-// elements a launch of matrix-core passes must have, see mfma_degrees
+// elements a launch of matrix-core passes must have, see mfma_degree
 constexpr uint32_t kMfmaMinElems = 1u << 19;
 
-// Largest pass degree per transform size; 0 = kMaxDeg.  Set by the
+// Largest pass degree per transform size; 0 = the default plan.  Set by the
 // autotuner (zk_ntt_set_max_deg), read by every plan, possibly from other
 // threads: atomic (the plan changes only the speed, never the result).
 std::atomic<uint8_t> g_max_deg[31];
 
-// Radix plan: ceil(log_n / max_deg) passes, bits spread evenly (larger first).
-// Where every pass of a large transform would have degree 8 (2^24: 8 8 8) one
-// pass more is faster: all of them have degrees that run on the matrix cores, of
-// degree 8 only the first does (2^24, one transform 1970 us as 8 8 8 and 1789
-// as 6 6 6 6; four 7986 and 6654; with one degree below 8, 2^23 = 8 8 7, 937
-// and 942, four 3451 and 3584).
+// Passes of the untuned plan: ceil(log_n / 8), but one more where that would be
+// three or more of degree 8, of which only the first would run on the matrix
+// cores (up to 2^30: 2^24 alone, 6 6 6 6 1803 us and 8 8 8 2091; four of them
+// 6654 and 7986).  Two passes of degree 8 stay: 2^16, one transform 34 us and
+// 43 as 6 5 5, sixteen 85 and 110; so do plans with one degree below 8 (2^23 =
+// 8 8 7, 937 and 942 us, four 3451 and 3584).
+static uint32_t default_passes(uint32_t log_n) {
+    const uint32_t passes = (log_n + kMaxDeg - 1) / kMaxDeg;
+    return passes > 2 && log_n % kMaxDeg == 0 ? passes + 1 : passes;
+}
+
+// Radix plan: the default's passes or, tuned, ceil(log_n / max_deg); bits
+// spread evenly (larger first).
 int ntt_plan(uint32_t log_n, uint32_t *degs) {
     if (log_n == 0) return 0;
     const uint8_t tuned = log_n < 31 ? g_max_deg[log_n].load(std::memory_order_relaxed) : 0;
-    const uint32_t md = tuned ? tuned : kMaxDeg;
-    uint32_t passes = (log_n + md - 1) / md;
-    if (!tuned && (1ull << log_n) >= kMfmaMinElems && log_n % kMaxDeg == 0) passes++;
+    const uint32_t passes = tuned ? (log_n + tuned - 1) / tuned : default_passes(log_n);
     uint32_t rem = log_n;
     for (uint32_t i = 0; i < passes; i++) {
         uint32_t left = passes - i;
@@ -1041,7 +1046,8 @@ hipError_t zk_coset_extend_batch(const zk_coset_item *items, int count, const vo
 }
 
 // Autotuner hook: the largest pass degree (radix 2^max_deg) for transforms
-// of 2^log_n elements; 0 restores the default (8).
+// of 2^log_n elements; 0 restores the default.  The value read is one that, set
+// again, gives the plan in force.
 hipError_t zk_ntt_set_max_deg(int log_n, int max_deg) {
     if (log_n < 1 || log_n > 30 || max_deg < 0 || max_deg > (int)kMaxDeg) return hipErrorInvalidValue;
     g_max_deg[log_n].store((uint8_t)max_deg, std::memory_order_relaxed);
@@ -1050,7 +1056,9 @@ hipError_t zk_ntt_set_max_deg(int log_n, int max_deg) {
 int zk_ntt_get_max_deg(int log_n) {
     if (log_n < 1 || log_n > 30) return 0;
     const uint8_t tuned = g_max_deg[log_n].load(std::memory_order_relaxed);
-    return tuned ? tuned : (int)kMaxDeg;
+    if (tuned) return tuned;
+    const uint32_t passes = default_passes((uint32_t)log_n), deg = ((uint32_t)log_n + passes - 1) / passes;
+    return (int)(passes > ((uint32_t)log_n + kMaxDeg - 1) / kMaxDeg ? deg : kMaxDeg);
 }
 
 // Autotuner: times the NTT of 2^log_n elements (buf / tmp device buffers,
