@@ -454,6 +454,11 @@ hipError_t zk_msm_autotune(const void *points, const void *scalars, int n, int r
 hipError_t zk_fr_op(void *out, const void *a, const void *b, int op, int n, hipStream_t stream);
 hipError_t zk_fp_op(void *out, const void *a, const void *b, int op, int n, hipStream_t stream);
 hipError_t zk_g1_op(void *out, const void *a, const void *b, int op, int n, hipStream_t stream);
+/* the wave-wide inversion inside the batch inversions, without the check and
+ * the fallback that follow it there: out[i] = v with a[i]^-1 = v 2^36 mod r,
+ * a[i] and v plain numbers below r, ok[i] (u32) = 1, or 0 where it failed
+ * (a[i] = 0) */
+hipError_t zk_fr_inv_wave(void *out, void *ok, const void *a, int n, hipStream_t stream);
 /* the 29-bit-limb Fp of the bucket accumulation through its conversions:
  * op 0 a*b, 1 a+b, 2 a-b, 3 a^2, 4 round trip (32-bit Montgomery in and out) */
 hipError_t zk_fp29_op(void *out, const void *a, const void *b, int op, int n, hipStream_t stream);

@@ -130,3 +130,27 @@ def test_captured_batch_replays(gpu, zo):
                 assert (dv.from_dev(tmps[m] if swapped[m] else bufs[m]) == exps[m]).all(), (rep, m)
     finally:
         call("zk_graph_destroy", exec_)
+
+
+def _to_int(v):
+    return sum(int(v[i]) << (64 * i) for i in range(4))
+
+
+@pytest.mark.parametrize("inverse", [False, True])
+def test_2e24_known_values(gpu, zo, inverse):
+    """2^24 (four passes of degree 6) on five nonzero inputs: out[k] = s sum a_j
+    w^(j k), s = 1 / n in the inverse, at 3000 outputs"""
+    k, n = 24, 1 << 24
+    rng = np.random.default_rng(24 + inverse)
+    where = np.concatenate([[1, n - 1, n // 3], rng.integers(0, n, 2)])
+    x = np.zeros((n, 4), dtype=np.uint64)
+    x[where] = zo.rand_fr(5, 24)
+    w, n_inv, scale = zo.root_of_unity(k), None, 1
+    if inverse:
+        w, n_inv, scale = zo.fr_inv(w), zo.fr_inv(zo.fr_from_u64(n)), pow(n, -1, R)
+    got = _gpu_ntt(zo, x, k, w, n_inv)
+    root = zo.from_mont(w)[0]
+    vals = [_to_int(x[j]) * scale % R for j in where]
+    for o in np.concatenate([[0, 1, n - 1, n // 2, 4096, 4095], rng.integers(0, n, 3000)]):
+        exp = sum(v * pow(root, int(j) * int(o) % n, R) for j, v in zip(where, vals)) % R
+        assert _to_int(got[o]) == exp, o

@@ -277,6 +277,18 @@ __global__ __launch_bounds__(256) void k_fscan_apply(Fr *z, uint32_t n, const Fr
     }
 }
 
+// the wave-wide inversion's cofactor and whether its GCD ended, unchecked: one
+// wave per element
+__global__ __launch_bounds__(64) void k_fr_inv_wave(Fr *__restrict__ out, uint32_t *__restrict__ ok,
+                                                    const Fr *__restrict__ a) {
+    const Fr y = fe_load<FrParams>(&a[blockIdx.x]);
+    uint32_t v[8];
+    const bool good = zkinv::bingcd_wave(v, y.v, FrParams::M, FrParams::INV);
+    if (threadIdx.x) return;
+    fe_store<FrParams>(&out[blockIdx.x], fe_from_raw<FrParams>(v));
+    ok[blockIdx.x] = good ? 1u : 0u;
+}
+
 }  // namespace
 
 namespace zk {
@@ -339,6 +351,14 @@ extern "C" {
 hipError_t zk_batch_invert(void *a, void *temp, int n, hipStream_t stream) {
     if (n < 0 || (n > 0 && (!a || !temp))) return hipErrorInvalidValue;
     return batch_invert_ex((const Fr *)a, nullptr, (Fr *)a, OUT_SET, (uint32_t)n, stream);
+}
+
+// Test entry: v with y^-1 = v 2^36 mod r for y = a[i] as a plain number, and
+// ok[i] = 1 unless the GCD did not end at 1 (y = 0).
+hipError_t zk_fr_inv_wave(void *out, void *ok, const void *a, int n, hipStream_t stream) {
+    if (n <= 0 || !out || !ok || !a) return hipErrorInvalidValue;
+    k_fr_inv_wave<<<(uint32_t)n, 64, 0, stream>>>((Fr *)out, (uint32_t *)ok, (const Fr *)a);
+    return hipGetLastError();
 }
 
 // cuda/bn254.cu:1914-1934: sum[i] (=, or += when init != 0) 1/(input[i] + beta).
