@@ -76,3 +76,16 @@ def test_noalloc_rejects_sizes_beyond_the_array(gpu):
     assert L.zk_msm_noalloc(out.data_ptr(), dummy.data_ptr(), dummy.data_ptr(), MAX_N, 3,
                             dv.stream_handle()) != 0
     assert L.zk_msm_noalloc(out.data_ptr(), dummy.data_ptr(), dummy.data_ptr(), 0, 0, dv.stream_handle()) != 0
+
+
+# the largest size that each window accepts: the planner has to place its arrays
+# there too, and one point more is refused before the inputs are read
+@pytest.mark.parametrize("n,c", [(29488, 2), (73697, 5), (114748, 8), (137477, 11), (118483, 13), (15449, 14),
+                                 (131072, 0)])
+def test_noalloc_at_the_borders(gpu, zo, n, c):
+    import torch
+    from zkprover import device as dv
+    dp, ds = dv.to_dev(zo.gen_bases_random(n, 12).reshape(-1, 4)), dv.to_dev(zo.rand_fr(n, 13))
+    assert (_noalloc(dp, ds, n, c) == _with_scratch(dp, ds, n, c)).all()
+    out = torch.zeros(OUT_BYTES, dtype=torch.uint8, device=dv.device())
+    assert _lib().zk_msm_noalloc(out.data_ptr(), dp.data_ptr(), ds.data_ptr(), n + 1, c, dv.stream_handle()) != 0

@@ -47,8 +47,10 @@ enum BinvMode {
 // The products are the 29-bit ones (ff29.h): running products stay in the
 // 256-bit Montgomery domain below 2r, and one operand of each product is
 // shifted into the 2^261 domain (f29_from32 of an element, f29_shl5 of a
-// product).  Four waves per SIMD (128 registers, nine per prefix) measured
-// best: 2^22 elements 225 us with three, 191 with four, 208 with five.
+// product).  Four waves per SIMD measured best: 2^22 elements 225 us with
+// three, 191 with four, 208 with five, although the prefixes of eight elements
+// (nine registers each) don't fit its 128 registers: 88 B per lane go to
+// scratch (none with two or four elements).
 constexpr uint32_t kBT = 256;
 
 struct BinvNode {
@@ -115,7 +117,7 @@ __global__ __launch_bounds__(kBT, 4) void k_binv(Fr *x, const Fr *__restrict__ b
     }
     acc = node_load(tree[kBT + t]);
     Fr sum = fe_zero<FrParams>();
-    // fully unrolled: the prefixes stay in registers
+    // fully unrolled: an indexed array would go to scratch whole
 #pragma clang loop unroll(full)
     for (int k = E - 1; k >= 0; k--) {
         const uint64_t i = base + (uint32_t)k * kBT;

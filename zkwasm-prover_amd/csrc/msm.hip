@@ -1527,8 +1527,10 @@ uint32_t msm_default_window(uint32_t n) { return default_window(n); }
 // The size by which zk_msm_noalloc accepts or refuses an MSM of n points at
 // window c (0 = default): one block per array of a fixed layout (4096-scalar
 // sort tiles, chunks of 96 entries, or 2^16 of at least 8 below 2^21 entries).
-// A limit of that entry only, kept apart from the plan, which sizes its
-// chunks to the room there is and fits wherever this does.
+// A limit of that entry only, kept apart from the plan so that what it accepts
+// does not move with it.  The plan sizes its chunks and sort tiles to the room
+// there is; where it should not fit after all the call returns
+// hipErrorOutOfMemory (the largest accepted size of each window is a test).
 size_t msm_noalloc_bytes(uint32_t n, uint32_t c) {
     if (!c) c = default_window(n);
     const uint64_t W = (255 + c - 1) / c, B = 1ull << (c - 1), NB = W * B, entries = (uint64_t)n * W;

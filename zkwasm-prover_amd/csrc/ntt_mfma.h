@@ -4,7 +4,7 @@
 // SA over j2, a twiddle product, and a DFT of size SB over j1:
 //   X[k1 + SA k2] = sum_j1 w_SB^(j1 k2) w_D^(j1 k1) sum_j2 w_SA^(j2 k1) x[j2 SB + j1].
 // The small DFTs are contractions with a constant matrix that every column
-// shares, so they go to v_mfma_i32_32x32x32_i8: an element is 32 bytes, the
+// shares, so they go to v_mfma_i32_16x16x64_i8: an element is 32 bytes, the
 // matrix entry for (k, i, byte b) is w^(k i) 2^(8 b) mod r in balanced bytes, and
 // the sum over i and b of byte products gives the 32 byte columns of
 // sum_i w^(k i) x_i already reduced to 14 bits over r: no carries, no
