@@ -439,7 +439,7 @@ __global__ __launch_bounds__(kThreads) void k_ntt_pass(const NttPassArgs a) {
 // Bound by VALU issue (about 800 instructions per element of a 2^7 pass with
 // inter-pass twiddles, two 29-bit products of 260 among them; the radix-2
 // kernel has 1270 to 1580), then by the last pass's scattered reads of the
-// omegas.  2^22 elements: first pass 98 us, middle 157 us, last 184 us, against
+// omegas.  2^22 elements: first pass 95 us, middle 127 us, last 173 us, against
 // 173 us each in the radix-2 kernel.  Tried: 32x32x32 products with 512
 // elements per wave (two waves per SIMD: 140 and 220 us), 2048-element tiles
 // per workgroup with barriers in the exchange (batches 17% slower: the older
